@@ -271,12 +271,14 @@ __device__ inline bool box_hit_nf(const BoxRay& r, float nx, float fx, float ny,
     return tn <= tf;
 }
 
-// The same test from the slab distances themselves (near and far per axis).
-__device__ inline bool box_hit_t(const BoxRay& r, float tnx, float tfx, float tny, float tfy, float tnz, float tfz) {
-    const float tn = fmaxf(fmaxf(fmaxf(r.tlo, tnx), tny), tnz);
-    float tf = fminf(fminf(fminf(r.thi, tfx), tfy), tfz);
-    tf = tf + fabsf(tf) * 0x1p-20f;
-    return tn <= tf;
+// The test's two sides from the slab distances themselves: the near bound and
+// the far bound widened by |tfar| 2^-20 (one fused multiply-add).
+__device__ inline float box_near(const BoxRay& r, float tnx, float tny, float tnz) {
+    return fmaxf(fmaxf(fmaxf(r.tlo, tnx), tny), tnz);
+}
+__device__ inline float box_far(const BoxRay& r, float tfx, float tfy, float tfz) {
+    const float tf = fminf(fminf(fminf(r.thi, tfx), tfy), tfz);
+    return __builtin_fmaf(fabsf(tf), 0x1p-20f, tf);
 }
 
 __device__ inline bool box_hit(const BoxRay& r, float lox, float hix, float loy, float hiy,
