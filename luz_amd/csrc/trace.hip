@@ -153,8 +153,15 @@ __global__ __launch_bounds__(kBlock) void k_cull_rows(const uint32_t* counters, 
     cull_rows_lane(live_bits[g], R, w, g << 6, rows + row_base[g], hits + (size_t)g0 * R);
 }
 
-// Rays are claimed in chunks per wave (one device-scope atomic per chunk).
-// The chunk follows the launch's ray count, 1/kChunkShare of an even share per
+// Rays go to the waves in chunks.  A wave's first chunk is its own by its
+// position in the grid; the following ones it claims, one device-scope atomic
+// each.  A launch of at most kChunkMin rays per wave is dealt out whole that
+// way, in chunks as even as rows of 64 allow, and makes no claim: with every
+// chunk claimed, 256-ray chunks left most waves of a 256x256 frame without
+// work, and each of them tried all claim counters in vain (49k atomics on 8
+// addresses): the 256x256 cube frame 161 -> 74 us, 1M incoherent rays 241 ->
+// 202 us.  Above that the
+// chunk follows the launch's ray count, 1/kChunkShare of an even share per
 // wave, kept within kChunkMin .. kChunkMax rays: the rays in flight on the
 // whole GPU (waves x chunk) then cover few image rows of one light at a time,
 // so the BVH nodes they read stay in L2, while the claims stay below the rate
@@ -165,6 +172,7 @@ __global__ __launch_bounds__(kBlock) void k_cull_rows(const uint32_t* counters, 
 constexpr uint32_t kChunkMin = 256, kChunkMax = 512, kChunkShare = 12;
 
 __device__ inline uint32_t claim_chunk(uint32_t nrays, uint32_t nwaves) {
+    if (nrays <= nwaves * kChunkMin) return nrays ? ((nrays - 1) / nwaves / 64u + 1u) * 64u : 64u;
     const uint32_t c = (nrays / (nwaves * kChunkShare)) & ~63u;
     return c < kChunkMin ? kChunkMin : (c > kChunkMax ? kChunkMax : c);
 }
@@ -264,13 +272,23 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
     uint32_t ray = kNone;
     bool open = true;
     uint32_t chunk_next = 0, chunk_end = 0;  // wave-uniform
-    // Claim counter c hands out chunks c, c + 8, c + 16, ... of the launch's
-    // rays, so the waves still advance one front through the rays (the BVH
-    // nodes in use stay few) while their atomics spread over 8 addresses.  A
-    // wave starts on the counter of its workgroup and moves to the next one
-    // when a counter's chunks run past the last ray.
+    // Chunks c, c + 8, c + 16, ... of the launch's rays belong to claim counter
+    // c, so the waves advance one front through the rays (the BVH nodes in use
+    // stay few) while their atomics spread over 8 addresses.  The workgroups b
+    // with b % 8 == c take the first of them, one per wave, without a claim
+    // (`dealt` of them); the counter hands out the rest.  A wave claims from the
+    // counter of its workgroup and moves to the next one when a counter's chunks
+    // run past the last ray (known without an atomic where all were dealt).
     const uint32_t seg0 = blockIdx.x % kClaimSegments;
     uint32_t seg = 0;   // counters this wave has found exhausted (wave-uniform)
+    {
+        const uint64_t base = ((uint64_t)(blockIdx.x / kClaimSegments * (kBlock / 64) + (tid >> 6)) * kClaimSegments +
+                               seg0) * chunk;
+        if (base < nrays) {
+            chunk_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+            chunk_end = nrays - chunk_next > chunk ? chunk_next + chunk : nrays;
+        }
+    }
     for (;;) {
         if (open) {
             uint64_t idle = __ballot(ray == kNone);
@@ -282,11 +300,16 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
                         break;
                     }
                     const uint32_t c = (seg0 + seg) % kClaimSegments;
+                    const uint32_t dealt = (gridDim.x + kClaimSegments - 1 - c) / kClaimSegments * (kBlock / 64);
+                    if (((uint64_t)dealt * kClaimSegments + c) * chunk >= nrays) {
+                        ++seg;
+                        continue;
+                    }
                     uint32_t got = 0;
                     if (lane == 0) got = atomicAdd(&L.counters[kClaimBase + c * kClaimStride], 1u);
                     // only lane 0 holds the atomic's result: every decision
                     // below uses the broadcast copy, so the claim stays uniform
-                    const uint64_t base = ((uint64_t)__shfl(got, 0) * kClaimSegments + c) * chunk;
+                    const uint64_t base = ((uint64_t)(dealt + __shfl(got, 0)) * kClaimSegments + c) * chunk;
                     if (base < nrays) {
                         chunk_next = (uint32_t)base;
                         chunk_end = nrays - chunk_next > chunk ? chunk_next + chunk : nrays;
@@ -438,6 +461,7 @@ void launch_cull_scan(hipStream_t st, uint32_t* counts, uint32_t n, uint32_t* co
 
 luzrt_status launch_trace(luzrt_ctx* ctx, const TraceLaunch& L) {
     uint32_t groups = (uint32_t)ctx->num_cus * ctx->groups_per_cu;
+    if (L.max_rays > 0) groups = (uint32_t)std::min<uint64_t>(groups, (L.max_rays + kBlock - 1) / kBlock);
     if (groups == 0) groups = 1;
     size_t spill_bytes = (size_t)groups * kBlock * kSpill * 4;
     luzrt_status s = ensure(ctx, ctx->spill, spill_bytes);
@@ -578,6 +602,7 @@ luzrt_status visibility_core(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
         L.recs_count = tlas->count;
         L.hits = (uint8_t*)ctx->hits.ptr;
         L.counters = counters;
+        L.max_rays = (uint64_t)ngroups * kCullGroup * ds.r_total;
         L.wide = tlas->wide;
         L.gen = true;
         L.ds = dsd;
@@ -703,6 +728,7 @@ extern "C" luzrt_status luzrt_trace_rays(luzrt_ctx* ctx, const luzrt_tlas* tlas,
         L.ray_stride = 2;
         L.hits = hits;
         L.counters = counters;
+        L.max_rays = count;
         L.wide = tlas->wide;
         if ((s = launch_trace(ctx, L)) != LUZRT_OK) return s;
     }

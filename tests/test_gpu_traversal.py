@@ -1,12 +1,23 @@
-"""Rays with zero, infinite and NaN components through the 8-wide nodes against
-the binary ones."""
+"""Traversal launches at the edges of their dispatch: ray counts around the
+chunks that waves are dealt and claim, and rays with zero, infinite and NaN
+components through the 8-wide nodes against the binary ones."""
 import numpy as np
 import pytest
 
 from luz_amd import api
-from tests.helpers import random_rays
+from tests.helpers import oracle_scene, random_rays
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def cube(ctx):
+    s = api.HostScene(api.SCENE_CUBE, 0)
+    g = api.GPUScene(ctx, s)
+    rays = random_rays(np.random.default_rng(3), 1 << 19, (0, 0.5, 0), 2.0, 20.0)
+    want, _ = oracle_scene(s).any_hit(rays)
+    yield g, ctx.to_device(rays), want
+    g.close()
 
 
 def _hits(ctx, tlas, rays, n):
@@ -15,6 +26,18 @@ def _hits(ctx, tlas, rays, n):
     got = out.download(np.uint8, n + 64)
     assert (got[n:] == 7).all()      # nothing written past the last ray
     return got[:n]
+
+
+@pytest.mark.parametrize("groups", [0, 1])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 4097, 98303, 393217, 1 << 19])
+def test_ray_counts_around_chunks(ctx, cube, n, groups):
+    # one workgroup per CU (256 groups) claims chunks from 65,536 x 4 rays on
+    g, rays, want = cube
+    if groups:
+        ctx.set_trace_config(groups_per_cu=groups)
+    got = _hits(ctx, g.tlas, rays, n)
+    ctx.set_trace_config(groups_per_cu=6)
+    np.testing.assert_array_equal(got, want[:n])
 
 
 def test_special_rays_meet_the_same_triangles_in_both_trees(ctx):
