@@ -18,8 +18,8 @@
 // of K-step s is  k = 16 * (2s + e/4) + 4g + e%4.  Weight fragments are
 // packed in that order, so activations stay in registers through all five
 // layers, forward and backward (the transposed weights W^T are packed the
-// same way for the backward pass).  The features of layer 1 use k = 32s +
-// 8g + e.  Any K order works as long as A and B agree, because the hardware
+// same way for the backward pass).  The features of layer 1 go in the order of
+// infer_feature.  Any K order works as long as A and B agree, because the hardware
 // pairs element e of lane group g of A with the same element of B.
 //
 // Inference (k_dn_infer) takes 16-pixel tiles: the 125 features that do not
@@ -28,10 +28,11 @@
 //
 // Training: k_dn_forward runs forward, loss and the backward pass to
 // every layer's pre-activation gradient dz, and stores x, h and dz (BF16)
-// sample-minor ([feature][sample]); k_dn_wgrad forms dW = dz^T h per chunk of
-// 1024 samples with MFMA (K = samples) and bias sums; k_dn_reduce adds the
-// chunk partials in a fixed order (deterministic gradients); k_dn_adam and
-// k_dn_pack update the FP32 master weights and re-pack the BF16 fragments.
+// sample-major, each lane's fragments as they stand in its registers;
+// k_dn_wgrad forms dW = dz^T h per chunk of 1024 samples with MFMA (K =
+// samples, transposed from those rows in registers) and bias sums; k_dn_reduce
+// adds the chunk partials in a fixed order (deterministic gradients); k_dn_adam
+// updates the FP32 master weights and re-packs their BF16 fragments.
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -63,6 +64,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kIn = LUZRT_DN_FEATURES, kHid = LUZRT_DN_HIDDEN, kOut = 2;
 constexpr int kBlock = 256;
 constexpr uint32_t kChunkRows = 1024;
+constexpr int kX = 192;   // positions of a training row's inputs: 6 K-steps of 32, 42 of them zero
 // inference: one 16-pixel tile per wave at a time, 8 waves per group sharing
 // one copy of the weights in LDS
 constexpr int kInferBlock = 512;
@@ -79,12 +81,13 @@ constexpr int kWOff[5] = {oW1, oW2, oW3, oW4, oW5};
 constexpr int kBOff[5] = {oB1, oB2, oB3, oB4, oB5};
 
 // Fragment table (one fragment = 64 lanes x 8 BF16 = 1 KB):
-//   F1(t,s) t<4 s<5 | F2..F4(t,s) t<4 s<2 | G2..G4(t,s) | G5(t) t<4
-//   | FG(t,s) t<4 s<4 | FV(t) t<4
-// Layer 5 (64 -> 2) runs in FP32 (dn_out_fp32); G5 holds W5^T for the backward pass.
-// FG and FV hold layer 1 again in the inference order, which splits the
-// features of a (pixel, light) sample into the 125 that do not depend on the
-// light (one product per pixel) and the 25 visibilities (one K-step per light).
+//   F2..F4(t,s) t<4 s<2 | G2..G4(t,s) | G5(t) t<4 | FG(t,s) t<4 s<5 | FV(t) t<4
+//   | F5(s) s<2
+// In training layer 5 (64 -> 2) runs in FP32 (dn_out_fp32); G5 holds W5^T for
+// the backward pass.
+// FG and FV hold layer 1 in an order that splits the features of a (pixel,
+// light) sample into the 125 that do not depend on the light (one product per
+// pixel in inference) and the 25 visibilities (one K-step per light).
 // Lane group g only ever reads neighbours 8g .. 8g + 7 (those below 25):
 //   FG, K-steps s < 4: element e is channel (AO, n.x, n.y, n.z)[e % 4] of
 //       neighbour 8g + 2s + e / 4;
@@ -93,8 +96,8 @@ constexpr int kBOff[5] = {oB1, oB2, oB3, oB4, oB5};
 // F5(s) s < 2 holds layer 5 for inference, where it runs on MFMA: output row 0
 // and 1 are the BF16 rounding of W5's rows, rows 2 and 3 the BF16 rounding of
 // what that leaves (W5 - hi), rows 4..15 zero, K in the hidden-layer order.
-constexpr int kF1 = 0, kF2 = 20, kF3 = 28, kF4 = 36, kG2 = 44, kG3 = 52, kG4 = 60,
-              kG5 = 68, kFG = 72, kFV = 92, kF5 = 96, kFragTrain = 72, kFragAll = 98;
+constexpr int kF2 = 0, kF3 = 8, kF4 = 16, kG2 = 24, kG3 = 32, kG4 = 40, kG5 = 48, kFG = 52, kFV = 72,
+              kF5 = 76, kFragTrain = 76, kFragAll = 78;
 // inference fragments in LDS: F2..F4 (24), then FG and FV (24), then F5 (2)
 constexpr int kIF2 = 0, kIF3 = 8, kIF4 = 16, kIFG = 24, kIFV = 44, kIF5 = 48, kFragInfer = 50;
 
@@ -142,11 +145,11 @@ struct DnArgs {
     const uint32_t* samples;   // pixel | light << 24
     const float* target_ao;    // [npix]
     const float* target_vis;   // [L][npix]
-    uint32_t row_base, ldn;    // training rows of this call, leading dimension
-    uint16_t* XT;              // [160][ldn]
-    uint16_t* HT;              // [4][64][ldn]
-    uint16_t* ZT;              // [4][64][ldn]
-    uint16_t* YT;              // [16][ldn]
+    uint32_t row_base, cap;    // first training row of this call, rows of an array
+    uint4* X;                  // [cap][kX] BF16, K-step order (infer_feature)
+    uint4* H;                  // [4][cap][64] BF16, feature 16t + 4g + i at 16g + 4t + i
+    uint4* Z;                  // [4][cap][64] BF16, likewise
+    uint32_t* Y;               // [cap] two BF16
     float grad_scale;          // dLoss/dy = grad_scale * (y - target)
     float* loss_sum;
 };
@@ -190,37 +193,6 @@ __global__ __launch_bounds__(256) void k_dn_prep(DnFrameDev F, float4* pix, floa
     ao_frac[p] = (float)F.ao[p] / F.ao_n;
 }
 
-// The base the network's outputs are added to: the mean, over the foreground
-// pixels of the clamped 5x5 window, of the AO fraction and of the visibility
-// of `light` (0 without lights).  Summed per group of 8 neighbours (n = 8g + e,
-// in order of e), then ((g0 + g1) + (g2 + g3)): the order of the lane
-// reduction in k_dn_infer, so training and inference bases are identical.
-__device__ inline void dn_box(const DnFrameDev& F, uint32_t x, uint32_t y, uint32_t light, float& bao,
-                              float& bvis) {
-    float sa[4], sv[4];
-    int cnt = 0;
-    for (int g = 0; g < 4; ++g) {
-        sa[g] = 0.0f;
-        sv[g] = 0.0f;
-        for (int e = 0; e < 8; ++e) {
-            const int n = 8 * g + e;
-            if (n >= 25) break;
-            int qx = (int)x + n % 5 - 2, qy = (int)y + n / 5 - 2;
-            qx = qx < 0 ? 0 : (qx >= (int)F.width ? (int)F.width - 1 : qx);
-            qy = qy < 0 ? 0 : (qy >= (int)F.height ? (int)F.height - 1 : qy);
-            const size_t q = (size_t)qy * F.width + qx;
-            if (F.pix[q].x < 0.0f) continue;
-            cnt++;
-            sa[g] += F.ao_frac[q];
-            if (F.num_lights)
-                sv[g] += 1.0f - (float)F.shadow[(size_t)light * F.width * F.height + q] / F.shadow_n;
-        }
-    }
-    const float c = (float)(cnt ? cnt : 1);
-    bao = ((sa[0] + sa[1]) + (sa[2] + sa[3])) / c;
-    bvis = ((sv[0] + sv[1]) + (sv[2] + sv[3])) / c;
-}
-
 __device__ inline float nb_channel(const Nb& b, int c) {
     return c == 0 ? b.c0 : c == 1 ? b.c1 : c == 2 ? b.c2 : c == 3 ? b.c3 : c == 4 ? b.c4 : b.c5;
 }
@@ -253,11 +225,10 @@ __device__ inline uint4 dn_features(const DnFrameDev& F, bool valid, uint32_t x,
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Bias + ReLU of a hidden layer's 4x4 tiles of one sample column (training);
-// the next layer's B fragments, the ReLU mask (bit t*4+i) and h stored.
-__device__ inline void dn_hidden_epilogue(const f32x4 (&acc)[4], const float* bias, int g, uint4 (&hb)[2],
-                                          uint32_t& mask, uint16_t* HTl, uint32_t ldn, uint32_t row,
-                                          bool store) {
+// ReLU of a hidden layer's 4x4 tiles of one sample column (training; the bias
+// is in the accumulators): the next layer's B fragments and the ReLU mask (bit
+// t * 4 + i).
+__device__ inline void dn_hidden_epilogue(const f32x4 (&acc)[4], uint4 (&hb)[2], uint32_t& mask) {
     uint32_t w[2][4];
     mask = 0;
 #pragma unroll
@@ -265,22 +236,13 @@ __device__ inline void dn_hidden_epilogue(const f32x4 (&acc)[4], const float* bi
         float h[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float z = acc[t][i] + bias[16 * t + 4 * g + i];
-            const bool on = z > 0.0f;
-            h[i] = on ? z : 0.0f;
+            const bool on = acc[t][i] > 0.0f;
+            h[i] = on ? acc[t][i] : 0.0f;
             mask |= (on ? 1u : 0u) << (t * 4 + i);
         }
         // elements e = (t & 1) * 4 + i of K-step s = t / 2
 #pragma unroll
-        for (int i = 0; i < 4; i += 2) {
-            const uint32_t bits = bf16_pack2(h[i], h[i + 1]);
-            w[t >> 1][((t & 1) * 4 + i) >> 1] = bits;
-            if (store) {
-                const int o = 16 * t + 4 * g + i;
-                HTl[(size_t)o * ldn + row] = (uint16_t)bits;
-                HTl[(size_t)(o + 1) * ldn + row] = (uint16_t)(bits >> 16);
-            }
-        }
+        for (int i = 0; i < 4; i += 2) w[t >> 1][((t & 1) * 4 + i) >> 1] = bf16_pack2(h[i], h[i + 1]);
     }
     hb[0] = make_uint4(w[0][0], w[0][1], w[0][2], w[0][3]);
     hb[1] = make_uint4(w[1][0], w[1][1], w[1][2], w[1][3]);
@@ -332,28 +294,20 @@ __device__ inline void dn_out_fp32(const f32x4 (&h)[4], const float* w5, int g, 
     y1 = p1;
 }
 
-// Layer (k >= 2) with 2 K-steps: acc[q][t] = sum_s frag(t, s) * hb[q][s].
-template <int Q>
-__device__ inline void dn_layer64(const uint4* sfrag, int fbase, int lane, const uint4 (&hb)[Q][2],
-                                  f32x4 (&acc)[Q][4]) {
-#pragma unroll
-    for (int q = 0; q < Q; ++q)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[q][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+// A 64 -> 64 layer (2 K-steps) on top of the accumulators: acc[t] += sum_s
+// frag(t, s) * hb[s].
+__device__ inline void dn_layer64(const uint4* sfrag, int fbase, int lane, const uint4 (&hb)[2],
+                                  f32x4 (&acc)[4]) {
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            bf16x8 a = as_bf16x8(sfrag[(fbase + t * 2 + s) * 64 + lane]);
-#pragma unroll
-            for (int q = 0; q < Q; ++q) acc[q][t] = mfma(a, as_bf16x8(hb[q][s]), acc[q][t]);
-        }
+        for (int t = 0; t < 4; ++t)
+            acc[t] = mfma(as_bf16x8(sfrag[(fbase + t * 2 + s) * 64 + lane]), as_bf16x8(hb[s]), acc[t]);
 }
 
-// Backward through a hidden layer's ReLU: dz = dh * mask; stores dz (BF16)
-// when training rows are valid, and builds the B fragments of dz.
-__device__ inline void dn_relu_back(const f32x4 (&dh)[4], uint32_t mask, int g, uint4 (&zb)[2],
-                                    uint16_t* ZTl, uint32_t ldn, uint32_t row, bool store) {
+// Backward through a hidden layer's ReLU: dz = dh * mask as the B fragments of
+// the layer below (and as they are stored).
+__device__ inline void dn_relu_back(const f32x4 (&dh)[4], uint32_t mask, uint4 (&zb)[2]) {
     uint32_t w[2][4];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -361,178 +315,11 @@ __device__ inline void dn_relu_back(const f32x4 (&dh)[4], uint32_t mask, int g, 
         for (int i = 0; i < 4; i += 2) {
             const float d0 = (mask >> (t * 4 + i)) & 1u ? dh[t][i] : 0.0f;
             const float d1 = (mask >> (t * 4 + i + 1)) & 1u ? dh[t][i + 1] : 0.0f;
-            const uint32_t bits = bf16_pack2(d0, d1);
-            w[t >> 1][((t & 1) * 4 + i) >> 1] = bits;
-            if (store) {
-                const int o = 16 * t + 4 * g + i;
-                ZTl[(size_t)o * ldn + row] = (uint16_t)bits;
-                ZTl[(size_t)(o + 1) * ldn + row] = (uint16_t)(bits >> 16);
-            }
+            w[t >> 1][((t & 1) * 4 + i) >> 1] = bf16_pack2(d0, d1);
         }
     zb[0] = make_uint4(w[0][0], w[0][1], w[0][2], w[0][3]);
     zb[1] = make_uint4(w[1][0], w[1][1], w[1][2], w[1][3]);
 }
-
-// Training forward, loss and backward of explicit samples.  Q: 16-sample
-// tiles per wave and iteration (each weight fragment read from LDS feeds Q
-// MFMAs).
-template <int Q>
-__global__ __launch_bounds__(kBlock) void k_dn_forward(DnArgs A) {
-    __shared__ uint4 sfrag[kFragTrain * 64];
-    __shared__ float sbias[4 * kHid + kOut];
-    __shared__ __align__(16) float sw5[kOut * kHid];
-    for (int i = threadIdx.x; i < kFragTrain * 64; i += kBlock) sfrag[i] = A.frags[i];
-    for (int i = threadIdx.x; i < kOut * kHid; i += kBlock) sw5[i] = A.params[oW5 + i];
-    for (int i = threadIdx.x; i < 4 * kHid + kOut; i += kBlock)
-        sbias[i] = A.params[i < 4 * kHid ? kBOff[i / kHid] + i % kHid : oB5 + (i - 4 * kHid)];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
-    const uint32_t wave = threadIdx.x >> 6;
-    const uint32_t nwaves = gridDim.x * (kBlock / 64);
-    const DnFrameDev& F = A.F;
-    const uint32_t npix = F.width * F.height;
-    for (uint32_t base = (blockIdx.x * (kBlock / 64) + wave) * (16u * Q); base < A.nsamples;
-         base += nwaves * (16u * Q)) {
-        uint32_t px[Q], py[Q], pl[Q], pp[Q], row[Q];
-        bool valid[Q], inb[Q];
-        float dc[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            uint32_t i = base + 16u * q + (uint32_t)j;
-            uint32_t p = 0, l = 0;
-            float dcv = 0.0f;
-            bool in = i < A.nsamples, v = false;
-            if (in) {
-                uint32_t sm = A.samples[i];
-                p = sm & 0xFFFFFFu;
-                l = sm >> 24;
-                // caller-supplied samples outside the frame contribute nothing
-                if (p >= npix || l >= A.lights) { p = 0; l = 0; }
-                else {
-                    dcv = F.pix[p].x;
-                    v = dcv >= 0.0f;
-                }
-            }
-            pp[q] = p; pl[q] = l;
-            px[q] = p % F.width; py[q] = p / F.width;
-            row[q] = A.row_base + i;
-            dc[q] = v ? dcv : 0.0f;
-            valid[q] = v;
-            inb[q] = in;
-        }
-        // ---- layer 1: 150 (160) -> 64
-        f32x4 acc[Q][4];   // [q][t]
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-#pragma unroll
-            for (int t = 0; t < 4; ++t) acc[q][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int s = 0; s < 5; ++s) {
-            bf16x8 b[Q];
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                uint4 fb = dn_features(F, valid[q], px[q], py[q], pl[q], dc[q], 32 * s + 8 * g);
-                b[q] = as_bf16x8(fb);
-                if (inb[q]) {
-                    const uint32_t ws[4] = {fb.x, fb.y, fb.z, fb.w};
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        A.XT[(size_t)(32 * s + 8 * g + e) * A.ldn + row[q]] =
-                            (uint16_t)(ws[e >> 1] >> (16 * (e & 1)));
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                bf16x8 a = as_bf16x8(sfrag[(kF1 + t * 5 + s) * 64 + lane]);
-#pragma unroll
-                for (int q = 0; q < Q; ++q) acc[q][t] = mfma(a, b[q], acc[q][t]);
-            }
-        }
-        uint4 hb[Q][2];
-        uint32_t mask[4][Q];   // [layer][q]
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-            dn_hidden_epilogue(acc[q], sbias, g, hb[q], mask[0][q], A.HT, A.ldn, row[q], inb[q]);
-        // ---- layers 2..4: 64 -> 64
-#pragma unroll
-        for (int k = 1; k < 4; ++k) {
-            dn_layer64<Q>(sfrag, k == 1 ? kF2 : (k == 2 ? kF3 : kF4), lane, hb, acc);
-#pragma unroll
-            for (int q = 0; q < Q; ++q)
-                dn_hidden_epilogue(acc[q], sbias + k * kHid, g, hb[q], mask[k][q],
-                                   A.HT + (size_t)k * kHid * A.ldn, A.ldn, row[q], inb[q]);
-        }
-        // ---- layer 5: 64 -> 2 in FP32 on layer 4's activations (as in dn_hidden_epilogue)
-        float out[Q][2];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            f32x4 h[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float z = acc[q][t][i] + sbias[3 * kHid + 16 * t + 4 * g + i];
-                    h[t][i] = z > 0.0f ? z : 0.0f;
-                }
-            dn_out_fp32(h, sw5, g, out[q][0], out[q][1]);
-        }
-        const float b50 = sbias[4 * kHid], b51 = sbias[4 * kHid + 1];
-        // ---- loss and backward
-        float loss = 0.0f;
-        uint4 db[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            float d0 = 0.0f, d1 = 0.0f;
-            if (g == 0 && valid[q]) {
-                float bao, bvis;
-                dn_box(F, px[q], py[q], pl[q], bao, bvis);
-                float e0 = (out[q][0] + b50) + bao - A.target_ao[pp[q]];
-                float e1 = (out[q][1] + b51) + bvis -
-                           (F.num_lights ? A.target_vis[(size_t)pl[q] * npix + pp[q]] : 0.0f);
-                loss += e0 * e0 + e1 * e1;
-                d0 = A.grad_scale * e0;
-                d1 = A.grad_scale * e1;
-            }
-            const uint32_t b01 = bf16_pack2(d0, d1);
-            if (g == 0 && inb[q]) {
-                A.YT[row[q]] = (uint16_t)b01;
-                A.YT[(size_t)A.ldn + row[q]] = (uint16_t)(b01 >> 16);
-            }
-            db[q] = make_uint4(g == 0 ? b01 : 0u, 0u, 0u, 0u);
-        }
-        // dh4 = W5^T dy
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                acc[q][t] = mfma(as_bf16x8(sfrag[(kG5 + t) * 64 + lane]), as_bf16x8(db[q]),
-                                 f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-#pragma unroll
-        for (int k = 3; k >= 0; --k) {
-            uint4 zb[Q][2];
-#pragma unroll
-            for (int q = 0; q < Q; ++q)
-                dn_relu_back(acc[q], mask[k][q], g, zb[q], A.ZT + (size_t)k * kHid * A.ldn, A.ldn, row[q],
-                             inb[q]);
-            if (k == 0) break;
-            // dh_{k} = W_{k+1}^T dz_{k+1}  (fragments G2..G4 hold W2^T..W4^T)
-            dn_layer64<Q>(sfrag, k == 3 ? kG4 : (k == 2 ? kG3 : kG2), lane, zb, acc);
-        }
-        // per-wave loss sum (lanes g == 0 hold the outputs)
-        for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
-        if (lane == 0) atomicAdd(A.loss_sum, loss);
-    }
-}
-
-struct InferArgs {
-    DnFrameDev F;
-    const uint4* frags;
-    const float* params;
-    uint32_t lights;    // max(L, 1)
-    uint32_t ntiles;    // 16-pixel tiles of the frame
-    float* ao_out;      // [npix]
-    float* vis_out;     // [L][npix]
-};
 
 // Index of neighbour n (< 25) of pixel (x, y), clamped to the image.
 __device__ inline uint32_t dn_nb_index(const DnFrameDev& F, uint32_t x, uint32_t y, int n) {
@@ -541,17 +328,6 @@ __device__ inline uint32_t dn_nb_index(const DnFrameDev& F, uint32_t x, uint32_t
     qy = qy < 0 ? 0 : (qy >= (int)F.height ? (int)F.height - 1 : qy);
     return (uint32_t)qy * F.width + (uint32_t)qx;
 }
-
-// The per-pixel state a tile's light groups share: lane (j, g) holds pixel j
-// of the tile and neighbours 8g + e (e < 8) of its 5x5 window.
-struct InferTile {
-    uint32_t vq[8];   // neighbour indices (0 off the window and for invalid pixels)
-    uint32_t bo[8];   // visibility table offset: 0 for a foreground neighbour, else
-                      // 2048 bytes (the table's zero half)
-    float cnt, bao;   // foreground pixels of the window, box base of AO
-    uint32_t pp;      // pixel index (0 beyond the frame)
-    bool valid, inb;
-};
 
 // Sum of a value over the four lane groups (rows of 16 lanes) of a pixel
 // column, as ((g0 + g1) + (g2 + g3)), in every lane: v_permlane16_swap pairs
@@ -569,6 +345,196 @@ __device__ inline uint32_t col_sum(uint32_t v) {
     const auto b = __builtin_amdgcn_permlane32_swap(s, s, false, false);
     return b[0] + b[1];
 }
+
+// Training forward, loss and backward of explicit samples, 16 per wave at a
+// time (lane column j: sample j).
+//
+// What bounds it is latency: a call has a few thousand samples, so each wave
+// runs one chain of gather, five layers and four layers back once or twice.
+// The gather is one trip: lane group g reads neighbours 8g .. 8g + 7 of each
+// sample straight from the G-buffer and count planes, all loads in flight
+// together, and the centre's distance comes from the lane that read it.  (In
+// feature order, with the neighbour changing at another element in each lane
+// group, the loads came one after the other, in 64-sample waves, behind a
+// prepass over the frame, and the rows were stored in 2-byte pieces: 8192
+// samples of a 256x256 frame took 150 us, now 21 us.)  16-sample waves rather
+// than 64: four times as many waves to spread over the CUs.
+__global__ __launch_bounds__(kBlock) void k_dn_forward(DnArgs A) {
+    __shared__ uint4 sfrag[kFragTrain * 64];
+    __shared__ __align__(16) float sbias[4 * kHid + 4];
+    __shared__ __align__(16) float sw5[kOut * kHid];
+    {
+        constexpr int kPer = kFragTrain * 64 / kBlock;   // all of a thread's loads in flight together
+        static_assert(kPer * kBlock == kFragTrain * 64, "whole fragments per thread");
+        uint4 fr[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) fr[i] = A.frags[i * kBlock + threadIdx.x];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) sfrag[i * kBlock + threadIdx.x] = fr[i];
+    }
+    for (int i = threadIdx.x; i < kOut * kHid; i += kBlock) sw5[i] = A.params[oW5 + i];
+    for (int i = threadIdx.x; i < 4 * kHid + kOut; i += kBlock)
+        sbias[i] = A.params[i < 4 * kHid ? kBOff[i / kHid] + i % kHid : oB5 + (i - 4 * kHid)];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t nwaves = gridDim.x * (kBlock / 64);
+    const DnFrameDev& F = A.F;
+    const uint32_t npix = F.width * F.height;
+    // the sample count is a multiple of 64: every tile is whole
+    for (uint32_t base = (blockIdx.x * (kBlock / 64) + wave) * 16u; base < A.nsamples; base += nwaves * 16u) {
+        const uint32_t sm = A.samples[base + (uint32_t)j];
+        uint32_t p = sm & 0xFFFFFFu, l = sm >> 24;
+        // caller-supplied samples outside the frame contribute nothing
+        const bool in_frame = p < npix && l < A.lights;
+        if (!in_frame) { p = 0; l = 0; }
+        const size_t row = A.row_base + base + (uint32_t)j;
+        const uint32_t px = p % F.width, py = p / F.width;
+        float d[8], n3[8][3], ao[8], vis[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t q = dn_nb_index(F, px, py, 8 * g + e < 25 ? 8 * g + e : 0);
+            const float* N = F.normal + (size_t)q * 3;
+            const float* P = F.position + (size_t)q * 3;
+            const float dist = vlen(v3(P[0] - F.cam[0], P[1] - F.cam[1], P[2] - F.cam[2]));
+            n3[e][0] = N[0]; n3[e][1] = N[1]; n3[e][2] = N[2];
+            ao[e] = (float)F.ao[q] / F.ao_n;
+            vis[e] = F.num_lights ? 1.0f - (float)F.shadow[(size_t)l * npix + q] / F.shadow_n : 0.0f;
+            d[e] = vlen(v3(N[0], N[1], N[2])) == 0.0f ? -1.0f : dist;   // -1: background
+        }
+        const float t_ao = g == 0 ? A.target_ao[p] : 0.0f;
+        const float t_vis = g == 0 && F.num_lights ? A.target_vis[(size_t)l * npix + p] : 0.0f;
+        // the centre is neighbour 12: element 4 of lane group 1
+        const float dcv = __shfl(d[4], 16 + j);
+        const bool valid = in_frame && dcv >= 0.0f;
+        const float dc = valid ? dcv : 0.0f;
+        // ---- features (all zero for an invalid sample) and the sums of the box base
+        uint4 xb[6];
+        float sa = 0.0f, sv = 0.0f;
+        uint32_t cnt = 0;
+        {
+            float rel[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const bool in = valid && 8 * g + e < 25, bg = d[e] < 0.0f;
+                const float r = dc > 0.0f ? (d[e] - dc) / dc * 16.0f : 0.0f;
+                rel[e] = !in ? 0.0f : (bg ? 1.0f : (r < -1.0f ? -1.0f : (r > 1.0f ? 1.0f : r)));
+                const bool fg = in && !bg;
+                ao[e] = fg ? ao[e] : 0.0f;
+                vis[e] = fg ? vis[e] : 0.0f;
+#pragma unroll
+                for (int c = 0; c < 3; ++c) n3[e][c] = fg ? n3[e][c] : 0.0f;
+                sa += ao[e];
+                sv += vis[e];
+                cnt += fg ? 1u : 0u;
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                xb[s] = make_uint4(bf16_pack2(ao[2 * s], n3[2 * s][0]), bf16_pack2(n3[2 * s][1], n3[2 * s][2]),
+                                   bf16_pack2(ao[2 * s + 1], n3[2 * s + 1][0]),
+                                   bf16_pack2(n3[2 * s + 1][1], n3[2 * s + 1][2]));
+            xb[4] = make_uint4(bf16_pack2(rel[0], rel[1]), bf16_pack2(rel[2], rel[3]), bf16_pack2(rel[4], rel[5]),
+                               bf16_pack2(rel[6], rel[7]));
+            xb[5] = make_uint4(bf16_pack2(vis[0], vis[1]), bf16_pack2(vis[2], vis[3]), bf16_pack2(vis[4], vis[5]),
+                               bf16_pack2(vis[6], vis[7]));
+        }
+#pragma unroll
+        for (int s = 0; s < 6; ++s) A.X[row * (kX / 8) + s * 4 + g] = xb[s];
+        // the base the outputs are added to: the means of the AO fraction and of
+        // the visibility over the window's foreground pixels, summed as k_dn_infer does
+        const uint32_t c = col_sum(cnt);
+        const float fc = (float)(c ? c : 1u);
+        const float bao = col_sum(sa) / fc, bvis = col_sum(sv) / fc;
+        // ---- layer 1: 150 (192) -> 64
+        f32x4 acc[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] = *reinterpret_cast<const f32x4*>(&sbias[16 * t + 4 * g]);
+#pragma unroll
+        for (int s = 0; s < 6; ++s)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                acc[t] = mfma(as_bf16x8(sfrag[(s < 5 ? kFG + t * 5 + s : kFV + t) * 64 + lane]), as_bf16x8(xb[s]),
+                              acc[t]);
+        uint4 hb[2];
+        uint32_t mask[4];
+        // ---- layers 2..4: 64 -> 64
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (k > 0) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) acc[t] = *reinterpret_cast<const f32x4*>(&sbias[k * kHid + 16 * t + 4 * g]);
+                dn_layer64(sfrag, k == 1 ? kF2 : (k == 2 ? kF3 : kF4), lane, hb, acc);
+            }
+            dn_hidden_epilogue(acc, hb, mask[k]);
+            uint4* h = A.H + ((size_t)k * A.cap + row) * 8 + 2 * g;
+            h[0] = hb[0];
+            h[1] = hb[1];
+        }
+        // ---- layer 5: 64 -> 2 in FP32 on layer 4's activations (as in dn_hidden_epilogue)
+        float o0, o1;
+        {
+            f32x4 h[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) h[t][i] = acc[t][i] > 0.0f ? acc[t][i] : 0.0f;
+            dn_out_fp32(h, sw5, g, o0, o1);
+        }
+        // ---- loss and backward
+        float loss = 0.0f, d0 = 0.0f, d1 = 0.0f;
+        if (g == 0 && valid) {
+            const float e0 = (o0 + sbias[4 * kHid]) + bao - t_ao;
+            const float e1 = (o1 + sbias[4 * kHid + 1]) + bvis - t_vis;
+            loss = e0 * e0 + e1 * e1;
+            d0 = A.grad_scale * e0;
+            d1 = A.grad_scale * e1;
+        }
+        const uint32_t b01 = bf16_pack2(d0, d1);
+        if (g == 0) A.Y[row] = b01;
+        // dh4 = W5^T dy
+        const uint4 db = make_uint4(g == 0 ? b01 : 0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            acc[t] = mfma(as_bf16x8(sfrag[(kG5 + t) * 64 + lane]), as_bf16x8(db), f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+        for (int k = 3; k >= 0; --k) {
+            uint4 zb[2];
+            dn_relu_back(acc, mask[k], zb);
+            uint4* z = A.Z + ((size_t)k * A.cap + row) * 8 + 2 * g;
+            z[0] = zb[0];
+            z[1] = zb[1];
+            if (k == 0) break;
+            // dh_{k} = W_{k+1}^T dz_{k+1}  (fragments G2..G4 hold W2^T..W4^T)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            dn_layer64(sfrag, k == 3 ? kG4 : (k == 2 ? kG3 : kG2), lane, zb, acc);
+        }
+        // per-wave loss sum (lanes g == 0 hold the outputs)
+        for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+        if (lane == 0) atomicAdd(A.loss_sum, loss);
+    }
+}
+
+struct InferArgs {
+    DnFrameDev F;
+    const uint4* frags;
+    const float* params;
+    uint32_t lights;    // max(L, 1)
+    uint32_t ntiles;    // 16-pixel tiles of the frame
+    float* ao_out;      // [npix]
+    float* vis_out;     // [L][npix]
+};
+
+// The per-pixel state a tile's light groups share: lane (j, g) holds pixel j
+// of the tile and neighbours 8g + e (e < 8) of its 5x5 window.
+struct InferTile {
+    uint32_t vq[8];   // neighbour indices (0 off the window and for invalid pixels)
+    uint32_t bo[8];   // visibility table offset: 0 for a foreground neighbour, else
+                      // 2048 bytes (the table's zero half)
+    float cnt, bao;   // foreground pixels of the window, box base of AO
+    uint32_t pp;      // pixel index (0 beyond the frame)
+    bool valid, inb;
+};
 
 // Buffer resource over `bytes` bytes at p for raw loads (32-bit offsets in a
 // VGPR, no 64-bit address arithmetic per load).
@@ -837,72 +803,199 @@ __global__ __launch_bounds__(kInferBlock, 2) void k_dn_infer(InferArgs A) {
     }
 }
 
-// dW[o][i] = sum_n dz[o][n] h[i][n] over one chunk of samples, for layer
-// blockIdx.y (0..4); bias gradients = sum_n dz[o][n].  One partial per chunk.
+// dW[o][i] = sum_n dz[o][n] h[i][n] over one chunk of samples, in jobs of 64
+// input positions (blockIdx.y: 0..2 layer 1, whose rows have 192, 3..5 layers
+// 2..4, 6 layer 5); bias gradients = sum_n dz[o][n].  One partial per chunk.
+//
+// The rows are sample-major as k_dn_forward's lanes wrote them (whole lines;
+// the feature-major form they had before was stored in 2-byte pieces and read
+// with a stride of the batch capacity: 105 us for 65536 rows, now 19 us).  Lane
+// (j, g) reads positions 4j .. 4j + 3 of samples 8g .. 8g + 7 of a K-step and
+// transposes them in registers into four fragments, fragment t holding position
+// 4j + t in row j.  A wave takes a quarter of the chunk for all 16 tiles of the
+// job, and the four waves' sums are added in order.
 struct WgArgs {
-    const uint16_t* XT;
-    const uint16_t* HT;
-    const uint16_t* ZT;
-    const uint16_t* YT;
-    uint32_t ldn, rows;
+    const uint2* X;
+    const uint2* H;
+    const uint2* Z;
+    const uint4* Y;
+    uint32_t cap, rows;
     float* partial;   // [chunks][kParams]
 };
+constexpr int kWgJobs = 7;
+
+// The four fragments of rows v[k] (sample k, positions 4j .. 4j + 3).
+__device__ inline void wg_fragments(const uint2 (&v)[8], bf16x8 (&f)[4]) {
+    uint32_t w[4][4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        w[0][m] = __builtin_amdgcn_perm(v[2 * m + 1].x, v[2 * m].x, 0x05040100u);
+        w[1][m] = __builtin_amdgcn_perm(v[2 * m + 1].x, v[2 * m].x, 0x07060302u);
+        w[2][m] = __builtin_amdgcn_perm(v[2 * m + 1].y, v[2 * m].y, 0x05040100u);
+        w[3][m] = __builtin_amdgcn_perm(v[2 * m + 1].y, v[2 * m].y, 0x07060302u);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) f[t] = as_bf16x8(make_uint4(w[t][0], w[t][1], w[t][2], w[t][3]));
+}
+
+// Feature of position p of a 64-wide row.
+__device__ inline int wg_feature(int p) { return 16 * ((p >> 2) & 3) + 4 * (p >> 4) + (p & 3); }
 
 __global__ __launch_bounds__(kBlock) void k_dn_wgrad(WgArgs A) {
-    const int layer = blockIdx.y;
+    __shared__ f32x4 sacc[kBlock / 64][16 * 64];
+    __shared__ f32x4 sb[kBlock / 64][4 * 4];
+    const int job = blockIdx.y, layer = job < 3 ? 0 : job - 2;
+    const bool out = layer == 4;   // the output layer: its dz is the two values of Y
     const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
     const int wave = threadIdx.x >> 6;
-    const uint16_t* Z = layer < 4 ? A.ZT + (size_t)layer * kHid * A.ldn : A.YT;
-    const uint16_t* H = layer == 0 ? A.XT : A.HT + (size_t)(layer - 1) * kHid * A.ldn;
-    const int Mt = layer < 4 ? 4 : 1, Kt = layer == 0 ? 10 : 4;
-    const int nin = layer == 0 ? kIn : kHid, nout = layer < 4 ? kHid : kOut;
+    const uint2* Z = out ? nullptr : A.Z + (size_t)layer * A.cap * 16 + j;
+    const uint32_t hstep = layer == 0 ? kX / 4 : 16;   // 8-byte words of a row
+    const uint2* H = layer == 0 ? A.X + job * 16 + j : A.H + (size_t)(layer - 1) * A.cap * 16 + j;
     const uint32_t n_begin = blockIdx.x * kChunkRows;
     const uint32_t n_end = n_begin + kChunkRows < A.rows ? n_begin + kChunkRows : A.rows;
-    float* part = A.partial + (size_t)blockIdx.x * kParams;
-    for (int tile = wave; tile < Mt * Kt; tile += kBlock / 64) {
-        const int mt = tile / Kt, kt = tile % Kt;
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        const uint16_t* za = Z + (size_t)(16 * mt + j) * A.ldn + 8 * g;
-        const uint16_t* hb = H + (size_t)(16 * kt + j) * A.ldn + 8 * g;
-        for (uint32_t n0 = n_begin; n0 < n_end; n0 += 32) {
-            uint4 a = *reinterpret_cast<const uint4*>(za + n0);
-            uint4 b = *reinterpret_cast<const uint4*>(hb + n0);
-            acc = mfma(as_bf16x8(a), as_bf16x8(b), acc);
+    const bf16x8 ones = as_bf16x8(make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u));
+    f32x4 acc[4][4], bias[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        bias[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[t][u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    // rows are a multiple of 64, so every K-step of 32 samples is whole; the
+    // next K-step's rows are loaded while this one's are multiplied
+    uint2 hv[8], zv[8];
+    auto load = [&](uint32_t n0) {
+        const size_t n = n0 + 8u * (uint32_t)g;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) hv[k] = H[(n + k) * hstep];
+        if (out) {
+            const uint4 ya = A.Y[n / 4], yb = A.Y[n / 4 + 1];
+            zv[0] = make_uint2(ya.x, ya.y);
+            zv[1] = make_uint2(ya.z, ya.w);
+            zv[2] = make_uint2(yb.x, yb.y);
+            zv[3] = make_uint2(yb.z, yb.w);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) zv[k] = Z[(n + k) * 16];
         }
-        const int in = 16 * kt + j;
+    };
+    uint32_t n0 = n_begin + 32u * (uint32_t)wave;
+    if (n0 < n_end) load(n0);
+    while (n0 < n_end) {
+        bf16x8 fz[4], fh[4];
+        wg_fragments(hv, fh);
+        if (out) {
+            // row j < 2 is output j: its half of each sample's pair
+            const uint32_t sel = j == 0 ? 0x05040100u : 0x07060302u;
+            uint32_t w[4];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) w[m] = j < 2 ? __builtin_amdgcn_perm(zv[m].y, zv[m].x, sel) : 0u;
+            fz[0] = as_bf16x8(make_uint4(w[0], w[1], w[2], w[3]));
+        } else {
+            wg_fragments(zv, fz);
+        }
+        n0 += 32u * (kBlock / 64);
+        if (n0 < n_end) load(n0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            if (out && t > 0) break;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[t][u] = mfma(fz[t], fh[u], acc[t][u]);
+            bias[t] = mfma(fz[t], ones, bias[t]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sacc[wave][(t * 4 + u) * 64 + lane] = acc[t][u];
+        if (j == 0) sb[wave][t * 4 + g] = bias[t];
+    }
+    __syncthreads();
+    // wave t adds the tiles (t, 0..3) of the four waves: lane (j, g), element i
+    // is dz row 4g + i (position 4 (4g + i) + t), input column j (position 4j + u)
+    const int t = wave;
+    if (out && t > 0) return;
+    const int nin = layer == 0 ? kIn : kHid;
+    float* part = A.partial + (size_t)blockIdx.x * kParams;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        f32x4 v = sacc[0][(t * 4 + u) * 64 + lane];
+        for (int w = 1; w < kBlock / 64; ++w) v += sacc[w][(t * 4 + u) * 64 + lane];
+        int in = 4 * j + u;
+        if (layer == 0) {
+            const int q = 64 * job + in;
+            in = infer_feature(q / 32, (q & 31) >> 3, q & 7);
+        } else {
+            in = wg_feature(in);
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int o = 16 * mt + 4 * g + i;
-            if (o < nout && in < nin) part[kWOff[layer] + o * nin + in] = acc[i];
+            const int r = 4 * g + i, o = out ? r : wg_feature(4 * r + t);
+            if (in >= 0 && (!out || r < kOut)) part[kWOff[layer] + o * nin + in] = v[i];
         }
     }
-    // bias: four threads per output row, each a quarter of the chunk
-    for (int r = threadIdx.x; r < nout * 4; r += kBlock) {
-        const int o = r >> 2, part4 = r & 3;
-        const uint16_t* zr = Z + (size_t)o * A.ldn;
-        float s = 0.0f;
-        for (uint32_t n = n_begin + part4 * 8; n < n_end; n += 32) {
-            uint4 v = *reinterpret_cast<const uint4*>(zr + n);
-            const uint32_t ws[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) s += bf16_val((ws[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
+    if (j == 0 && (job == 0 || job >= 3)) {
+        f32x4 v = sb[0][t * 4 + g];
+        for (int w = 1; w < kBlock / 64; ++w) v += sb[w][t * 4 + g];
+        for (int i = 0; i < 4; ++i) {
+            const int r = 4 * g + i;
+            if (!out || r < kOut) part[kBOff[layer] + (out ? r : wg_feature(4 * r + t))] = v[i];
         }
-        s += __shfl_xor(s, 1);
-        s += __shfl_xor(s, 2);
-        if (part4 == 0) part[kBOff[layer] + o] = s;
     }
 }
 
-__global__ void k_dn_reduce(const float* partial, uint32_t chunks, float* grad) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint32_t)kParams) return;
+// The chunk partials added in order, four threads per parameter (each a
+// quarter of the chunks, so that the loads of a long batch overlap).
+__global__ __launch_bounds__(kBlock) void k_dn_reduce(const float* partial, uint32_t chunks, float* grad) {
+    __shared__ float sh[kBlock];
+    const uint32_t i = blockIdx.x * (kBlock / 4) + (threadIdx.x & 63u), q = threadIdx.x >> 6;
+    const uint32_t per = (chunks + 3) / 4, c0 = q * per, c1 = c0 + per < chunks ? c0 + per : chunks;
     float s = 0.0f;
-    for (uint32_t c = 0; c < chunks; ++c) s += partial[(size_t)c * kParams + i];
-    grad[i] = s;
+    if (i < (uint32_t)kParams) {
+#pragma unroll 8
+        for (uint32_t c = c0; c < c1; ++c) s += partial[(size_t)c * kParams + i];
+    }
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    if (q == 0 && i < (uint32_t)kParams) grad[i] = ((sh[threadIdx.x] + sh[64 + threadIdx.x]) + sh[128 + threadIdx.x]) + sh[192 + threadIdx.x];
 }
 
+// Writes parameter i (value w) to its places in the BF16 fragments.
+__device__ inline void dn_pack_param(uint32_t i, float w, uint16_t* frags) {
+    auto put = [&](int f, int row, int g, int e, float v) {
+        frags[((size_t)f * 64 + row + 16 * g) * 8 + e] = (uint16_t)bf16_bits(v);
+    };
+    // K-step, lane group and element of hidden feature k (the inverse of khid)
+    auto ks = [](int k) { return k >> 5; };
+    auto kg = [](int k) { return (k >> 2) & 3; };
+    auto ke = [](int k) { return ((k >> 4) & 1) * 4 + (k & 3); };
+    const int p = (int)i;
+    if (p < oB1) {
+        const int o = p / kIn, k = p % kIn, n = k / 6, c = k % 6, g = n >> 3, m = n & 7, t = o >> 4;
+        if (c == 1) put(kFV + t, o & 15, g, m, w);
+        else if (c == 2) put(kFG + t * 5 + 4, o & 15, g, m, w);
+        else put(kFG + t * 5 + (m >> 1), o & 15, g, (m & 1) * 4 + (c == 0 ? 0 : c - 2), w);
+        return;
+    }
+    for (int layer = 1; layer < 4; ++layer) {
+        const int q = p - kWOff[layer];
+        if (q < 0 || q >= kHid * kHid) continue;
+        const int o = q / kHid, k = q % kHid;
+        put(kF2 + (layer - 1) * 8 + (o >> 4) * 2 + ks(k), o & 15, kg(k), ke(k), w);
+        put(kG2 + (layer - 1) * 8 + (k >> 4) * 2 + ks(o), k & 15, kg(o), ke(o), w);
+    }
+    if (p >= oW5 && p < oB5) {
+        const int o = (p - oW5) / kHid, k = (p - oW5) % kHid;
+        put(kG5 + (k >> 4), k & 15, 0, o, w);
+        const float hi = bf16_val(bf16_bits(w));
+        put(kF5 + ks(k), o, kg(k), ke(k), hi);
+        put(kF5 + ks(k), o + 2, kg(k), ke(k), w - hi);
+    }
+}
+
+// One Adam step; each thread re-packs the parameter it updates.
 __global__ void k_dn_adam(float* params, float* m, float* v, const float* grad, float lr_t, float b1,
-                          float b2, float eps) {
+                          float b2, float eps, uint16_t* frags) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (uint32_t)kParams) return;
     float gr = grad[i];
@@ -910,38 +1003,16 @@ __global__ void k_dn_adam(float* params, float* m, float* v, const float* grad, 
     float vi = b2 * v[i] + (1.0f - b2) * gr * gr;
     m[i] = mi;
     v[i] = vi;
-    params[i] -= lr_t * mi / (sqrtf(vi) + eps);
+    const float w = params[i] - lr_t * mi / (sqrtf(vi) + eps);
+    params[i] = w;
+    dn_pack_param(i, w, frags);
 }
 
-// BF16 fragments of every weight matrix from the FP32 master copy.
+// BF16 fragments of every weight matrix from the FP32 master copy (positions
+// that hold no parameter were zeroed when the fragments were allocated).
 __global__ void k_dn_pack(const float* P, uint16_t* frags) {
-    const uint32_t id = blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= (uint32_t)kFragAll * 64 * 8) return;
-    const int f = id / 512, l = (id / 8) % 64, e = id % 8;
-    const int j = l & 15, g = l >> 4;
-    float val = 0.0f;
-    if (f < kF2) {
-        const int t = f / 5, s = f % 5, o = 16 * t + j, k = 32 * s + 8 * g + e;
-        if (k < kIn) val = P[oW1 + o * kIn + k];
-    } else if (f < kG2) {
-        const int layer = 1 + (f - kF2) / 8, r = (f - kF2) % 8, t = r / 2, s = r % 2;
-        val = P[kWOff[layer] + (16 * t + j) * kHid + khid(s, g, e)];
-    } else if (f < kG5) {
-        const int layer = 1 + (f - kG2) / 8, r = (f - kG2) % 8, t = r / 2, s = r % 2;
-        val = P[kWOff[layer] + khid(s, g, e) * kHid + (16 * t + j)];
-    } else if (f < kFG) {
-        const int t = f - kG5, o = khid(0, g, e);
-        if (o < kOut) val = P[oW5 + o * kHid + (16 * t + j)];
-    } else if (f < kF5) {
-        const int t = f < kFV ? (f - kFG) / 5 : f - kFV, s = f < kFV ? (f - kFG) % 5 : 5;
-        const int k = infer_feature(s, g, e);
-        if (k >= 0) val = P[oW1 + (16 * t + j) * kIn + k];
-    } else if (j < 4) {
-        const float w = P[oW5 + (j & 1) * kHid + khid(f - kF5, g, e)];
-        const float hi = bf16_val(bf16_bits(w));
-        val = j < 2 ? hi : w - hi;
-    }
-    frags[id] = (uint16_t)bf16_bits(val);
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < (uint32_t)kParams) dn_pack_param(i, P[i], frags);
 }
 
 // Input features of explicit samples, [count][150] BF16 bits (inspection).
@@ -983,10 +1054,10 @@ struct luzrt_denoiser {
     float* partial = nullptr;
     float* loss = nullptr;     // device loss sum
     uint16_t* frags = nullptr;
-    uint16_t* XT = nullptr;
-    uint16_t* HT = nullptr;
-    uint16_t* ZT = nullptr;
-    uint16_t* YT = nullptr;
+    uint4* X = nullptr;
+    uint4* H = nullptr;
+    uint4* Z = nullptr;
+    uint32_t* Y = nullptr;
     DevBuf pix, ao_frac;    // prepass planes of the current frame
 };
 
@@ -994,8 +1065,8 @@ namespace {
 
 void dn_free(luzrt_denoiser* d) {
     for (void* p : {(void*)d->params, (void*)d->grad, (void*)d->adam_m, (void*)d->adam_v,
-                    (void*)d->partial, (void*)d->loss, (void*)d->frags, (void*)d->XT, (void*)d->HT,
-                    (void*)d->ZT, (void*)d->YT, d->pix.ptr, d->ao_frac.ptr})
+                    (void*)d->partial, (void*)d->loss, (void*)d->frags, (void*)d->X, (void*)d->H,
+                    (void*)d->Z, (void*)d->Y, d->pix.ptr, d->ao_frac.ptr})
         if (p) (void)hipFree(p);
     delete d;
 }
@@ -1035,8 +1106,7 @@ luzrt_status prep_frame(luzrt_ctx* ctx, DnFrameDev& F, DevBuf& pix, DevBuf& ao_f
 }
 
 luzrt_status repack(luzrt_ctx* ctx, luzrt_denoiser* d) {
-    const uint32_t n = kFragAll * 64 * 8;
-    k_dn_pack<<<cdiv(n, 256), 256, 0, ctx->stream>>>(d->params, d->frags);
+    k_dn_pack<<<cdiv(kParams, 256), 256, 0, ctx->stream>>>(d->params, d->frags);
     LUZ_HIP(ctx, hipGetLastError());
     return LUZRT_OK;
 }
@@ -1061,15 +1131,15 @@ luzrt_status luzrt_denoiser_create(luzrt_ctx* ctx, uint32_t batch_capacity, uint
     struct A { void** p; size_t bytes; } allocs[] = {
         {(void**)&d->params, pb}, {(void**)&d->grad, pb}, {(void**)&d->adam_m, pb},
         {(void**)&d->adam_v, pb}, {(void**)&d->partial, pb * chunks}, {(void**)&d->loss, 256},
-        {(void**)&d->frags, (size_t)kFragAll * 1024}, {(void**)&d->XT, (size_t)160 * cap * 2},
-        {(void**)&d->HT, (size_t)4 * kHid * cap * 2}, {(void**)&d->ZT, (size_t)4 * kHid * cap * 2},
-        {(void**)&d->YT, (size_t)16 * cap * 2}};
+        {(void**)&d->frags, (size_t)kFragAll * 1024}, {(void**)&d->X, (size_t)kX * cap * 2},
+        {(void**)&d->H, (size_t)4 * kHid * cap * 2}, {(void**)&d->Z, (size_t)4 * kHid * cap * 2},
+        {(void**)&d->Y, (size_t)cap * 4}};
     for (auto& a : allocs) {
         hipError_t e = hipMalloc(a.p, a.bytes);
         if (e != hipSuccess) { dn_free(d); return hip_fail(ctx, e, "hipMalloc(denoiser)"); }
     }
-    // rows 2..15 of dy are never written: zero them once
-    LUZ_HIP(ctx, hipMemset(d->YT, 0, (size_t)16 * cap * 2));
+    // fragment positions that hold no parameter stay zero
+    LUZ_HIP(ctx, hipMemset(d->frags, 0, (size_t)kFragAll * 1024));
     LUZ_HIP(ctx, hipMemset(d->adam_m, 0, pb));
     LUZ_HIP(ctx, hipMemset(d->adam_v, 0, pb));
     LUZ_HIP(ctx, hipMemset(d->grad, 0, pb));
@@ -1195,7 +1265,6 @@ luzrt_status luzrt_denoiser_accumulate(luzrt_ctx* ctx, luzrt_denoiser* d, const 
     luzrt_status s = frame_dev(ctx, f, A.F);
     if (s != LUZRT_OK) return s;
     if (count == 0) return LUZRT_OK;
-    if ((s = prep_frame(ctx, A.F, d->pix, d->ao_frac)) != LUZRT_OK) return s;
     A.frags = reinterpret_cast<const uint4*>(d->frags);
     A.params = d->params;
     A.nsamples = count;
@@ -1204,17 +1273,19 @@ luzrt_status luzrt_denoiser_accumulate(luzrt_ctx* ctx, luzrt_denoiser* d, const 
     A.target_ao = target_ao;
     A.target_vis = target_vis;
     A.row_base = d->rows;
-    A.ldn = d->capacity;
-    A.XT = d->XT;
-    A.HT = d->HT;
-    A.ZT = d->ZT;
-    A.YT = d->YT;
+    A.cap = d->capacity;
+    A.X = d->X;
+    A.H = d->H;
+    A.Z = d->Z;
+    A.Y = d->Y;
     A.grad_scale = grad_scale;
     A.loss_sum = d->loss;
-    uint32_t groups = cdiv(count, kBlock);
-    const uint32_t maxg = (uint32_t)(ctx->num_cus > 0 ? ctx->num_cus : 1) * 4;
+    // one 16-sample tile per wave, up to the two groups per CU that their
+    // fragments in LDS leave room for
+    uint32_t groups = cdiv(count, 16 * (kBlock / 64));
+    const uint32_t maxg = (uint32_t)(ctx->num_cus > 0 ? ctx->num_cus : 1) * 2;
     if (groups > maxg) groups = maxg;
-    k_dn_forward<4><<<groups, kBlock, 0, ctx->stream>>>(A);
+    k_dn_forward<<<groups, kBlock, 0, ctx->stream>>>(A);
     LUZ_HIP(ctx, hipGetLastError());
     d->rows += count;
     return LUZRT_OK;
@@ -1225,10 +1296,11 @@ luzrt_status luzrt_denoiser_gradient(luzrt_ctx* ctx, luzrt_denoiser* d, float* h
     if (!d) return fail(ctx, LUZRT_E_INVALID_ARG, "luzrt_denoiser_gradient: null denoiser");
     hipStream_t st = ctx->stream;
     if (d->rows > 0) {
-        WgArgs W{d->XT, d->HT, d->ZT, d->YT, d->capacity, d->rows, d->partial};
+        WgArgs W{(const uint2*)d->X, (const uint2*)d->H, (const uint2*)d->Z, (const uint4*)d->Y, d->capacity, d->rows,
+                 d->partial};
         const uint32_t chunks = cdiv(d->rows, kChunkRows);
-        k_dn_wgrad<<<dim3(chunks, 5), kBlock, 0, st>>>(W);
-        k_dn_reduce<<<cdiv(kParams, 256), 256, 0, st>>>(d->partial, chunks, d->grad);
+        k_dn_wgrad<<<dim3(chunks, kWgJobs), kBlock, 0, st>>>(W);
+        k_dn_reduce<<<cdiv(kParams, kBlock / 4), kBlock, 0, st>>>(d->partial, chunks, d->grad);
         LUZ_HIP(ctx, hipGetLastError());
     } else {
         LUZ_HIP(ctx, hipMemsetAsync(d->grad, 0, (size_t)kParams * 4, st));
@@ -1252,9 +1324,9 @@ luzrt_status luzrt_denoiser_adam(luzrt_ctx* ctx, luzrt_denoiser* d, float lr, fl
     double c2 = 1.0 - std::pow((double)beta2, (double)d->step);
     float lr_t = (float)(lr * std::sqrt(c2) / c1);
     k_dn_adam<<<cdiv(kParams, 256), 256, 0, ctx->stream>>>(d->params, d->adam_m, d->adam_v, d->grad, lr_t,
-                                                          beta1, beta2, eps);
+                                                          beta1, beta2, eps, d->frags);
     LUZ_HIP(ctx, hipGetLastError());
-    return repack(ctx, d);
+    return LUZRT_OK;
 }
 
 }  // extern "C"

@@ -135,6 +135,53 @@ def test_gradient_matches_fp64_oracle_and_is_deterministic(ctx, frame):
     dn.close()
 
 
+@pytest.mark.parametrize("nl,counts", [(0, [64]), (1, [64, 1024]), (9, [1024, 1088])])
+def test_gradient_of_ragged_batches(ctx, frame, nl, counts):
+    """Batches of one and of several calls that end inside a chunk of 1024 rows and below
+    the capacity, with border pixels and samples that contribute nothing (background,
+    outside the frame, no such light).  BF16 activations (2^-9 per term) bound the error as
+    in the test above; 64 samples average less of it, hence 3e-2."""
+    n, N = frame.width * frame.height, sum(counts)
+    sh = frame.shadow.download(np.uint8, (frame.num_lights, n))[:max(nl, 1)]
+    vis = frame.target_vis_host[:max(nl, 1)].astype(np.float32)
+    sub = dnm.Frame(ctx, frame.width, frame.height, frame.position, frame.normal, frame.cam_pos, nl,
+                    ctx.to_device(np.ascontiguousarray(sh)), frame.shadow_samples, frame.ao, frame.ao_samples)
+    sub.target_ao, sub.target_vis = frame.target_ao, ctx.to_device(np.ascontiguousarray(vis))
+    dn = dnm.Denoiser(ctx, N + 2048 - N % 64, seed=1)
+    dn.params = _params(9)
+    rng = np.random.default_rng(nl + N)
+    px = frame.foreground[rng.integers(0, len(frame.foreground), N)].astype(np.int64)
+    edge = frame.foreground[(frame.foreground % frame.width < 2) | (frame.foreground // frame.width > frame.height - 3)]
+    px[:len(edge[:20])] = edge[:20]
+    li = rng.integers(0, max(nl, 1), N)
+    bg = np.setdiff1d(np.arange(n), frame.foreground)
+    dead = np.zeros(N, bool)
+    dead[40:46] = True
+    px[40:44], li[44:46] = n + np.arange(4), 70
+    if len(bg):
+        dead[46:50] = True
+        px[46:50] = bg[:4] if len(bg) >= 4 else bg[0]
+    at = 0
+    for c in counts:
+        buf = ctx.to_device((px[at:at + c] | (li[at:at + c] << 24)).astype(np.uint32))
+        dn.accumulate(sub, buf, c, 1.0 / N)
+        at += c
+    got, _ = dn.gradient(host=True)
+    px, li = px[~dead], li[~dead]
+    host = sub.host()
+    X = odn.features(host, px, li)
+    T = np.stack([frame.target_ao_host[px], vis[li, px] if nl else np.zeros(len(px))], 1).astype(np.float64)
+    want = odn.backward(odn.device_weights(dn.params), X, T - odn.box_base(host, px, li), scale=1.0 / N)
+    o = 0
+    for k, shape in enumerate(odn.SHAPES):
+        m = int(np.prod(shape))
+        rel = np.linalg.norm(got[o:o + m] - want[o:o + m]) / max(np.linalg.norm(want[o:o + m]), 1e-30)
+        print(f"param block {k} {shape}: rel err {rel:.2e}", flush=True)
+        assert rel < 3e-2
+        o += m
+    dn.close()
+
+
 def test_training_on_tracer_pairs_reduces_error(ctx):
     frames = [dnm.make_frame(ctx, 200 + i, crop=(64, 64), target_spp=64, focus="instance") for i in range(16)]
     held = dnm.make_frame(ctx, 300, crop=(128, 128), target_spp=128, focus="instance")
