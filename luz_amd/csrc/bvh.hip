@@ -492,65 +492,262 @@ __global__ void k_small_root(const uint8_t* verts, uint32_t stride, uint32_t nv,
 }
 
 // ---------------------------------------------------------------- 8-wide form
-// Collapse of the binary LBVH into 8-wide nodes, one breadth-first level per
-// pass: k_wide_collapse lists each wide node's slots (repeatedly replacing the
-// internal slot of largest surface area, first on ties, by its two children),
-// two scans number the next level's nodes and this level's leaves, and
-// k_wide_emit quantises the child boxes and writes nodes and leaf triangles.
-struct WRef {
-    uint32_t c;
-    float lo[3], hi[3];
-    uint32_t pad;
+// Collapse of the binary LBVH into 8-wide nodes, numbered breadth first.  The
+// eight slots of a wide node depend on its binary root alone, so the long part
+// needs no order: k_wide_slots lists them for every binary node at once.  What
+// goes level by level is only the numbering (k_wide_number, one workgroup per
+// BLAS, or k_wide_level_* with the whole chip for large ones), and k_wide_emit
+// then writes all wide nodes together.  One launch of each serves up to
+// kWideJobs BLASes and the host waits for none of it.  (With the slots found
+// level by level, seven launches and copies and a wait for the host per level,
+// five 20,480-triangle meshes took 3.3 ms, now WIDE_T us.)
+struct WideJob {
+    const Node* bn;
+    const uint32_t* leaf_parent;
+    const float* tris;
+    const uint32_t* prims;
+    uint4* slots;          // two per binary node: its 8 slots, left to right (kEmpty: none)
+    uint32_t* root;        // per wide node: its binary root
+    uint32_t* child_base;  // first child and first triangle of a wide node
+    uint32_t* tri_base;
+    Node8* out;
+    float* tris8;
+    uint32_t* prims8;
+    uint32_t* count;       // wide nodes
+    uint32_t n;            // binary nodes
+    uint32_t block;        // first workgroup of this job in a launch over all jobs' nodes
 };
+constexpr uint32_t kWideJobs = 8;
+struct WideJobs {
+    uint32_t n, pad;
+    WideJob j[kWideJobs];
+};
+
+__device__ inline const WideJob& wide_job_of(const WideJobs& J, uint32_t block) {
+    uint32_t k = 0;
+    while (k + 1 < J.n && J.j[k + 1].block <= block) ++k;
+    return J.j[k];
+}
 
 __device__ inline float surface_area(const float* lo, const float* hi) {
     float dx = hi[0] - lo[0], dy = hi[1] - lo[1], dz = hi[2] - lo[2];
     return dx * dy + dy * dz + dz * dx;
 }
 
-__device__ inline WRef child_ref(const Node& n, int c) {
-    WRef r;
-    r.c = n.child[c];
-    r.lo[0] = n.lox[c]; r.lo[1] = n.loy[c]; r.lo[2] = n.loz[c];
-    r.hi[0] = n.hix[c]; r.hi[1] = n.hiy[c]; r.hi[2] = n.hiz[c];
-    r.pad = 0;
-    return r;
+__device__ inline float child_area(const Node& n, int c) {
+    const float lo[3] = {n.lox[c], n.loy[c], n.loz[c]}, hi[3] = {n.hix[c], n.hiy[c], n.hiz[c]};
+    return surface_area(lo, hi);
 }
 
-__global__ __launch_bounds__(kBlock) void k_wide_collapse(const Node* bn, const uint32_t* level,
-                                                          uint32_t count, WRef* slots_out,
-                                                          uint32_t* nslots, uint32_t* n_int,
-                                                          uint32_t* n_leaf) {
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= count) return;
-    WRef s[8];
+// The slots of the wide node rooted at each binary node: its two children, then
+// repeatedly the internal slot of largest surface area, first on ties, replaced
+// in place by its two children.  Bound by the chain of up to six node reads;
+// the slots stay in registers (every index is a constant after unrolling).
+__global__ __launch_bounds__(kBlock) void k_wide_slots(WideJobs jobs) {
+    const WideJob& J = wide_job_of(jobs, blockIdx.x);
+    const uint32_t i = (blockIdx.x - J.block) * kBlock + threadIdx.x;
+    if (i >= J.n) return;
+    uint32_t c[8];
+    float sa[8];
     int n = 0;
-    const Node& root = bn[level[i]];
-    for (int c = 0; c < 2; ++c)
-        if (root.child[c] != kEmpty) s[n++] = child_ref(root, c);
+    {
+        const Node nd = J.bn[i];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) { c[k] = kEmpty; sa[k] = 0.0f; }
+        c[0] = nd.child[0];
+        sa[0] = child_area(nd, 0);
+        n = c[0] != kEmpty ? 1 : 0;
+        if (nd.child[1] != kEmpty) {
+            c[1] = nd.child[1];
+            sa[1] = child_area(nd, 1);
+            n = 2;
+        }
+    }
     while (n < 8) {
         int best = -1;
         float best_sa = 0.0f;
-        for (int k = 0; k < n; ++k) {
-            if (s[k].c & kLeaf) continue;
-            float sa = surface_area(s[k].lo, s[k].hi);
-            if (best < 0 || sa > best_sa) { best = k; best_sa = sa; }
-        }
+        uint32_t bc = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)   // kEmpty has the leaf bit
+            if (!(c[k] & kLeaf) && (best < 0 || sa[k] > best_sa)) { best = k; best_sa = sa[k]; bc = c[k]; }
         if (best < 0) break;
-        const Node& in = bn[s[best].c];
-        for (int k = n; k > best + 1; --k) s[k] = s[k - 1];
-        s[best] = child_ref(in, 0);
-        s[best + 1] = child_ref(in, 1);
+        const Node nd = J.bn[bc];
+        const float a0 = child_area(nd, 0), a1 = child_area(nd, 1);
+#pragma unroll
+        for (int k = 7; k > 0; --k) {
+            if (k > best + 1) { c[k] = c[k - 1]; sa[k] = sa[k - 1]; }
+            else if (k == best + 1) { c[k] = nd.child[1]; sa[k] = a1; }
+            else if (k == best) { c[k] = nd.child[0]; sa[k] = a0; }
+        }
+        if (best == 0) { c[0] = nd.child[0]; sa[0] = a0; }
         ++n;
     }
-    uint32_t ni = 0, nl = 0;
-    for (int k = 0; k < n; ++k) {
-        slots_out[(size_t)i * 8 + k] = s[k];
-        if (s[k].c & kLeaf) ++nl; else ++ni;
+    J.slots[2 * (size_t)i] = make_uint4(c[0], c[1], c[2], c[3]);
+    J.slots[2 * (size_t)i + 1] = make_uint4(c[4], c[5], c[6], c[7]);
+}
+
+__device__ inline void slot_array(uint4 a, uint4 b, uint32_t (&c)[8]) {
+    c[0] = a.x; c[1] = a.y; c[2] = a.z; c[3] = a.w;
+    c[4] = b.x; c[5] = b.y; c[6] = b.z; c[7] = b.w;
+}
+
+// Internal (low half) and leaf (high half) slots.
+__device__ inline uint32_t slot_counts(const uint32_t (&c)[8]) {
+    uint32_t k = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) k += c[i] == kEmpty ? 0u : ((c[i] & kLeaf) ? 0x10000u : 1u);
+    return k;
+}
+
+// Exclusive prefix of v among the workgroup's threads (thread order) and its
+// total; the halves of v are summed apart (8 x 1024 fits 16 bits).  sums: one
+// word per wave.
+__device__ inline uint32_t block_prefix_sum(uint32_t v, uint32_t* sums, uint32_t& total) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint32_t incl = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(incl, off);
+        if (lane >= (uint32_t)off) incl += y;
     }
-    nslots[i] = (uint32_t)n;
-    n_int[i] = ni;
-    n_leaf[i] = nl;
+    if (lane == 63) sums[wave] = incl;
+    __syncthreads();
+    uint32_t before = 0;
+    total = 0;
+    for (uint32_t w = 0; w < blockDim.x / 64; ++w) {
+        const uint32_t t = sums[w];
+        if (w < wave) before += t;
+        total += t;
+    }
+    __syncthreads();
+    return before + incl - v;
+}
+
+// Numbers wide node w (of binary root whose slots are c) given the first child
+// and triangle its level has left for it, and lists its children's roots.
+__device__ inline void wide_place(const WideJob& J, uint32_t w, const uint32_t (&c)[8], uint32_t child, uint32_t tri) {
+    J.child_base[w] = child;
+    J.tri_base[w] = tri;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        if (!(c[k] & kLeaf)) J.root[child++] = c[k];
+}
+
+// Breadth-first numbering of one BLAS by one workgroup: per level, running
+// sums of the nodes' child and triangle counts.  About 2 us per 1024 wide nodes.
+__global__ __launch_bounds__(1024) void k_wide_number(WideJobs jobs) {
+    __shared__ uint32_t sums[1024 / 64];
+    const WideJob& J = jobs.j[blockIdx.x];
+    if (threadIdx.x == 0) J.root[0] = 0;
+    uint32_t start = 0, count = 1, tri = 0;
+    while (count > 0) {
+        __syncthreads();   // the level's roots are written
+        const uint32_t next = start + count;
+        uint32_t children = 0, leaves = 0;
+        for (uint32_t base = 0; base < count; base += 1024) {
+            const uint32_t i = base + threadIdx.x, w = start + i;
+            uint32_t c[8] = {kEmpty, kEmpty, kEmpty, kEmpty, kEmpty, kEmpty, kEmpty, kEmpty};
+            if (i < count) {
+                const uint32_t r = J.root[w];
+                slot_array(J.slots[2 * (size_t)r], J.slots[2 * (size_t)r + 1], c);
+            }
+            uint32_t total;
+            const uint32_t pre = block_prefix_sum(slot_counts(c), sums, total);
+            if (i < count) wide_place(J, w, c, next + children + (pre & 0xFFFFu), tri + leaves + (pre >> 16));
+            children += total & 0xFFFFu;
+            leaves += total >> 16;
+        }
+        tri += leaves;
+        start = next;
+        count = children;
+    }
+    if (threadIdx.x == 0) *J.count = start;
+}
+
+// The same for one large BLAS, a level per pair of launches: workgroup b takes
+// the b-th run of the level's nodes, k_wide_level_count sums the runs and
+// k_wide_level_write numbers them.  levels[l] = (first wide node, nodes, first
+// triangle) of level l.
+constexpr uint32_t kWideLevelBlocks = 512;
+__device__ inline uint32_t level_run(uint32_t count) {
+    return (count + kWideLevelBlocks * kBlock - 1) / (kWideLevelBlocks * kBlock) * kBlock;
+}
+
+__global__ __launch_bounds__(kBlock) void k_wide_level_count(WideJob J, const uint3* level, uint2* run_sums) {
+    __shared__ uint32_t sums[kBlock / 64];
+    const uint3 L = *level;
+    const uint32_t per = level_run(L.y), begin = blockIdx.x * per;
+    const uint32_t end = begin + per < L.y ? begin + per : L.y;
+    uint2 s = make_uint2(0u, 0u);
+    for (uint32_t base = begin; base < end; base += kBlock) {
+        const uint32_t i = base + threadIdx.x;
+        uint32_t v = 0, total;
+        if (i < end) {
+            uint32_t c[8];
+            const uint32_t r = J.root[L.x + i];
+            slot_array(J.slots[2 * (size_t)r], J.slots[2 * (size_t)r + 1], c);
+            v = slot_counts(c);
+        }
+        block_prefix_sum(v, sums, total);
+        s.x += total & 0xFFFFu;
+        s.y += total >> 16;
+    }
+    if (threadIdx.x == 0) run_sums[blockIdx.x] = s;
+}
+
+__global__ __launch_bounds__(kBlock) void k_wide_level_write(WideJob J, uint3* level, const uint2* run_sums) {
+    __shared__ uint32_t sums[kBlock / 64];
+    __shared__ uint32_t s_red[4];   // children, leaves before this run; in the level
+    const uint3 L = *level;
+    if (L.y == 0) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            level[1] = make_uint3(L.x, 0u, L.z);
+            *J.count = L.x;
+        }
+        return;
+    }
+    if (threadIdx.x < 4) s_red[threadIdx.x] = 0;
+    __syncthreads();
+    uint32_t a = 0, b = 0, ta = 0, tb = 0;
+    for (uint32_t k = threadIdx.x; k < kWideLevelBlocks; k += kBlock) {
+        const uint2 v = run_sums[k];
+        ta += v.x;
+        tb += v.y;
+        if (k < blockIdx.x) { a += v.x; b += v.y; }
+    }
+    atomicAdd(&s_red[0], a);
+    atomicAdd(&s_red[1], b);
+    atomicAdd(&s_red[2], ta);
+    atomicAdd(&s_red[3], tb);
+    __syncthreads();
+    const uint32_t next = L.x + L.y;
+    uint32_t child = next + s_red[0], tri = L.z + s_red[1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        level[1] = make_uint3(next, s_red[2], L.z + s_red[3]);
+        *J.count = next;
+    }
+    const uint32_t per = level_run(L.y), begin = blockIdx.x * per;
+    const uint32_t end = begin + per < L.y ? begin + per : L.y;
+    for (uint32_t base = begin; base < end; base += kBlock) {
+        const uint32_t i = base + threadIdx.x;
+        uint32_t c[8] = {kEmpty, kEmpty, kEmpty, kEmpty, kEmpty, kEmpty, kEmpty, kEmpty}, total;
+        if (i < end) {
+            const uint32_t r = J.root[L.x + i];
+            slot_array(J.slots[2 * (size_t)r], J.slots[2 * (size_t)r + 1], c);
+        }
+        const uint32_t pre = block_prefix_sum(slot_counts(c), sums, total);
+        if (i < end) wide_place(J, L.x + i, c, child + (pre & 0xFFFFu), tri + (pre >> 16));
+        child += total & 0xFFFFu;
+        tri += total >> 16;
+    }
+}
+
+// The first level of a large BLAS: its root.
+__global__ void k_wide_level_init(WideJob J, uint3* level) {
+    if (threadIdx.x == 0) {
+        J.root[0] = 0;
+        level[0] = make_uint3(0u, 1u, 0u);
+    }
 }
 
 __device__ inline void quant_frame(float lo, float hi, float& origin, int& e) {
@@ -570,66 +767,89 @@ __device__ inline void quant_frame(float lo, float hi, float& origin, int& e) {
     }
 }
 
-__device__ inline uint8_t quant_lo(float v, float origin, float sc) {
-    float q = floorf((v - origin) / sc);
+// Quantised bounds: (v - origin) / 2^e by the exact reciprocal of the scale.
+__device__ inline uint32_t quant_lo(float v, float origin, float sc, float inv) {
+    float q = floorf((v - origin) * inv);
     q = q < 0.0f ? 0.0f : (q > 255.0f ? 255.0f : q);
     while (q > 0.0f && origin + q * sc > v) q = q - 1.0f;
-    return (uint8_t)q;
+    return (uint32_t)(uint8_t)q;
 }
 
-__device__ inline uint8_t quant_hi(float v, float origin, float sc) {
-    float q = ceilf((v - origin) / sc);
+__device__ inline uint32_t quant_hi(float v, float origin, float sc, float inv) {
+    float q = ceilf((v - origin) * inv);
     q = q < 0.0f ? 0.0f : (q > 255.0f ? 255.0f : q);
     while (q < 255.0f && origin + q * sc < v) q = q + 1.0f;
-    return (uint8_t)q;
+    return (uint32_t)(uint8_t)q;
 }
 
-__global__ __launch_bounds__(kBlock) void k_wide_emit(const WRef* slots, const uint32_t* nslots,
-                                                      uint32_t count, uint32_t level_start,
-                                                      uint32_t next_start, uint32_t tri_start,
-                                                      const uint32_t* int_off,
-                                                      const uint32_t* leaf_off, Node8* out,
-                                                      uint32_t* next_level, const float* tris,
-                                                      const uint32_t* prims, float* tris8,
-                                                      uint32_t* prims8) {
-    uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= count) return;
-    const uint32_t n = nslots[i];
-    const WRef* s = slots + (size_t)i * 8;
-    Node8 w;
-    uint32_t* wz = reinterpret_cast<uint32_t*>(&w);
-    for (int k = 0; k < 24; ++k) wz[k] = 0;
-    w.nchild = (uint8_t)n;
-    w.child_base = next_start + int_off[i];
-    w.tri_base = tri_start + leaf_off[i];
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (uint32_t k = 0; k < n; ++k)
-        for (int a = 0; a < 3; ++a) { lo[a] = fmin_(lo[a], s[k].lo[a]); hi[a] = fmax_(hi[a], s[k].hi[a]); }
-    float origin[3] = {0.0f, 0.0f, 0.0f};
-    int e[3] = {0, 0, 0};
-    if (n > 0)
-        for (int a = 0; a < 3; ++a) quant_frame(lo[a], hi[a], origin[a], e[a]);
-    w.ox = origin[0]; w.oy = origin[1]; w.oz = origin[2];
-    w.ex = (int8_t)e[0]; w.ey = (int8_t)e[1]; w.ez = (int8_t)e[2];
-    uint32_t ni = 0, nl = 0;
-    for (uint32_t k = 0; k < n; ++k) {
-        for (int a = 0; a < 3; ++a) {
-            float sc = ldexpf(1.0f, e[a]);
-            w.qlo[a][k] = quant_lo(s[k].lo[a], origin[a], sc);
-            w.qhi[a][k] = quant_hi(s[k].hi[a], origin[a], sc);
-        }
-        if (s[k].c & kLeaf) {
-            uint32_t slot = s[k].c & ~kLeaf;
-            uint32_t dst = w.tri_base + nl;
-            for (int q = 0; q < 9; ++q) tris8[(size_t)dst * 9 + q] = tris[(size_t)slot * 9 + q];
-            prims8[dst] = prims[slot];
-            w.meta[k] = (uint8_t)nl++;
+// Writes the wide nodes: child boxes (kept by the slots' binary parents)
+// quantised in the node's frame, and the leaves' triangles in wide order.
+__global__ __launch_bounds__(kBlock) void k_wide_emit(WideJobs jobs) {
+    const WideJob& J = wide_job_of(jobs, blockIdx.x);
+    const uint32_t w = (blockIdx.x - J.block) * kBlock + threadIdx.x;
+    if (w >= *J.count) return;
+    const uint32_t r = J.root[w];
+    uint32_t c[8];
+    slot_array(J.slots[2 * (size_t)r], J.slots[2 * (size_t)r + 1], c);
+    uint32_t at[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        at[k] = c[k] == kEmpty || J.n == 1   // (a lone triangle's leaf_parent is not written)
+                    ? r
+                    : ((c[k] & kLeaf) ? J.leaf_parent[c[k] & ~kLeaf] : J.bn[c[k]].parent);
+    float lo[8][3], hi[8][3];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const Node& p = J.bn[at[k]];
+        const bool second = p.child[0] != c[k];
+        lo[k][0] = second ? p.lox[1] : p.lox[0]; hi[k][0] = second ? p.hix[1] : p.hix[0];
+        lo[k][1] = second ? p.loy[1] : p.loy[0]; hi[k][1] = second ? p.hiy[1] : p.hiy[0];
+        lo[k][2] = second ? p.loz[1] : p.loz[0]; hi[k][2] = second ? p.hiz[1] : p.hiz[0];
+    }
+    const uint32_t tri_base = J.tri_base[w];
+    uint32_t word[24];
+    for (int k = 0; k < 24; ++k) word[k] = 0;
+    uint32_t n = 0, ni = 0, nl = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        if (c[k] == kEmpty) continue;
+        ++n;
+        uint32_t m;
+        if (c[k] & kLeaf) {
+            const uint32_t slot = c[k] & ~kLeaf, dst = tri_base + nl;
+            for (int q = 0; q < 9; ++q) J.tris8[(size_t)dst * 9 + q] = J.tris[(size_t)slot * 9 + q];
+            J.prims8[dst] = J.prims[slot];
+            m = nl++;
         } else {
-            next_level[int_off[i] + ni] = s[k].c;
-            w.meta[k] = (uint8_t)(0x80u | ni++);
+            m = 0x80u | ni++;
+        }
+        word[6 + k / 4] |= m << (8 * (k & 3));
+    }
+    word[4] = J.child_base[w];
+    word[5] = tri_base;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        float l = INFINITY, h = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (c[k] != kEmpty) { l = fmin_(l, lo[k][a]); h = fmax_(h, hi[k][a]); }
+        float origin = 0.0f;
+        int e = 0;
+        if (n > 0) quant_frame(l, h, origin, e);
+        word[a] = __float_as_uint(origin);
+        word[3] |= ((uint32_t)e & 0xFFu) << (8 * a);
+        const float sc = ldexpf(1.0f, (int)(int8_t)e), inv = ldexpf(1.0f, -(int)(int8_t)e);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (c[k] == kEmpty) continue;
+            word[8 + 2 * a + k / 4] |= quant_lo(lo[k][a], origin, sc, inv) << (8 * (k & 3));
+            word[14 + 2 * a + k / 4] |= quant_hi(hi[k][a], origin, sc, inv) << (8 * (k & 3));
         }
     }
-    out[level_start + i] = w;
+    word[3] |= n << 24;
+    uint4* out = reinterpret_cast<uint4*>(J.out + w);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) out[k] = make_uint4(word[4 * k], word[4 * k + 1], word[4 * k + 2], word[4 * k + 3]);
 }
 
 // ---------------------------------------------------------------- TLAS
@@ -1176,65 +1396,139 @@ luzrt_status blas_refit_device(luzrt_ctx* ctx, luzrt_blas* b, const void* vertic
     return LUZRT_OK;
 }
 
-luzrt_status blas_wide_device(luzrt_ctx* ctx, luzrt_blas* b) {
-    ctx->release_clean = false;   // BLAS data written on the context's stream
+namespace {
+
+// Bytes of a job's work arrays (slots, roots, child and triangle bases).
+size_t wide_work_bytes(uint32_t nodes) { return ((size_t)nodes * 44 + 255) & ~(size_t)255; }
+
+// Above this many binary nodes a BLAS is numbered with the whole chip.
+constexpr uint32_t kWideOneGroup = 1u << 17;
+// Work arrays up to this size are kept by the context for the next build (an
+// animated scene makes one per frame); larger ones are given back.
+constexpr size_t kWideKeptBytes = 32u << 20;
+
+luzrt_status wide_number_large(luzrt_ctx* ctx, const WideJob& J, uint8_t* level_mem) {
     hipStream_t st = ctx->stream;
-    const uint32_t n = b->tri_count;
-    const size_t cap = n > 1 ? n - 1 : 1;   // wide nodes <= binary internal nodes
-    if (!b->wide) {
-        LUZ_HIP(ctx, hipMalloc((void**)&b->wide, cap * sizeof(Node8)));
-        LUZ_HIP(ctx, hipMalloc((void**)&b->tris8, (size_t)(n ? n : 1) * 36));
-        LUZ_HIP(ctx, hipMalloc((void**)&b->prims8, (size_t)(n ? n : 1) * 4));
-    }
-    // scratch: two level lists, slots, counts and offsets
-    // 8 sub-allocations, each rounded up to 256 bytes
-    size_t bytes = cap * 4 * 2 + cap * 8 * sizeof(WRef) + cap * 4 * 5 + 8 * 256;
-    uint8_t* scratch = nullptr;
-    LUZ_HIP(ctx, hipMallocAsync((void**)&scratch, bytes, st));
-    uint8_t* p = scratch;
-    auto take = [&](size_t sz) { uint8_t* r = p; p += (sz + 255) & ~(size_t)255; return r; };
-    uint32_t* lvl[2] = {(uint32_t*)take(cap * 4), (uint32_t*)take(cap * 4)};
-    WRef* slots = (WRef*)take(cap * 8 * sizeof(WRef));
-    uint32_t* nslots = (uint32_t*)take(cap * 4);
-    uint32_t* n_int = (uint32_t*)take(cap * 4);
-    uint32_t* n_leaf = (uint32_t*)take(cap * 4);
-    uint32_t* int_off = (uint32_t*)take(cap * 4);
-    uint32_t* leaf_off = (uint32_t*)take(cap * 4);
-    (void)bytes;
-    LUZ_HIP(ctx, hipMemsetAsync(lvl[0], 0, 4, st));   // level 0 = binary root
-    uint32_t count = 1, level_start = 0, tri_start = 0;
-    int cur = 0;
-    while (count > 0) {
-        const uint32_t blocks = cdiv(count, kBlock);
-        k_wide_collapse<<<blocks, kBlock, 0, st>>>(b->nodes, lvl[cur], count, slots, nslots, n_int, n_leaf);
-        LUZ_HIP(ctx, hipMemcpyAsync(int_off, n_int, (size_t)count * 4, hipMemcpyDeviceToDevice, st));
-        LUZ_HIP(ctx, hipMemcpyAsync(leaf_off, n_leaf, (size_t)count * 4, hipMemcpyDeviceToDevice, st));
-        k_scan<<<1, 1024, 0, st>>>(int_off, count);
-        k_scan<<<1, 1024, 0, st>>>(leaf_off, count);
-        uint32_t tail[4];
-        LUZ_HIP(ctx, hipMemcpyAsync(&tail[0], int_off + count - 1, 4, hipMemcpyDeviceToHost, st));
-        LUZ_HIP(ctx, hipMemcpyAsync(&tail[1], n_int + count - 1, 4, hipMemcpyDeviceToHost, st));
-        LUZ_HIP(ctx, hipMemcpyAsync(&tail[2], leaf_off + count - 1, 4, hipMemcpyDeviceToHost, st));
-        LUZ_HIP(ctx, hipMemcpyAsync(&tail[3], n_leaf + count - 1, 4, hipMemcpyDeviceToHost, st));
-        LUZ_HIP(ctx, hipStreamSynchronize(st));
-        const uint32_t next_count = tail[0] + tail[1], leaves = tail[2] + tail[3];
-        const uint32_t next_start = level_start + count;
-        if ((size_t)next_start + next_count > cap || (size_t)tri_start + leaves > (n ? n : 1)) {
-            hipFreeAsync(scratch, st);
-            return fail(ctx, LUZRT_E_DEVICE, "8-wide collapse overflowed its arrays");
+    uint3* level = reinterpret_cast<uint3*>(level_mem);
+    uint2* sums = reinterpret_cast<uint2*>(level_mem + 1024);
+    k_wide_level_init<<<1, 64, 0, st>>>(J, level);
+    // a level has at most eight times the nodes of the one before; the host
+    // looks whether the tree has ended after the levels that most trees have
+    uint32_t done = 0;
+    for (uint32_t upto = 10; upto <= 64; upto += 6) {
+        for (; done < upto; ++done) {
+            k_wide_level_count<<<kWideLevelBlocks, kBlock, 0, st>>>(J, level + done, sums);
+            k_wide_level_write<<<kWideLevelBlocks, kBlock, 0, st>>>(J, level + done, sums);
         }
-        k_wide_emit<<<blocks, kBlock, 0, st>>>(slots, nslots, count, level_start, next_start, tri_start,
-                                               int_off, leaf_off, b->wide, lvl[cur ^ 1], b->tris,
-                                               b->prims, b->tris8, b->prims8);
+        uint3 last;
         LUZ_HIP(ctx, hipGetLastError());
-        level_start = next_start;
-        tri_start += leaves;
-        count = next_count;
-        cur ^= 1;
+        LUZ_HIP(ctx, hipMemcpyAsync(&last, level + done, sizeof(last), hipMemcpyDeviceToHost, st));
+        LUZ_HIP(ctx, hipStreamSynchronize(st));
+        if (last.y == 0) return LUZRT_OK;
     }
-    LUZ_HIP(ctx, hipFreeAsync(scratch, st));
-    b->wide_count = level_start;
-    b->wide_valid = true;
+    return fail(ctx, LUZRT_E_DEVICE, "8-wide collapse: deeper than 64 levels");
+}
+
+// Collapses up to kWideJobs BLASes on the context's stream.
+luzrt_status wide_build_some(luzrt_ctx* ctx, luzrt_blas* const* list, uint32_t count) {
+    hipStream_t st = ctx->stream;
+    constexpr size_t kLevelBytes = 1024 + kWideLevelBlocks * sizeof(uint2);
+    size_t bytes = kLevelBytes;
+    for (uint32_t k = 0; k < count; ++k) bytes += wide_work_bytes(list[k]->node_count);
+    uint8_t* work = nullptr;
+    const bool kept = bytes <= kWideKeptBytes;
+    if (kept) {
+        luzrt_status s = ensure(ctx, ctx->wide_work, bytes);
+        if (s != LUZRT_OK) return s;
+        work = (uint8_t*)ctx->wide_work.ptr;
+    } else {
+        LUZ_HIP(ctx, hipMallocAsync((void**)&work, bytes, st));
+    }
+    uint8_t* p = work + kLevelBytes;
+    WideJobs jobs{};
+    jobs.n = count;
+    uint32_t blocks = 0, small = 0;
+    for (uint32_t k = 0; k < count; ++k) {
+        luzrt_blas* b = list[k];
+        WideJob& J = jobs.j[k];
+        J.bn = b->nodes;
+        J.leaf_parent = b->leaf_parent;
+        J.tris = b->tris;
+        J.prims = b->prims;
+        J.n = b->node_count;
+        J.slots = (uint4*)p;
+        J.root = (uint32_t*)(p + (size_t)J.n * 32);
+        J.child_base = J.root + J.n;
+        J.tri_base = J.child_base + J.n;
+        p += wide_work_bytes(J.n);
+        J.out = b->wide;
+        J.tris8 = b->tris8;
+        J.prims8 = b->prims8;
+        J.count = b->wide_count_dev;
+        J.block = blocks;
+        blocks += cdiv(J.n, kBlock);
+        if (J.n <= kWideOneGroup) ++small;
+    }
+    k_wide_slots<<<blocks, kBlock, 0, st>>>(jobs);
+    luzrt_status s = LUZRT_OK;
+    if (small == count) {
+        k_wide_number<<<count, 1024, 0, st>>>(jobs);
+    } else {
+        WideJobs few{};
+        for (uint32_t k = 0; k < count; ++k)
+            if (jobs.j[k].n <= kWideOneGroup) few.j[few.n++] = jobs.j[k];
+        if (few.n) k_wide_number<<<few.n, 1024, 0, st>>>(few);
+        for (uint32_t k = 0; k < count && s == LUZRT_OK; ++k)
+            if (jobs.j[k].n > kWideOneGroup) s = wide_number_large(ctx, jobs.j[k], work);
+    }
+    if (s == LUZRT_OK) {
+        k_wide_emit<<<blocks, kBlock, 0, st>>>(jobs);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) s = hip_fail(ctx, e, "8-wide collapse");
+    }
+    if (!kept) {
+        hipError_t e = hipFreeAsync(work, st);
+        if (e != hipSuccess && s == LUZRT_OK) s = hip_fail(ctx, e, "hipFreeAsync");
+    }
+    if (s != LUZRT_OK) return s;
+    for (uint32_t k = 0; k < count; ++k) {
+        list[k]->wide_valid = true;
+        list[k]->wide_counted = false;
+    }
+    return LUZRT_OK;
+}
+
+}  // namespace
+
+luzrt_status blas_wide_device(luzrt_ctx* ctx, luzrt_blas* const* list, uint32_t count) {
+    ctx->release_clean = false;   // BLAS data written on the context's stream
+    for (uint32_t k = 0; k < count; ++k) {
+        luzrt_blas* b = list[k];
+        const size_t n = b->tri_count ? b->tri_count : 1;
+        auto alloc = [](auto** p, size_t bytes) { return *p ? hipSuccess : hipMalloc((void**)p, bytes); };
+        LUZ_HIP(ctx, alloc(&b->wide, (size_t)b->node_count * sizeof(Node8)));   // wide nodes <= binary internal nodes
+        LUZ_HIP(ctx, alloc(&b->tris8, n * 36));
+        LUZ_HIP(ctx, alloc(&b->prims8, n * 4));
+        LUZ_HIP(ctx, alloc(&b->wide_count_dev, 4));
+    }
+    for (uint32_t k = 0; k < count; k += kWideJobs) {
+        luzrt_status s = wide_build_some(ctx, list + k, count - k < kWideJobs ? count - k : kWideJobs);
+        if (s != LUZRT_OK) return s;
+    }
+    return LUZRT_OK;
+}
+
+luzrt_status blas_wide_count(luzrt_ctx* ctx, luzrt_blas* b, uint32_t* count) {
+    if (!b->wide_counted) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        LUZ_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cs));
+        if (cs != hipStreamCaptureStatusNone)
+            return fail(ctx, LUZRT_E_UNSUPPORTED, "the 8-wide node count cannot be read while the stream is captured");
+        LUZ_HIP(ctx, hipMemcpyAsync(&b->wide_count, b->wide_count_dev, 4, hipMemcpyDeviceToHost, ctx->stream));
+        LUZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        b->wide_counted = true;
+    }
+    *count = b->wide_count;
     return LUZRT_OK;
 }
 

@@ -47,6 +47,7 @@ struct luzrt_ctx {
     // ray-group culling of visibility calls: candidate masks, live-row masks
     // and counts, the live-row list
     luz::DevBuf cull_cand, cull_bits, cull_rows;
+    luz::DevBuf wide_work;         // work arrays of 8-wide collapses (bvh.hip)
     bool group_cull = true;        // luzrt_set_group_culling
     bool last_culled = false;      // the last visibility call traced live rows only
     // timing
@@ -97,7 +98,9 @@ struct luzrt_blas {
     int refs = 0;                   // live TLASes built over this BLAS
     // precision form: 8-wide quantised nodes, built on demand from the binary tree
     luz::Node8* wide = nullptr;
-    uint32_t wide_count = 0;
+    uint32_t* wide_count_dev = nullptr;   // wide nodes, as the last collapse counted them
+    uint32_t wide_count = 0;         // the host's copy (blas_wide_count)
+    bool wide_counted = false;
     float* tris8 = nullptr;          // 9 floats per wide leaf
     uint32_t* prims8 = nullptr;
     bool wide_valid = false;
@@ -158,7 +161,10 @@ struct alignas(16) InstIn {
 luzrt_status blas_build_device(luzrt_ctx* ctx, luzrt_blas* b, const void* vertices,
                                const uint32_t* indices);
 luzrt_status blas_refit_device(luzrt_ctx* ctx, luzrt_blas* b, const void* vertices);
-luzrt_status blas_wide_device(luzrt_ctx* ctx, luzrt_blas* b);
+// The 8-wide forms of `count` BLASes, on the context's stream.
+luzrt_status blas_wide_device(luzrt_ctx* ctx, luzrt_blas* const* list, uint32_t count);
+// Wide nodes of a BLAS with a valid 8-wide form (waits for it once per collapse).
+luzrt_status blas_wide_count(luzrt_ctx* ctx, luzrt_blas* b, uint32_t* count);
 luzrt_status tlas_build_device(luzrt_ctx* ctx, luzrt_tlas* t, const InstIn* dev_in, uint32_t n,
                                hipStream_t st);
 // Before the first kernel of a call that reads `tlas` on the context's stream:
@@ -355,7 +361,7 @@ luzrt_status stage_upload(luzrt_ctx* ctx, void* dst, const void* src, size_t byt
 luzrt_status upload_scene(luzrt_ctx* ctx, const luzrt_scene* scene, DevScene* host_copy,
                           uint32_t ray_group = 0, bool trace = false);
 // Ray group of a visibility call on `tlas` under the context's ray order.
-uint32_t ray_group_for(const luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt_scene* scene = nullptr);
+uint32_t ray_group_for(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt_scene* scene = nullptr);
 // Validates a G-buffer descriptor and writes it with its layout filled in
 // (zero strides and pitches replaced by the packed defaults; the depth
 // pointer cleared when a position plane is given): the form kernels take.

@@ -309,7 +309,7 @@ static bool invert_3x4(const float m[12], float out[12], float nmat[9]) {
 // 4.2 M triangles, 36 lights + 8 AO rays: 32.8 ms grouped, 29.3 ms by slot.
 constexpr size_t kGroupedBvhBytes = 32u << 20;   // the L2 of all XCDs together
 
-uint32_t ray_group_for(const luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt_scene* scene) {
+uint32_t ray_group_for(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt_scene* scene) {
     if (ctx->ray_order == LUZRT_RAY_ORDER_SLOT) return 0;
     if (ctx->ray_order == LUZRT_RAY_ORDER_GROUPED) return kRayGroup;
     // a call that can cull its ray groups (which needs the grouped order)
@@ -327,9 +327,14 @@ uint32_t ray_group_for(const luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
     std::sort(seen.begin(), seen.end());
     seen.erase(std::unique(seen.begin(), seen.end()), seen.end());
     size_t bytes = 0;
-    for (const luzrt_blas* b : seen)
-        bytes += tlas->wide ? (size_t)b->wide_count * sizeof(Node8) + (size_t)b->tri_count * 36
-                            : (size_t)b->node_count * sizeof(Node) + (size_t)b->tri_count * 36;
+    for (const luzrt_blas* b : seen) {
+        // a captured call cannot wait for a new collapse's count: the last
+        // count, or the bound, then serves
+        uint32_t wide = b->wide_count ? b->wide_count : b->node_count;
+        if (tlas->wide && b->wide_valid) (void)blas_wide_count(ctx, const_cast<luzrt_blas*>(b), &wide);
+        bytes += (tlas->wide ? (size_t)wide * sizeof(Node8) : (size_t)b->node_count * sizeof(Node)) +
+                 (size_t)b->tri_count * 36;
+    }
     return bytes <= kGroupedBvhBytes ? kRayGroup : 0;
 }
 
@@ -399,7 +404,7 @@ luzrt_status luzrt_destroy(luzrt_ctx* ctx) {
     if (ctx->build_stream) hipStreamSynchronize(ctx->build_stream);
     DevBuf* bufs[] = {&ctx->hits, &ctx->active, &ctx->act_index, &ctx->act_rec,
                       &ctx->counters, &ctx->spill, &ctx->lut, &ctx->scene, &ctx->vis_shadow,
-                      &ctx->vis_ao, &ctx->cull_cand, &ctx->cull_bits, &ctx->cull_rows};
+                      &ctx->vis_ao, &ctx->cull_cand, &ctx->cull_bits, &ctx->cull_rows, &ctx->wide_work};
     for (DevBuf* b : bufs)
         if (b->ptr) hipFree(b->ptr);
     for (int s = 0; s < kStageCount; ++s)
@@ -536,11 +541,16 @@ luzrt_status luzrt_blas_wide_arrays(luzrt_ctx* ctx, luzrt_blas* b, const void** 
     if (!ctx) return LUZRT_E_INVALID_ARG;
     if (!b) return fail(ctx, LUZRT_E_INVALID_ARG, "luzrt_blas_wide_arrays: null BLAS");
     if (b->tri_count > 0 && !b->wide_valid) {
-        luzrt_status s = blas_wide_device(ctx, b);
+        luzrt_status s = blas_wide_device(ctx, &b, 1);
+        if (s != LUZRT_OK) return s;
+    }
+    uint32_t count = 0;
+    if (b->tri_count > 0) {
+        luzrt_status s = blas_wide_count(ctx, b, &count);
         if (s != LUZRT_OK) return s;
     }
     if (nodes) *nodes = b->wide;
-    if (node_count) *node_count = b->tri_count > 0 ? b->wide_count : 0;
+    if (node_count) *node_count = count;
     if (tris) *tris = b->tris8;
     if (prims) *prims = b->prims8;
     if (tri_count) *tri_count = b->tri_count;
@@ -655,7 +665,7 @@ luzrt_status luzrt_blas_destroy(luzrt_ctx* ctx, luzrt_blas* b) {
         return fail(ctx, LUZRT_E_IN_USE, "BLAS is referenced by %d TLAS(es)", b->refs);
     hipStreamSynchronize(ctx->stream);
     void* ptrs[] = {b->nodes, b->tris, b->nrms, b->prims, b->slot_idx, b->leaf_parent, b->counters,
-                    b->node_end, b->span, b->wide, b->tris8, b->prims8};
+                    b->node_end, b->span, b->wide, b->tris8, b->prims8, b->wide_count_dev};
     for (void* p : ptrs)
         if (p) hipFree(p);
     delete b;
@@ -712,6 +722,19 @@ luzrt_status pack_instances(luzrt_ctx* ctx, luzrt_tlas* t, const luzrt_instance*
                     t->capacity);
     host.clear();
     host.reserve(count);
+    // the 8-wide forms that are missing or out of date, all together
+    if (ctx->precision != LUZRT_PRECISION_PLAIN) {
+        std::vector<luzrt_blas*> todo;
+        for (uint32_t i = 0; i < count; ++i) {
+            luzrt_blas* b = const_cast<luzrt_blas*>(inst[i].blas);
+            if (b && b->tri_count > 0 && !b->wide_valid && std::find(todo.begin(), todo.end(), b) == todo.end())
+                todo.push_back(b);
+        }
+        if (!todo.empty()) {
+            luzrt_status ws = blas_wide_device(ctx, todo.data(), (uint32_t)todo.size());
+            if (ws != LUZRT_OK) return ws;
+        }
+    }
     std::vector<const luzrt_blas*> refs;
     for (uint32_t i = 0; i < count; ++i) {
         const luzrt_instance& in = inst[i];
@@ -732,13 +755,8 @@ luzrt_status pack_instances(luzrt_ctx* ctx, luzrt_tlas* t, const luzrt_instance*
         r.nrms = in.blas->nrms;
         r.prims = in.blas->prims;
         if (ctx->precision != LUZRT_PRECISION_PLAIN && in.blas->tri_count > 0) {
-            luzrt_blas* b = const_cast<luzrt_blas*>(in.blas);
-            if (!b->wide_valid) {
-                luzrt_status ws = blas_wide_device(ctx, b);
-                if (ws != LUZRT_OK) return ws;
-            }
-            r.wnodes = b->wide;
-            r.wtris = b->tris8;
+            r.wnodes = in.blas->wide;
+            r.wtris = in.blas->tris8;
         }
         refs.push_back(in.blas);
         // empty meshes and mask-0 instances can never be hit by a 0xFF ray mask

@@ -34,6 +34,32 @@ def test_wide_bytes_match_oracle(compact, kind):
     g.close()
 
 
+@pytest.mark.parametrize("tris", [1, 2, 3, 9, 64, 1025, 131072, 131074, 200003])
+def test_wide_bytes_of_any_size_match_oracle(compact, tris):
+    """The 8-wide form of meshes of one to a few triangles, a few levels, and on both
+    sides of the size from which the numbering uses the whole chip (131,072 binary nodes)."""
+    from oracle import oracle as orc
+    rng = np.random.default_rng(tris)
+    c = rng.normal(size=(tris, 1, 3)) * (40, 3, 40)
+    pos = (c + rng.normal(size=(tris, 3, 3)) * 0.3).astype(np.float32).reshape(-1, 3)
+    verts = np.zeros((3 * tris, 12), np.float32)
+    verts[:, :3] = pos
+    idx = np.arange(3 * tris, dtype=np.uint32)
+    blas = compact.create_blas(compact.to_device(verts), 48, len(verts), compact.to_device(idx), len(idx))
+    o = orc.OracleScene()
+    m = o.add_mesh(verts, idx)
+    o.set_instances(np.eye(3, 4, dtype=np.float32).reshape(1, 12), [m])
+    o.build_wide()
+    on, ot, op = o.blas_wide_arrays(m)
+    for _ in range(2):      # a refit's second collapse reuses the arrays of the first
+        gn, gt, gp = blas.wide_arrays()
+        np.testing.assert_array_equal(gp, op)
+        np.testing.assert_array_equal(gt.view(np.uint32), ot.view(np.uint32))
+        np.testing.assert_array_equal(gn, on)
+        blas.refit(compact.to_device(verts))
+    blas.destroy()
+
+
 def test_wide_trace_rays_match_oracle(compact):
     s = api.HostScene(api.SCENE_SPHERES, 0)
     g = api.GPUScene(compact, s)
