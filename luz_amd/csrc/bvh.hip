@@ -16,6 +16,7 @@
 // FP64 frame, Morton codes, bitonic sort of (code, index) in LDS, Karras,
 // refit.  Both produce byte-identical nodes to a sequential CPU build.
 #include "internal.hpp"
+#include "scan.hpp"
 
 namespace luz {
 namespace {
@@ -173,31 +174,10 @@ __global__ __launch_bounds__(kBlock) void k_sort_hist(const uint32_t* keys, uint
     hist[threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
 }
 
-// Exclusive scan of count entries with one workgroup of 1024 threads.
-__global__ __launch_bounds__(1024) void k_scan(uint32_t* data, uint32_t count) {
-    __shared__ uint32_t sh[1024];
-    __shared__ uint32_t carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (uint32_t base = 0; base < count; base += 1024) {
-        uint32_t i = base + threadIdx.x;
-        uint32_t v = i < count ? data[i] : 0u;
-        sh[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            uint32_t add = threadIdx.x >= (uint32_t)off ? sh[threadIdx.x - off] : 0u;
-            __syncthreads();
-            sh[threadIdx.x] += add;
-            __syncthreads();
-        }
-        uint32_t incl = sh[threadIdx.x];
-        uint32_t c = carry;
-        if (i < count) data[i] = c + incl - v;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry = c + incl;
-        __syncthreads();
-    }
-}
+// Exclusive scan of the digit counts (16-byte aligned).  A run of consecutive
+// counts per thread, read as 16-byte vectors: 200k keys (12,800 counts) 5.7 us
+// a pass against 24 us with 1024 counts at a time and twenty barriers each.
+__global__ __launch_bounds__(1024) void k_sort_scan(uint32_t* data, uint32_t count) { scan_runs_1024(data, count); }
 
 __global__ __launch_bounds__(kBlock) void k_sort_scatter(const uint32_t* keys_in,
                                                          const uint32_t* vals_in, uint32_t n,
@@ -333,8 +313,8 @@ __device__ inline void store_child_box(Node* nd, int side, const float* b) {
 }
 
 
-constexpr int kRefitChunk = 256;    // leaf slots per workgroup of the chunk pass
-constexpr int kSpanThreads = 512;   // threads per BLAS of the span pass
+constexpr int kRefitChunk = 1024;   // leaf slots per workgroup of the chunk pass
+constexpr int kSpanThreads = 1024;  // threads per BLAS of the span pass
 
 // Union of a node's two child boxes, child 0 first (the operand order of
 // fmin_/fmax_ matters for signed zeros).
@@ -355,72 +335,95 @@ __device__ inline uint32_t chunk_job_of(const RefitJob* jobs, uint32_t njobs, ui
     return lo;
 }
 
-// Chunk pass of a refit (or of a build): one workgroup per 256 consecutive
-// leaf slots of a BLAS.  Every internal node covers a contiguous range of
-// slots (Karras), so a node whose range lies inside the chunk has both
-// children completed by this workgroup: the second child to arrive forms the
-// node's box, with arrival counters and child boxes in LDS.  A node whose
-// parent's range leaves the chunk stores its box in the parent and hands the
-// parent to the span pass through the BLAS's span list.  Also zeroes the span
-// pass's arrival counters of the chunk's node ids.  jobs == nullptr: `single`.
+// Chunk pass of a refit (or of a build): one workgroup per kRefitChunk
+// consecutive leaf slots of a BLAS.  Every internal node covers a contiguous
+// range of slots that starts or ends at the slot of its own number (Karras), so
+// a node whose range lies inside the chunk has both children completed by this
+// workgroup: the second child to arrive forms the node's box and writes its two
+// child boxes.  A node whose parent's range leaves the chunk stores its box in
+// the parent and hands the parent to the span pass through the BLAS's span
+// list.  Also zeroes the span pass's arrival counters of the chunk's node ids.
+// jobs == nullptr: `single`.
+//
+// Bound by the length of the climb.  The chunk's part of the hierarchy, the
+// arrival counters and the child boxes are in LDS, so a step up waits for no
+// global load or store; 1024 slots leave the span pass, which climbs in global
+// memory, few nodes.  20,480 triangles: chunk pass 18 -> 22 us, span pass 39 ->
+// 23 us against 256-slot chunks with the hierarchy read at every step; 200,978
+// triangles 96 -> 38 and 251 -> 66 us (512 slots: 16, 26, 56, 109).
+constexpr uint32_t kOutside = 0x80000000u;   // the node's range leaves the chunk
 template <bool FROM_VERTS>
 __global__ __launch_bounds__(kRefitChunk) void k_refit_chunks(const RefitJob* jobs, uint32_t njobs,
                                                               RefitJob single, uint32_t* error) {
     __shared__ uint32_t scnt[kRefitChunk];
+    __shared__ uint2 stopo[kRefitChunk];   // child 0; parent (31 bits, all set at the root) and kOutside
     __shared__ float sbox[kRefitChunk * 12];
     const RefitJob& J = jobs ? jobs[chunk_job_of(jobs, njobs, blockIdx.x)] : single;
     const uint32_t c0 = (blockIdx.x - J.chunk_offset) * kRefitChunk;
     const uint32_t c1 = (c0 + kRefitChunk < J.n ? c0 + kRefitChunk : J.n) - 1;   // last slot
     const uint32_t s = c0 + threadIdx.x;
     scnt[threadIdx.x] = 0;
-    if (s < J.n - 1) J.counters[s] = 0;
+    if (s < J.n - 1) {
+        J.counters[s] = 0;
+        const uint32_t e = J.node_end[s], up = J.nodes[s].parent;
+        const uint32_t lo = s < e ? s : e, hi = s < e ? e : s;
+        stopo[threadIdx.x] = make_uint2(J.nodes[s].child[0], (up & ~kOutside) | (lo < c0 || hi > c1 ? kOutside : 0u));
+    }
+    float box[6];
+    uint32_t p = 0;
+    if (s < J.n) {
+        p = J.leaf_parent[s];
+        if (FROM_VERTS) {
+            // slot_idx was validated by the build
+            V3 v[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) v[k] = load_pos(J.verts, J.stride, J.slot_idx[3 * s + k]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                J.tris[(size_t)s * 9 + k * 3 + 0] = v[k].x;
+                J.tris[(size_t)s * 9 + k * 3 + 1] = v[k].y;
+                J.tris[(size_t)s * 9 + k * 3 + 2] = v[k].z;
+            }
+            tri_box(v[0], v[1], v[2], box);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) box[k] = J.leaf_box[(size_t)s * 6 + k];
+        }
+    }
     __syncthreads();
     if (s >= J.n) return;
-    float box[6];
-    if (FROM_VERTS) {
-        // slot_idx was validated by the build
-        V3 v[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            v[k] = load_pos(J.verts, J.stride, J.slot_idx[3 * s + k]);
-            J.tris[(size_t)s * 9 + k * 3 + 0] = v[k].x;
-            J.tris[(size_t)s * 9 + k * 3 + 1] = v[k].y;
-            J.tris[(size_t)s * 9 + k * 3 + 2] = v[k].z;
-        }
-        tri_box(v[0], v[1], v[2], box);
-    } else {
-#pragma unroll
-        for (int k = 0; k < 6; ++k) box[k] = J.leaf_box[(size_t)s * 6 + k];
-    }
     uint32_t c = kLeaf | s;
-    uint32_t p = J.leaf_parent[s];
     for (int level = 0; p != kNone; ++level) {
         if (level > 80) { atomicOr(error, 1u); return; }
         Node* nd = &J.nodes[p];
-        const int side = nd->child[0] == c ? 0 : 1;
-        store_child_box(nd, side, box);
-        const uint32_t e = J.node_end[p];
-        const uint32_t lo = p < e ? p : e, hi = p < e ? e : p;
-        if (lo < c0 || hi > c1) {
+        const bool mine = p >= c0 && p <= c1;
+        const uint2 t = mine ? stopo[p - c0] : make_uint2(0u, kOutside);
+        if (t.y & kOutside) {
+            store_child_box(nd, (mine ? t.x : nd->child[0]) == c ? 0 : 1, box);
             const uint32_t k = atomicAdd(&J.span[0], 1u);
             J.span[1 + k] = p;
             return;
         }
+        const int side = t.x == c ? 0 : 1;
         float* sb = &sbox[(p - c0) * 12];
 #pragma unroll
         for (int k = 0; k < 6; ++k) sb[side * 6 + k] = box[k];
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         if (atomicAdd(&scnt[p - c0], 1u) == 0) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        float other[6];
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        float b[2][6];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) other[k] = sb[(1 - side) * 6 + k];
-        float u[6];
-        child_union(side, box, other, u);
+        for (int k = 0; k < 6; ++k) {
+            const float other = sb[(1 - side) * 6 + k];
+            b[0][k] = side == 0 ? box[k] : other;
+            b[1][k] = side == 0 ? other : box[k];
+        }
+        float4* q = reinterpret_cast<float4*>(nd);
 #pragma unroll
-        for (int k = 0; k < 6; ++k) box[k] = u[k];
+        for (int a = 0; a < 3; ++a) q[a] = make_float4(b[0][a], b[1][a], b[0][3 + a], b[1][3 + a]);
+        child_union(0, b[0], b[1], box);
         c = p;
-        p = nd->parent;
+        p = t.y == ~kOutside ? kNone : t.y;
     }
 }
 
@@ -500,7 +503,7 @@ __global__ void k_small_root(const uint8_t* verts, uint32_t stride, uint32_t nv,
 // then writes all wide nodes together.  One launch of each serves up to
 // kWideJobs BLASes and the host waits for none of it.  (With the slots found
 // level by level, seven launches and copies and a wait for the host per level,
-// five 20,480-triangle meshes took 3.3 ms, now WIDE_T us.)
+// five 20,480-triangle meshes took 3.3 ms, now 93 us.)
 struct WideJob {
     const Node* bn;
     const uint32_t* leaf_parent;
@@ -515,7 +518,7 @@ struct WideJob {
     uint32_t* prims8;
     uint32_t* count;       // wide nodes
     uint32_t n;            // binary nodes
-    uint32_t block;        // first workgroup of this job in a launch over all jobs' nodes
+    uint32_t block, blocks;   // this job's workgroups in a launch over all jobs' nodes
 };
 constexpr uint32_t kWideJobs = 8;
 struct WideJobs {
@@ -634,13 +637,14 @@ __device__ inline void wide_place(const WideJob& J, uint32_t w, const uint32_t (
 }
 
 // Breadth-first numbering of one BLAS by one workgroup: per level, running
-// sums of the nodes' child and triangle counts.  About 2 us per 1024 wide nodes.
-__global__ __launch_bounds__(1024) void k_wide_number(WideJobs jobs) {
+// sums of the nodes' child and triangle counts.  About 2.6 us per 1024 wide
+// nodes.  Stops before a level of more than `stop` nodes, left in *level.
+__global__ __launch_bounds__(1024) void k_wide_number(WideJobs jobs, uint32_t stop, uint3* level) {
     __shared__ uint32_t sums[1024 / 64];
     const WideJob& J = jobs.j[blockIdx.x];
     if (threadIdx.x == 0) J.root[0] = 0;
     uint32_t start = 0, count = 1, tri = 0;
-    while (count > 0) {
+    while (count > 0 && count <= stop) {
         __syncthreads();   // the level's roots are written
         const uint32_t next = start + count;
         uint32_t children = 0, leaves = 0;
@@ -661,10 +665,13 @@ __global__ __launch_bounds__(1024) void k_wide_number(WideJobs jobs) {
         start = next;
         count = children;
     }
-    if (threadIdx.x == 0) *J.count = start;
+    if (threadIdx.x == 0) {
+        *J.count = start;
+        if (level) *level = make_uint3(start, count, tri);
+    }
 }
 
-// The same for one large BLAS, a level per pair of launches: workgroup b takes
+// The wide levels of a large BLAS, one per pair of launches: workgroup b takes
 // the b-th run of the level's nodes, k_wide_level_count sums the runs and
 // k_wide_level_write numbers them.  levels[l] = (first wide node, nodes, first
 // triangle) of level l.
@@ -742,14 +749,6 @@ __global__ __launch_bounds__(kBlock) void k_wide_level_write(WideJob J, uint3* l
     }
 }
 
-// The first level of a large BLAS: its root.
-__global__ void k_wide_level_init(WideJob J, uint3* level) {
-    if (threadIdx.x == 0) {
-        J.root[0] = 0;
-        level[0] = make_uint3(0u, 1u, 0u);
-    }
-}
-
 __device__ inline void quant_frame(float lo, float hi, float& origin, int& e) {
     float t = (hi - lo) / 255.0f;
     int e0 = -126, em = -126;
@@ -762,7 +761,7 @@ __device__ inline void quant_frame(float lo, float hi, float& origin, int& e) {
         float sc = ldexpf(1.0f, e);
         origin = floorf(lo / sc) * sc;
         if (origin > lo) origin = origin - sc;
-        if (origin + 255.0f * sc >= hi) break;
+        if (origin + 255.0f * sc >= hi || e >= 127) break;   // (127: a box that is not finite)
         ++e;
     }
 }
@@ -782,74 +781,76 @@ __device__ inline uint32_t quant_hi(float v, float origin, float sc, float inv) 
     return (uint32_t)(uint8_t)q;
 }
 
+// The earlier of a and b unless b is less or equal: the minimum as a left-to-right
+// fold of fmin_ takes it (the last of equal zeros), and likewise the maximum.
+template <bool MAX>
+__device__ inline float fold8(float v, uint32_t k) {
+#pragma unroll
+    for (uint32_t off = 1; off < 8; off <<= 1) {
+        const float o = __shfl_xor(v, (int)off);
+        const float a = (k & off) ? o : v, b = (k & off) ? v : o;
+        v = MAX ? fmax_(a, b) : fmin_(a, b);
+    }
+    return v;
+}
+
 // Writes the wide nodes: child boxes (kept by the slots' binary parents)
 // quantised in the node's frame, and the leaves' triangles in wide order.
+// Eight threads per node, one per slot: the quantisation is most of the work
+// (five 20,480-triangle meshes 22 us, 49 with one thread per node).
 __global__ __launch_bounds__(kBlock) void k_wide_emit(WideJobs jobs) {
     const WideJob& J = wide_job_of(jobs, blockIdx.x);
-    const uint32_t w = (blockIdx.x - J.block) * kBlock + threadIdx.x;
-    if (w >= *J.count) return;
-    const uint32_t r = J.root[w];
-    uint32_t c[8];
-    slot_array(J.slots[2 * (size_t)r], J.slots[2 * (size_t)r + 1], c);
-    uint32_t at[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-        at[k] = c[k] == kEmpty || J.n == 1   // (a lone triangle's leaf_parent is not written)
-                    ? r
-                    : ((c[k] & kLeaf) ? J.leaf_parent[c[k] & ~kLeaf] : J.bn[c[k]].parent);
-    float lo[8][3], hi[8][3];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const Node& p = J.bn[at[k]];
-        const bool second = p.child[0] != c[k];
-        lo[k][0] = second ? p.lox[1] : p.lox[0]; hi[k][0] = second ? p.hix[1] : p.hix[0];
-        lo[k][1] = second ? p.loy[1] : p.loy[0]; hi[k][1] = second ? p.hiy[1] : p.hiy[0];
-        lo[k][2] = second ? p.loz[1] : p.loz[0]; hi[k][2] = second ? p.hiz[1] : p.hiz[0];
-    }
-    const uint32_t tri_base = J.tri_base[w];
-    uint32_t word[24];
-    for (int k = 0; k < 24; ++k) word[k] = 0;
-    uint32_t n = 0, ni = 0, nl = 0;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        if (c[k] == kEmpty) continue;
-        ++n;
-        uint32_t m;
-        if (c[k] & kLeaf) {
-            const uint32_t slot = c[k] & ~kLeaf, dst = tri_base + nl;
+    const uint32_t t = (blockIdx.x - J.block) * kBlock + threadIdx.x, k = t & 7u;
+    const uint32_t count = *J.count;
+    for (uint32_t w = t >> 3; w < count; w += J.blocks * (kBlock / 8)) {
+        const uint32_t r = J.root[w];
+        const uint32_t c = reinterpret_cast<const uint32_t*>(J.slots)[(size_t)r * 8 + k];
+        const bool used = c != kEmpty, leaf = used && (c & kLeaf);
+        const uint32_t at = !used || J.n == 1   // (a lone triangle's leaf_parent is not written)
+                                ? r
+                                : (leaf ? J.leaf_parent[c & ~kLeaf] : J.bn[c].parent);
+        const Node& p = J.bn[at];
+        const bool second = p.child[0] != c;
+        const float lo[3] = {second ? p.lox[1] : p.lox[0], second ? p.loy[1] : p.loy[0], second ? p.loz[1] : p.loz[0]};
+        const float hi[3] = {second ? p.hix[1] : p.hix[0], second ? p.hiy[1] : p.hiy[0], second ? p.hiz[1] : p.hiz[0]};
+        // this node's lanes, and this slot's rank among the slots of its sort
+        const uint32_t group = (threadIdx.x & 63u) & ~7u, below = (1u << k) - 1u;
+        const uint32_t leaves = (uint32_t)(__ballot(leaf) >> group) & 0xFFu;
+        const uint32_t inner = (uint32_t)(__ballot(used && !leaf) >> group) & 0xFFu;
+        const uint32_t tri_base = J.tri_base[w];
+        uint8_t* out = reinterpret_cast<uint8_t*>(J.out + w);
+        uint32_t meta = 0;
+        if (leaf) {
+            meta = (uint32_t)__popc(leaves & below);
+            const uint32_t slot = c & ~kLeaf, dst = tri_base + meta;
             for (int q = 0; q < 9; ++q) J.tris8[(size_t)dst * 9 + q] = J.tris[(size_t)slot * 9 + q];
             J.prims8[dst] = J.prims[slot];
-            m = nl++;
-        } else {
-            m = 0x80u | ni++;
+        } else if (used) {
+            meta = 0x80u | (uint32_t)__popc(inner & below);
         }
-        word[6 + k / 4] |= m << (8 * (k & 3));
-    }
-    word[4] = J.child_base[w];
-    word[5] = tri_base;
+        out[24 + k] = (uint8_t)meta;
+        const uint32_t n = (uint32_t)__popc(leaves | inner);
+        float origin[3];
+        uint32_t es = n << 24;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        float l = INFINITY, h = -INFINITY;
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (c[k] != kEmpty) { l = fmin_(l, lo[k][a]); h = fmax_(h, hi[k][a]); }
-        float origin = 0.0f;
-        int e = 0;
-        if (n > 0) quant_frame(l, h, origin, e);
-        word[a] = __float_as_uint(origin);
-        word[3] |= ((uint32_t)e & 0xFFu) << (8 * a);
-        const float sc = ldexpf(1.0f, (int)(int8_t)e), inv = ldexpf(1.0f, -(int)(int8_t)e);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (c[k] == kEmpty) continue;
-            word[8 + 2 * a + k / 4] |= quant_lo(lo[k][a], origin, sc, inv) << (8 * (k & 3));
-            word[14 + 2 * a + k / 4] |= quant_hi(hi[k][a], origin, sc, inv) << (8 * (k & 3));
+        for (int a = 0; a < 3; ++a) {
+            const float l = fold8<false>(used ? lo[a] : INFINITY, k), h = fold8<true>(used ? hi[a] : -INFINITY, k);
+            int e = 0;
+            origin[a] = 0.0f;
+            if (n > 0) quant_frame(l, h, origin[a], e);
+            es |= ((uint32_t)e & 0xFFu) << (8 * a);
+            const float sc = ldexpf(1.0f, (int)(int8_t)e), inv = ldexpf(1.0f, -(int)(int8_t)e);
+            out[32 + 8 * a + k] = (uint8_t)(used ? quant_lo(lo[a], origin[a], sc, inv) : 0u);
+            out[56 + 8 * a + k] = (uint8_t)(used ? quant_hi(hi[a], origin[a], sc, inv) : 0u);
+        }
+        if (k == 0) {
+            reinterpret_cast<uint4*>(out)[0] = make_uint4(__float_as_uint(origin[0]), __float_as_uint(origin[1]),
+                                                          __float_as_uint(origin[2]), es);
+            reinterpret_cast<uint2*>(out)[2] = make_uint2(J.child_base[w], tri_base);
+        } else if (k == 1) {
+            reinterpret_cast<uint4*>(out)[5] = make_uint4(0u, 0u, 0u, 0u);
         }
     }
-    word[3] |= n << 24;
-    uint4* out = reinterpret_cast<uint4*>(J.out + w);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) out[k] = make_uint4(word[4 * k], word[4 * k + 1], word[4 * k + 2], word[4 * k + 3]);
 }
 
 // ---------------------------------------------------------------- TLAS
@@ -1358,7 +1359,7 @@ luzrt_status blas_build_device(luzrt_ctx* ctx, luzrt_blas* b, const void* vertic
     for (int pass = 0; pass < 4; ++pass) {
         int shift = pass * 8;
         k_sort_hist<<<sb, kBlock, 0, st>>>(kin, n, shift, hist, sb);
-        k_scan<<<1, 1024, 0, st>>>(hist, 256 * sb);
+        k_sort_scan<<<1, 1024, 0, st>>>(hist, 256 * sb);
         k_sort_scatter<<<sb, kBlock, 0, st>>>(kin, vin, n, shift, hist, sb, kout, vout);
         std::swap(kin, kout);
         std::swap(vin, vout);
@@ -1411,11 +1412,14 @@ luzrt_status wide_number_large(luzrt_ctx* ctx, const WideJob& J, uint8_t* level_
     hipStream_t st = ctx->stream;
     uint3* level = reinterpret_cast<uint3*>(level_mem);
     uint2* sums = reinterpret_cast<uint2*>(level_mem + 1024);
-    k_wide_level_init<<<1, 64, 0, st>>>(J, level);
-    // a level has at most eight times the nodes of the one before; the host
-    // looks whether the tree has ended after the levels that most trees have
+    // the narrow levels by one workgroup, the wide ones by the whole chip; the
+    // host looks whether the tree has ended after as many as most trees have
+    WideJobs one{};
+    one.n = 1;
+    one.j[0] = J;
+    k_wide_number<<<1, 1024, 0, st>>>(one, 4096u, level);
     uint32_t done = 0;
-    for (uint32_t upto = 10; upto <= 64; upto += 6) {
+    for (uint32_t upto = 4; upto <= 64; upto += 4) {
         for (; done < upto; ++done) {
             k_wide_level_count<<<kWideLevelBlocks, kBlock, 0, st>>>(J, level + done, sums);
             k_wide_level_write<<<kWideLevelBlocks, kBlock, 0, st>>>(J, level + done, sums);
@@ -1466,18 +1470,19 @@ luzrt_status wide_build_some(luzrt_ctx* ctx, luzrt_blas* const* list, uint32_t c
         J.prims8 = b->prims8;
         J.count = b->wide_count_dev;
         J.block = blocks;
-        blocks += cdiv(J.n, kBlock);
+        J.blocks = cdiv(J.n, kBlock);
+        blocks += J.blocks;
         if (J.n <= kWideOneGroup) ++small;
     }
     k_wide_slots<<<blocks, kBlock, 0, st>>>(jobs);
     luzrt_status s = LUZRT_OK;
     if (small == count) {
-        k_wide_number<<<count, 1024, 0, st>>>(jobs);
+        k_wide_number<<<count, 1024, 0, st>>>(jobs, ~0u, nullptr);
     } else {
         WideJobs few{};
         for (uint32_t k = 0; k < count; ++k)
             if (jobs.j[k].n <= kWideOneGroup) few.j[few.n++] = jobs.j[k];
-        if (few.n) k_wide_number<<<few.n, 1024, 0, st>>>(few);
+        if (few.n) k_wide_number<<<few.n, 1024, 0, st>>>(few, ~0u, nullptr);
         for (uint32_t k = 0; k < count && s == LUZRT_OK; ++k)
             if (jobs.j[k].n > kWideOneGroup) s = wide_number_large(ctx, jobs.j[k], work);
     }
