@@ -311,37 +311,37 @@ __device__ inline int ray_step(RayState& r, STACK& st, const Node* tlas_nodes, c
     const bool b1 = box_hit(cur, qx.y, qx.w, qy.y, qy.w, qz.y, qz.w, tn1);
     const bool h0 = (qc.x != kEmpty) & b0;
     const bool h1 = (qc.y != kEmpty) & b1;
-    int first = (h0 && h1) ? (tn1 < tn0 ? 1 : 0) : (h0 ? 0 : 1);
-    r.next = kNone;
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        int c = k == 0 ? first : 1 - first;
-        bool h = c == 0 ? h0 : h1;
-        if (!h) continue;
-        uint32_t ch = c == 0 ? qc.x : qc.y;
-        if ((TLAS_FREE || r.in_blas) && (ch & kLeaf)) {
-            uint32_t slot = ch & ~kLeaf;
-            V3 a, b, cc;
-            load_tri(r.btris, slot, a, b, cc);
-            float T, det, U, V, W;
-            if (tri_test(r.tr, r.br.o, r.tmin, r.tmax, a, b, cc, T, det, U, V, W)) {
-                if (!CLOSEST) return kStepHit;
-                float t = __fdiv_rn(T, det);
-                if (better_hit(t, r.inst_slot, slot, *best, aux)) {
-                    best->found = true;
-                    best->t = t;
-                    best->inst_slot = r.inst_slot;
-                    best->tri_slot = slot;
-                    best->T = T; best->det = det; best->U = U; best->V = V; best->W = W;
-                    float m = t_margin(t);
-                    r.br.thi = t + m;
-                    r.wbr.thi = t + m;
-                }
-            }
-            continue;
+    // the hit leaves of a BLAS node (0, 1 or 2 triangles), and its other hit
+    // children: the nearer one next, the other stacked
+    const bool blas = TLAS_FREE || r.in_blas;
+    const bool l0 = h0 && blas && (qc.x & kLeaf), l1 = h1 && blas && (qc.y & kLeaf);
+    const bool n0 = h0 && !l0, n1 = h1 && !l1;
+    const bool second = n1 && (!n0 || tn1 < tn0);
+    r.next = second ? qc.y : (n0 ? qc.x : kNone);
+    if (n0 && n1 && !st.push(second ? qc.x : qc.y)) return kStepOverflow;
+    // One triangle test in a loop instead of one per child: lanes whose only
+    // leaf is child 0 and lanes whose only leaf is child 1 share a pass.
+    uint32_t leaf = l0 ? qc.x : qc.y, left = (l0 ? 1u : 0u) + (l1 ? 1u : 0u);
+    while (left) {
+        const uint32_t slot = leaf & ~kLeaf;
+        leaf = qc.y;
+        --left;
+        V3 a, b, cc;
+        load_tri(r.btris, slot, a, b, cc);
+        float T, det, U, V, W;
+        if (!tri_test(r.tr, r.br.o, r.tmin, r.tmax, a, b, cc, T, det, U, V, W)) continue;
+        if (!CLOSEST) return kStepHit;
+        float t = __fdiv_rn(T, det);
+        if (better_hit(t, r.inst_slot, slot, *best, aux)) {
+            best->found = true;
+            best->t = t;
+            best->inst_slot = r.inst_slot;
+            best->tri_slot = slot;
+            best->T = T; best->det = det; best->U = U; best->V = V; best->W = W;
+            float m = t_margin(t);
+            r.br.thi = t + m;
+            r.wbr.thi = t + m;
         }
-        if (r.next == kNone) r.next = ch;
-        else if (!st.push(ch)) return kStepOverflow;
     }
     return kStepContinue;
 }
