@@ -273,6 +273,7 @@ struct TraceLaunch {
     uint32_t* spill;       // per-lane overflow stack
     uint32_t max_steps;    // traversal steps per ray before it is abandoned (the context's limit)
     uint64_t max_rays;     // host's bound of the ray count (0: none); no more workgroups than it needs
+    uint32_t resident;     // workgroups that fit the chip at once
     bool wide;             // instance records point to 8-wide BLASes
     // Multi-scene launch (nscenes > 0): ray i belongs to the scene s with
     // scene_ray_base[s] <= i < scene_ray_base[s + 1], is generated from that

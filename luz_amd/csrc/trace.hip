@@ -153,15 +153,17 @@ __global__ __launch_bounds__(kBlock) void k_cull_rows(const uint32_t* counters, 
     cull_rows_lane(live_bits[g], R, w, g << 6, rows + row_base[g], hits + (size_t)g0 * R);
 }
 
-// Rays go to the waves in chunks.  A wave's first chunk is its own by its
-// position in the grid; the following ones it claims, one device-scope atomic
-// each.  A launch of at most kChunkMin rays per wave is dealt out whole that
-// way, in chunks as even as rows of 64 allow, and makes no claim: with every
-// chunk claimed, 256-ray chunks left most waves of a 256x256 frame without
-// work, and each of them tried all claim counters in vain (49k atomics on 8
-// addresses): the 256x256 cube frame 161 -> 74 us, 1M incoherent rays 241 ->
-// 202 us.  Above that the
-// chunk follows the launch's ray count, 1/kChunkShare of an even share per
+// Rays go to the waves in chunks.  A launch of at most kChunkMin rays per
+// resident wave is dealt out, each of them one chunk by its position in the
+// grid (the first waves of all workgroups before their second ones, so that few
+// rays spread over all CUs), as even as rows of 64 allow, and makes no claim: with every chunk claimed, 256-ray
+// chunks left most waves of a 256x256 frame without work, and each of them
+// tried all claim counters in vain (49k atomics on 8 addresses): the 256x256
+// cube frame 161 -> 68 us, 1M incoherent rays 241 -> 183 us.
+// Above that a wave claims its chunks, one device-scope atomic each (the
+// workgroups that wait for a place on the chip would sit on a dealt chunk until
+// the end: the soft-shadow frame lost 4%).  The
+// chunk then follows the launch's ray count, 1/kChunkShare of an even share per
 // wave, kept within kChunkMin .. kChunkMax rays: the rays in flight on the
 // whole GPU (waves x chunk) then cover few image rows of one light at a time,
 // so the BVH nodes they read stay in L2, while the claims stay below the rate
@@ -171,8 +173,10 @@ __global__ __launch_bounds__(kBlock) void k_cull_rows(const uint32_t* counters, 
 // chunks of 64 or 128 lost again to the counter (3.6 and 2.3 ms at 1 + 1).
 constexpr uint32_t kChunkMin = 256, kChunkMax = 512, kChunkShare = 12;
 
-__device__ inline uint32_t claim_chunk(uint32_t nrays, uint32_t nwaves) {
-    if (nrays <= nwaves * kChunkMin) return nrays ? ((nrays - 1) / nwaves / 64u + 1u) * 64u : 64u;
+__device__ inline bool deal_rays(uint32_t nrays, uint32_t resident) { return nrays <= resident * kChunkMin; }
+// grain: 64 where a wave's rays should be whole rows of neighbouring pixels
+__device__ inline uint32_t claim_chunk(uint32_t nrays, uint32_t nwaves, uint32_t resident, uint32_t grain) {
+    if (deal_rays(nrays, resident)) return nrays ? ((nrays - 1) / resident / grain + 1u) * grain : grain;
     const uint32_t c = (nrays / (nwaves * kChunkShare)) & ~63u;
     return c < kChunkMin ? kChunkMin : (c > kChunkMax ? kChunkMax : c);
 }
@@ -266,28 +270,28 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
     const uint32_t A = SRC == kGen ? L.counters[kCntActive] : 1u;   // active pixels
     const uint32_t R = SRC == kGen ? L.ds->r_total : 1u;             // ray slots per pixel
     const uint32_t G = SRC == kGen ? L.ds->ray_group : 0u;           // pixels per ray group
-    const uint32_t chunk = claim_chunk(nrays, total / 64u);
+    const uint32_t resident = min(gridDim.x, L.resident) * (kBlock / 64);   // waves on the chip at once
+    const uint32_t chunk = claim_chunk(nrays, total / 64u, resident, SRC == kRays ? 16u : 64u);
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     RayState r;
     uint32_t ray = kNone;
     bool open = true;
     uint32_t chunk_next = 0, chunk_end = 0;  // wave-uniform
-    // Chunks c, c + 8, c + 16, ... of the launch's rays belong to claim counter
-    // c, so the waves advance one front through the rays (the BVH nodes in use
-    // stay few) while their atomics spread over 8 addresses.  The workgroups b
-    // with b % 8 == c take the first of them, one per wave, without a claim
-    // (`dealt` of them); the counter hands out the rest.  A wave claims from the
-    // counter of its workgroup and moves to the next one when a counter's chunks
-    // run past the last ray (known without an atomic where all were dealt).
+    // Claim counter c hands out chunks c, c + 8, c + 16, ... of the launch's
+    // rays, so the waves still advance one front through the rays (the BVH
+    // nodes in use stay few) while their atomics spread over 8 addresses.  A
+    // wave starts on the counter of its workgroup and moves to the next one
+    // when a counter's chunks run past the last ray.
     const uint32_t seg0 = blockIdx.x % kClaimSegments;
     uint32_t seg = 0;   // counters this wave has found exhausted (wave-uniform)
-    {
-        const uint64_t base = ((uint64_t)(blockIdx.x / kClaimSegments * (kBlock / 64) + (tid >> 6)) * kClaimSegments +
-                               seg0) * chunk;
+    if (deal_rays(nrays, resident)) {
+        const uint32_t w = (tid >> 6) * (resident / (kBlock / 64)) + blockIdx.x;
+        const uint64_t base = blockIdx.x < resident / (kBlock / 64) ? (uint64_t)w * chunk : nrays;
         if (base < nrays) {
             chunk_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
             chunk_end = nrays - chunk_next > chunk ? chunk_next + chunk : nrays;
         }
+        seg = kClaimSegments;
     }
     for (;;) {
         if (open) {
@@ -300,16 +304,11 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
                         break;
                     }
                     const uint32_t c = (seg0 + seg) % kClaimSegments;
-                    const uint32_t dealt = (gridDim.x + kClaimSegments - 1 - c) / kClaimSegments * (kBlock / 64);
-                    if (((uint64_t)dealt * kClaimSegments + c) * chunk >= nrays) {
-                        ++seg;
-                        continue;
-                    }
                     uint32_t got = 0;
                     if (lane == 0) got = atomicAdd(&L.counters[kClaimBase + c * kClaimStride], 1u);
                     // only lane 0 holds the atomic's result: every decision
                     // below uses the broadcast copy, so the claim stays uniform
-                    const uint64_t base = ((uint64_t)(dealt + __shfl(got, 0)) * kClaimSegments + c) * chunk;
+                    const uint64_t base = ((uint64_t)__shfl(got, 0) * kClaimSegments + c) * chunk;
                     if (base < nrays) {
                         chunk_next = (uint32_t)base;
                         chunk_end = nrays - chunk_next > chunk ? chunk_next + chunk : nrays;
@@ -469,6 +468,8 @@ luzrt_status launch_trace(luzrt_ctx* ctx, const TraceLaunch& L) {
     TraceLaunch l = L;
     l.spill = (uint32_t*)ctx->spill.ptr;
     l.max_steps = ctx->max_steps;
+    // five waves per SIMD (launch bounds), four with 32 LDS stack entries per lane
+    l.resident = std::max(1u, (uint32_t)ctx->num_cus * (ctx->stack_entries > 16 ? 4u : 5u));
     uint32_t refill = ctx->refill_threshold ? ctx->refill_threshold : 64u;
     auto launch = [&](auto kern) { kern<<<groups, kBlock, 0, ctx->stream>>>(l, refill); };
     const uint32_t sd = ctx->stack_entries;
@@ -824,6 +825,7 @@ extern "C" luzrt_status luzrt_trace_visibility_static(luzrt_ctx* ctx, const luzr
         L.act_rec = act_rec;
         uint32_t groups = (uint32_t)ctx->num_cus * ctx->groups_per_cu;
         groups = groups == 0 ? 1u : (groups > kStaticGroups ? kStaticGroups : groups);
+        L.resident = std::max(1u, (uint32_t)ctx->num_cus * 5u);
         const uint32_t refill = ctx->refill_threshold ? ctx->refill_threshold : 64u;
         if (L.wide)
             k_trace_any<true, kStaticShort, kGen, kStaticDepth><<<groups, kBlock, 0, st>>>(L, refill);
