@@ -194,9 +194,10 @@ __global__ void k_bray_base(BatchTables T, uint32_t* counters, uint32_t align) {
 // the group's pixel frames come from its scene's G-buffer planes as the
 // traversal generates them.
 __global__ __launch_bounds__(kBlock) void k_bcull(BatchTables T, const BatchTlas* tl, uint32_t groups_max,
-                                                  uint32_t kinds, uint64_t* cand, uint64_t* live_bits,
-                                                  uint32_t* live_count) {
-    __shared__ uint64_t s_mask[kBlock / 64][(LUZRT_MAX_LIGHTS + 1) * kCandWords];
+                                                  uint32_t kinds, uint64_t* cand, uint64_t* pix,
+                                                  GroupRows* live_bits, uint32_t* live_count) {
+    __shared__ uint64_t s_mask[kBlock / 64][(LUZRT_MAX_LIGHTS + 1) * kKindWords];
+    __shared__ SlotBox s_box[kBlock / 64][kMaxCullInst];
     __shared__ luzrt_light s_light[LUZRT_MAX_LIGHTS];
     __shared__ uint32_t s_slot[LUZRT_MAX_LIGHTS];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -219,7 +220,7 @@ __global__ __launch_bounds__(kBlock) void k_bcull(BatchTables T, const BatchTlas
     if (g >= groups_max) return;
     if (g >= total) {
         if (lane == 0) {
-            live_bits[g] = 0;
+            live_bits[g] = GroupRows{0, 0};
             live_count[g] = 0;
         }
         return;
@@ -232,23 +233,26 @@ __global__ __launch_bounds__(kBlock) void k_bcull(BatchTables T, const BatchTlas
     // lanes past the last active pixel repeat the group's first pixel
     const uint32_t ar = a < A ? a : g0;
     const PixelFrame f = pixel_frame(bt.position, bt.normal, bt.width, ds->s, bt.act_list[ar]);
-    uint64_t bits;
+    const uint64_t pixels = __ballot(a < A);
+    uint64_t* const cand_g = cand + (size_t)g * kinds * kCandWords;
+    uint64_t* const pix_g = pix + (size_t)g * kinds;
+    GroupRows bits;
     if (one_scene)
-        bits = cull_group(f, s_light, s_slot, (uint32_t)ds->s.num_lights, ds->r_shadow, ds->r_total,
-                          ds->s.ao_max, bt.slot_box, bt.ninst, s_mask[wave], cand + (size_t)g * kinds * kCandWords);
+        bits = cull_group(f, pixels, s_light, s_slot, (uint32_t)ds->s.num_lights, ds->r_shadow, ds->r_total,
+                          ds->s.ao_min, ds->s.ao_max, bt.slot_box, bt.ninst, s_mask[wave], s_box[wave], cand_g, pix_g);
     else
-        bits = cull_group(f, ds->s.lights, ds->slot_base, (uint32_t)ds->s.num_lights, ds->r_shadow, ds->r_total,
-                          ds->s.ao_max, bt.slot_box, bt.ninst, s_mask[wave], cand + (size_t)g * kinds * kCandWords);
+        bits = cull_group(f, pixels, ds->s.lights, ds->slot_base, (uint32_t)ds->s.num_lights, ds->r_shadow,
+                          ds->r_total, ds->s.ao_min, ds->s.ao_max, bt.slot_box, bt.ninst, s_mask[wave], s_box[wave], cand_g, pix_g);
     if (lane == 0) {
         live_bits[g] = bits;
-        live_count[g] = (uint32_t)__popcll(bits);
+        live_count[g] = (uint32_t)__popcll(bits.live);
     }
 }
 
 // Live rows of the batch's groups (codes g << 6 | j) and the culled rows' hit
 // bytes (misses), as k_cull_rows.
 __global__ __launch_bounds__(kBlock) void k_bcull_rows(BatchTables T, uint32_t groups_max,
-                                                       const uint64_t* live_bits, const uint32_t* row_base,
+                                                       const GroupRows* live_bits, const uint32_t* row_base,
                                                        uint32_t* rows, uint8_t* hits) {
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t g = blockIdx.x * (kBlock / 64) + wave;
@@ -341,12 +345,12 @@ struct luzrt_batch {
     uint64_t max_rays = 0;
     uint32_t total_cblk = 0, total_pblk = 0, total_ppx = 0;
     DevBuf hits;
-    // ray-group culling (decided at creation): candidate masks (kinds per
-    // group), live-row bits and counts, the live-row list
+    // ray-group culling (decided at creation): candidate and pixel masks (kinds
+    // per group), live-row bits and counts, the live-row list
     bool cull = false;
     uint32_t cull_kinds = 0, groups_max = 0;
     uint64_t* cull_cand = nullptr;
-    uint64_t* cull_bits = nullptr;
+    GroupRows* cull_bits = nullptr;
     uint32_t* cull_counts = nullptr;
     uint32_t* cull_rows = nullptr;
     // graph
@@ -438,6 +442,9 @@ luzrt_status upload_refits(luzrt_ctx* ctx, luzrt_batch* b) {
     return LUZRT_OK;
 }
 
+// The pixel masks, behind the candidate masks.
+uint64_t* batch_pixels(const luzrt_batch* b) { return b->cull_cand + (size_t)b->groups_max * b->cull_kinds * kCandWords; }
+
 // The frame's launches, in order, on ctx->stream (captured or issued directly).
 luzrt_status issue_frame(luzrt_ctx* ctx, luzrt_batch* b) {
     hipStream_t st = ctx->stream;
@@ -472,7 +479,7 @@ luzrt_status issue_frame(luzrt_ctx* ctx, luzrt_batch* b) {
     if (b->cull) {
         const uint32_t gblocks = cdiv(b->groups_max, kBlock / 64);
         k_bcull<<<gblocks, kBlock, 0, st>>>(b->tables, b->dev_tlas, b->groups_max, b->cull_kinds, b->cull_cand,
-                                           b->cull_bits, b->cull_counts);
+                                           batch_pixels(b), b->cull_bits, b->cull_counts);
         launch_cull_scan(st, b->cull_counts, b->groups_max, b->counters);
         k_bcull_rows<<<gblocks, kBlock, 0, st>>>(b->tables, b->groups_max, b->cull_bits, b->cull_counts,
                                                 b->cull_rows, (uint8_t*)b->hits.ptr);
@@ -482,6 +489,7 @@ luzrt_status issue_frame(luzrt_ctx* ctx, luzrt_batch* b) {
     if (b->cull) {
         L.live_rows = b->cull_rows;
         L.cand = b->cull_cand;
+        L.pixels = batch_pixels(b);
         L.cand_kinds = b->cull_kinds;
         L.scene_group_base = b->tables.gbase;
     }
@@ -666,8 +674,8 @@ luzrt_status luzrt_batch_create(luzrt_ctx* ctx, const luzrt_batch_scene* scenes,
     B_ALLOC(b->dev_tlas, count * sizeof(BatchTlas));
     B_ALLOC(b->dev_jobs, count * sizeof(TlasJob));
     if (b->cull) {
-        B_ALLOC(b->cull_cand, groups * kinds * kCandWords * 8);
-        B_ALLOC(b->cull_bits, groups * 8);
+        B_ALLOC(b->cull_cand, groups * kinds * kKindWords * 8);
+        B_ALLOC(b->cull_bits, groups * sizeof(GroupRows));
         B_ALLOC(b->cull_counts, ((groups + 3) & ~uint64_t(3)) * 4);
         B_ALLOC(b->cull_rows, groups * rmax * 4);
     }

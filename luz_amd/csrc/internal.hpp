@@ -298,9 +298,11 @@ struct TraceLaunch {
     // active pixels of group g, encoded g << 6 | j), and a ray of kind k (its
     // light, or num_lights for AO) starts from the candidate slots of mask
     // words cand[(g * cand_kinds + k) * kCandWords ..] instead of the TLAS root.
+    // A row is traced for the group's pixels in pixels[g * cand_kinds + k] only.
     // Null: no culling.
     const uint32_t* live_rows;
     const uint64_t* cand;
+    const uint64_t* pixels;
     const float* slot_box;   // the TLAS slots' padded world boxes (6 floats each)
     uint32_t cand_kinds;
 };

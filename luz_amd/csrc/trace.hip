@@ -93,9 +93,10 @@ __global__ __launch_bounds__(kBlock) void k_compact_write(const luzrt_gbuffer gb
 __global__ __launch_bounds__(kBlock) void k_cull(const float4* act_rec, const uint32_t* counters,
                                                  const DevScene* ds, const float* slot_box,
                                                  uint32_t ninst, uint32_t ngroups, uint32_t kinds,
-                                                 uint64_t* cand, uint64_t* live_bits,
+                                                 uint64_t* cand, uint64_t* pix, GroupRows* live_bits,
                                                  uint32_t* live_count) {
-    __shared__ uint64_t s_mask[kBlock / 64][(LUZRT_MAX_LIGHTS + 1) * kCandWords];
+    __shared__ uint64_t s_mask[kBlock / 64][(LUZRT_MAX_LIGHTS + 1) * kKindWords];
+    __shared__ SlotBox s_box[kBlock / 64][kMaxCullInst];
     __shared__ luzrt_light s_light[LUZRT_MAX_LIGHTS];
     __shared__ uint32_t s_slot[LUZRT_MAX_LIGHTS];
     {
@@ -112,7 +113,7 @@ __global__ __launch_bounds__(kBlock) void k_cull(const float4* act_rec, const ui
     const uint32_t A = counters[kCntActive];
     if ((uint64_t)g * kCullGroup >= A) {
         if (lane == 0) {
-            live_bits[g] = 0;
+            live_bits[g] = GroupRows{0, 0};
             live_count[g] = 0;
         }
         return;
@@ -121,12 +122,12 @@ __global__ __launch_bounds__(kBlock) void k_cull(const float4* act_rec, const ui
     // lanes past the last active pixel repeat the group's first pixel
     const uint32_t ar = a < A ? a : g * kCullGroup;
     const PixelFrame f = pixel_from_record(act_rec[2 * (size_t)ar], act_rec[2 * (size_t)ar + 1]);
-    const uint64_t bits = cull_group(f, s_light, s_slot, (uint32_t)ds->s.num_lights, ds->r_shadow, ds->r_total,
-                                     ds->s.ao_max, slot_box, ninst, s_mask[wave],
-                                     cand + (size_t)g * kinds * kCandWords);
+    const GroupRows bits = cull_group(f, __ballot(a < A), s_light, s_slot, (uint32_t)ds->s.num_lights, ds->r_shadow,
+                                      ds->r_total, ds->s.ao_min, ds->s.ao_max, slot_box, ninst, s_mask[wave], s_box[wave],
+                                      cand + (size_t)g * kinds * kCandWords, pix + (size_t)g * kinds);
     if (lane == 0) {
         live_bits[g] = bits;
-        live_count[g] = (uint32_t)__popcll(bits);
+        live_count[g] = (uint32_t)__popcll(bits.live);
     }
 }
 
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(1024) void k_cull_scan(uint32_t* counts, uint32_t n
 // One wave per group: its live rows into the row list, its culled rows'
 // hit bytes written as misses (cull_rows_lane).
 __global__ __launch_bounds__(kBlock) void k_cull_rows(const uint32_t* counters, const DevScene* ds,
-                                                      uint32_t ngroups, const uint64_t* live_bits,
+                                                      uint32_t ngroups, const GroupRows* live_bits,
                                                       const uint32_t* row_base, uint32_t* rows,
                                                       uint8_t* hits) {
     const uint32_t wave = threadIdx.x >> 6;
@@ -193,6 +194,13 @@ __device__ inline uint32_t scene_of_ray(const uint32_t* base, uint32_t n, uint32
     return lo;
 }
 
+// Kind of the rays of a live row in a multi-scene launch.
+__device__ inline uint32_t row_kind_of_scene(const TraceLaunch& L, const uint32_t* sgbase, uint32_t row) {
+    const DevScene* ds = L.scene_tlas[scene_of_ray(sgbase, L.nscenes, row >> 6)].ds;
+    const uint32_t slot = row & 63u;
+    return slot < ds->r_shadow ? (uint32_t)slot_light(ds, slot) : (uint32_t)ds->s.num_lights;
+}
+
 // Where a launch's rays come from.  kRays: ray records (origin, tmin;
 // direction, tmax).  kGen: computed at claim time from the G-buffer and the
 // scene block (gen_ray).  kBatch: likewise for many scenes in one launch,
@@ -204,8 +212,9 @@ enum RaySource { kRays = 0, kBatch = 1, kGen = 2 };
 // A culled ray's start: the candidate slots (mask words cw) whose padded
 // boxes it meets, the test the TLAS node above each slot would make; the
 // first is entered now, the others from the stack, and no TLAS node is visited.
+// False where it meets none.
 template <typename STACK>
-__device__ inline void enter_candidates(RayState& r, STACK& st, const uint64_t* cw, const float* slot_box) {
+__device__ inline bool enter_candidates(RayState& r, STACK& st, const uint64_t* cw, const float* slot_box) {
     r.next = kNone;
     for (uint32_t w = 0; w < kCandWords; ++w) {
         uint64_t m = cw[w];
@@ -220,7 +229,13 @@ __device__ inline void enter_candidates(RayState& r, STACK& st, const uint64_t* 
             }
         }
     }
+    return r.next != kNone;
 }
+// Lanes that wait for an instance entry at once (measured 1 / 8 / 16 / 32: soft
+// shadows at 1277x713 1096 / 936 / 1115 / 1342 us, the 1080p sphere field 838 /
+// 768 / 737 / 889 us, the 4K terrain 19.0 / 18.1 / 17.9 / 19.0 ms).
+constexpr uint32_t kEnterLanes = 8;
+
 
 // CULLED (gen launches after k_cull): the live rows only, each ray starting
 // from its group's candidate slots; no TLAS node is visited, so only the
@@ -236,7 +251,14 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
     // ray starts there, so its reads stop competing with BLAS data in L1.  15 KB
     // keeps five 256-lane workgroups (16-entry stacks) resident per CU.
     __shared__ float4 stlas[BATCH ? 4 : (CULLED ? kMaxCullInst * 4 : kTlasLdsEntries * 4)];
+    __shared__ uint8_t s_pick[kBlock / 64][CULLED ? 64 : 1];   // pixels of the row being given out, per wave
+    __shared__ uint8_t s_kind[CULLED && !BATCH ? 64 : 1];      // kind of each slot (its light, or num_lights)
     const uint32_t tid = threadIdx.x;
+    if (CULLED && !BATCH) {
+        if (tid < 64)
+            s_kind[tid] = (uint8_t)(tid < L.ds->r_shadow ? slot_light(L.ds, tid) : L.ds->s.num_lights);
+        __syncthreads();
+    }
     if (BATCH) {
         for (uint32_t i = tid; i <= L.nscenes; i += kBlock) {
             sbase[i] = L.scene_ray_base[i];
@@ -277,6 +299,8 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
     uint32_t ray = kNone;
     bool open = true;
     uint32_t chunk_next = 0, chunk_end = 0;  // wave-uniform
+    uint64_t pick = 0;        // CULLED: the current row's pixels not yet given out (wave-uniform)
+    uint32_t pick_row = 0;
     // Claim counter c hands out chunks c, c + 8, c + 16, ... of the launch's
     // rays, so the waves still advance one front through the rays (the BVH
     // nodes in use stay few) while their atomics spread over 8 addresses.  A
@@ -293,49 +317,83 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
         }
         seg = kClaimSegments;
     }
+    // The next chunk, when the current one is used up (all lanes).
+    auto claim = [&]() {
+        while (chunk_next >= chunk_end && open) {
+            if (seg == kClaimSegments) {
+                open = false;
+                break;
+            }
+            const uint32_t c = (seg0 + seg) % kClaimSegments;
+            uint32_t got = 0;
+            if (lane == 0) got = atomicAdd(&L.counters[kClaimBase + c * kClaimStride], 1u);
+            // only lane 0 holds the atomic's result: every decision
+            // below uses the broadcast copy, so the claim stays uniform
+            const uint64_t base = ((uint64_t)__shfl(got, 0) * kClaimSegments + c) * chunk;
+            if (base < nrays) {
+                chunk_next = (uint32_t)base;
+                chunk_end = nrays - chunk_next > chunk ? chunk_next + chunk : nrays;
+            } else {
+                ++seg;
+            }
+        }
+    };
     for (;;) {
         if (open) {
             uint64_t idle = __ballot(ray == kNone);
             uint32_t nidle = (uint32_t)__popcll(idle);
             if (nidle >= refill || nidle == 64u) {
-                while (chunk_next >= chunk_end && open) {
-                    if (seg == kClaimSegments) {
-                        open = false;
-                        break;
-                    }
-                    const uint32_t c = (seg0 + seg) % kClaimSegments;
-                    uint32_t got = 0;
-                    if (lane == 0) got = atomicAdd(&L.counters[kClaimBase + c * kClaimStride], 1u);
-                    // only lane 0 holds the atomic's result: every decision
-                    // below uses the broadcast copy, so the claim stays uniform
-                    const uint64_t base = ((uint64_t)__shfl(got, 0) * kClaimSegments + c) * chunk;
-                    if (base < nrays) {
-                        chunk_next = (uint32_t)base;
-                        chunk_end = nrays - chunk_next > chunk ? chunk_next + chunk : nrays;
-                    } else {
-                        ++seg;
+                if (!CULLED) claim();
+                // CULLED: the idle lanes take the pixels that the live rows are
+                // traced for, from as many rows as it takes: lane with idle rank
+                // k the k-th pixel left
+                const uint32_t rank = (uint32_t)__popcll(idle & lt);
+                uint32_t row = 0, row_px = kNone;
+                if (CULLED) {
+                    uint32_t given = 0;
+                    while (given < nidle) {
+                        if (pick == 0ull) {
+                            claim();
+                            if (!open) break;
+                            const uint32_t code = L.live_rows[chunk_next >> 6];
+                            chunk_next += 64;
+                            pick_row = (uint32_t)__builtin_amdgcn_readfirstlane((int)code);
+                            const uint32_t kind = bcull ? row_kind_of_scene(L, sgbase, pick_row) : s_kind[pick_row & 63u];
+                            const uint64_t px = L.pixels[(size_t)(pick_row >> 6) * L.cand_kinds + kind];
+                            pick = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(px >> 32)) << 32) |
+                                   (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)px);
+                            continue;
+                        }
+                        const uint32_t n = (uint32_t)__popcll(pick), take = n < nidle - given ? n : nidle - given;
+                        if ((pick >> lane) & 1ull) s_pick[tid >> 6][__popcll(pick & lt)] = (uint8_t)lane;
+                        __builtin_amdgcn_wave_barrier();
+                        if (ray == kNone && rank >= given && rank < given + take) {
+                            row = pick_row;
+                            row_px = s_pick[tid >> 6][rank - given];
+                        }
+                        const uint32_t last = s_pick[tid >> 6][take - 1];
+                        __builtin_amdgcn_wave_barrier();
+                        pick = take == n ? 0ull
+                                         : pick & ~((2ull << (uint32_t)__builtin_amdgcn_readfirstlane((int)last)) - 1ull);
+                        given += take;
                     }
                 }
-                uint32_t avail = chunk_end > chunk_next ? chunk_end - chunk_next : 0u;
-                uint32_t take = nidle < avail ? nidle : avail;
+                const uint32_t avail = CULLED ? 0u : (chunk_end > chunk_next ? chunk_end - chunk_next : 0u);
+                const uint32_t take = nidle < avail ? nidle : avail;
                 if (ray == kNone) {
-                    uint32_t rank = (uint32_t)__popcll(idle & lt);
-                    if (rank < take) {
-                        uint32_t rid = chunk_next + rank;
+                    if (CULLED ? row_px != kNone : rank < take) {
+                        const uint32_t rid = chunk_next + rank;
                         ray = rid;
                         if (bcull) {
                             // live row g << 6 | j of the batch's group space: the scene
                             // from the group bases, the hit byte at the ray's index
                             // in the scene's grouped order
-                            const uint32_t row = L.live_rows[rid >> 6], i = rid & 63u;
-                            const uint32_t g = row >> 6, slot = row & 63u;
+                            const uint32_t i = row_px, g = row >> 6, slot = row & 63u;
                             const uint32_t sc = scene_of_ray(sgbase, L.nscenes, g);
                             const BatchTlas& bt = L.scene_tlas[sc];
                             const uint32_t As = L.scene_active[sc], g0 = (g - sgbase[sc]) * kCullGroup;
                             const uint32_t a = g0 + i;
-                            if (a >= As) {
-                                ray = kNone;   // past the last pixel of a partial group
-                            } else {
+                            {
                                 const DevScene* dsc = bt.ds;
                                 const uint32_t Rs = dsc->r_total, rs = dsc->r_shadow;
                                 const uint32_t w = As - g0 < kCullGroup ? As - g0 : kCullGroup;
@@ -350,7 +408,10 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
                                                             bt.act_list[a]),
                                            slot, l, o, d, tmin, tmax);
                                 ray_begin(r, st, o, d, tmin, tmax);
-                                enter_candidates(r, st, cw, bt.slot_box);
+                                if (!enter_candidates(r, st, cw, bt.slot_box)) {
+                                    L.hits[ray] = 0;
+                                    ray = kNone;
+                                }
                             }
                         } else if (BATCH) {
                             const uint32_t sc = scene_of_ray(sbase, L.nscenes, rid);
@@ -379,30 +440,27 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
                                 if (cull) {
                                     // live row g << 6 | j: slot j of the group's pixel i; its hit
                                     // byte is the ray's grouped-order index
-                                    const uint32_t row = L.live_rows[rid >> 6], i = rid & 63u;
-                                    const uint32_t g = row >> 6, g0 = g * kCullGroup;
+                                    const uint32_t i = row_px, g = row >> 6, g0 = g * kCullGroup;
                                     slot = row & 63u;
                                     a = g0 + i;
-                                    if (a < A) {
-                                        const uint32_t w = A - g0 < kCullGroup ? A - g0 : kCullGroup;
-                                        ray = g0 * R + slot * w + i;
-                                        const uint32_t kind = slot < rs ? (uint32_t)slot_light(L.ds, slot)
-                                                                        : (uint32_t)L.ds->s.num_lights;
-                                        cw = L.cand + ((size_t)g * L.cand_kinds + kind) * kCandWords;
-                                    } else {
-                                        ray = kNone;   // past the last pixel of a partial group
-                                    }
+                                    const uint32_t w = A - g0 < kCullGroup ? A - g0 : kCullGroup;
+                                    ray = g0 * R + slot * w + i;
+                                    cw = L.cand + ((size_t)g * L.cand_kinds + s_kind[slot]) * kCandWords;
                                 } else {
                                     ray_slot(rid, A, R, G, slot, a);
                                 }
-                                if (ray != kNone) {
+                                {
                                     const float4 r0 = L.act_rec[2 * (size_t)a], r1 = L.act_rec[2 * (size_t)a + 1];
                                     V3 o, d;
                                     float tmin, tmax;
                                     gen_ray_of(L.ds, pixel_from_record(r0, r1), slot,
-                                               slot < rs ? slot_light(L.ds, slot) : 0, o, d, tmin, tmax);
+                                               slot < rs ? (cull ? (int)s_kind[slot] : slot_light(L.ds, slot)) : 0, o,
+                                               d, tmin, tmax);
                                     ray_begin(r, st, o, d, tmin, tmax);
-                                    if (cull) enter_candidates(r, st, cw, L.slot_box);
+                                    if (cull && !enter_candidates(r, st, cw, L.slot_box)) {
+                                        L.hits[ray] = 0;
+                                        ray = kNone;
+                                    }
                                 }
                             } else {
                                 float4 o = L.ray_o[(size_t)rid * L.ray_stride];
@@ -421,10 +479,32 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
         }
         if (ray != kNone) {
             for (;;) {
-                int res = ray_step<false, WIDE, StackT<SHORT, DEPTH>, CULLED>(r, st, tnodes, trecs, nullptr,
-                                                                          nullptr, tlas_lds, L.max_steps);
-                // a ray with nothing left to visit ends in this step, not in one more
-                if (res == kStepContinue && r.next == kNone && st.sp == 0) res = kStepDone;
+                int res = kStepContinue;
+                if (CULLED) {
+                    // Rays that stand before an instance wait until kEnterLanes of
+                    // them do, or until no ray of the wave is inside a BLAS: the
+                    // entry (two transforms, slab and triangle set-up) is as long
+                    // as a node visit, and one or two lanes at a time would run it
+                    // beside almost every visit of the others.
+                    const uint64_t before = __ballot(!r.in_blas);
+                    if ((uint32_t)__popcll(before) >= kEnterLanes || before == __ballot(true)) {
+                        if (!r.in_blas) {
+                            r.base = st.sp;
+                            if (++r.steps > L.max_steps) {
+                                res = kStepOverflow;
+                            } else if (!enter_instance<WIDE>(r, trecs, tlas_lds, r.next & ~kLeaf, r.tmax)) {
+                                if (st.sp == 0) res = kStepDone;
+                                else r.next = st.pop();
+                            }
+                        }
+                    }
+                    if (res == kStepContinue && r.in_blas) res = tlas_free_visit<WIDE>(r, st, L.max_steps);
+                } else {
+                    res = ray_step<false, WIDE, StackT<SHORT, DEPTH>>(r, st, tnodes, trecs, nullptr, nullptr, tlas_lds,
+                                                                      L.max_steps);
+                    // a ray with nothing left to visit ends in this step, not in one more
+                    if (res == kStepContinue && r.next == kNone && st.sp == 0) res = kStepDone;
+                }
                 if (res != kStepContinue) {
                     L.hits[ray] = res == kStepHit ? 1 : 0;
                     if (res == kStepOverflow) atomicOr(&L.counters[kCntError], 1u);
@@ -570,17 +650,20 @@ luzrt_status visibility_core(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
     ctx->last_culled = cull;
     const uint32_t kinds = (uint32_t)scene->num_lights + 1;
     if (cull) {
-        if ((s = ensure(ctx, ctx->cull_cand, (size_t)ngroups * kinds * kCandWords * 8)) != LUZRT_OK) return s;
-        const size_t counts_off = ((size_t)ngroups * 8 + 255) & ~size_t(255);   // 16-byte aligned counts
+        // candidate masks, then pixel masks
+        if ((s = ensure(ctx, ctx->cull_cand, (size_t)ngroups * kinds * kKindWords * 8)) != LUZRT_OK) return s;
+        const size_t counts_off = ((size_t)ngroups * sizeof(GroupRows) + 255) & ~size_t(255);   // 16-byte aligned counts
         if ((s = ensure(ctx, ctx->cull_bits, counts_off + (size_t)ngroups * 4 + 16)) != LUZRT_OK) return s;
         if ((s = ensure(ctx, ctx->cull_rows, (size_t)ngroups * ds.r_total * 4)) != LUZRT_OK) return s;
-        uint64_t* bits = (uint64_t*)ctx->cull_bits.ptr;
+        GroupRows* bits = (GroupRows*)ctx->cull_bits.ptr;
         uint32_t* counts = (uint32_t*)((uint8_t*)ctx->cull_bits.ptr + counts_off);
         const uint32_t gblocks = cdiv(ngroups, kBlock / 64);
         stage_begin(ctx, kStageRaygen);
         k_cull<<<gblocks, kBlock, 0, st>>>((const float4*)ctx->act_rec.ptr, counters, dsd,
                                            tlas_slot_boxes(tlas), tlas->count, ngroups, kinds,
-                                           (uint64_t*)ctx->cull_cand.ptr, bits, counts);
+                                           (uint64_t*)ctx->cull_cand.ptr,
+                                           (uint64_t*)ctx->cull_cand.ptr + (size_t)ngroups * kinds * kCandWords, bits,
+                                           counts);
         k_cull_scan<<<1, 1024, 0, st>>>(counts, ngroups, counters);
         k_cull_rows<<<gblocks, kBlock, 0, st>>>(counters, dsd, ngroups, bits, counts,
                                                 (uint32_t*)ctx->cull_rows.ptr, (uint8_t*)ctx->hits.ptr);
@@ -594,6 +677,7 @@ luzrt_status visibility_core(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
         if (cull) {
             L.live_rows = (const uint32_t*)ctx->cull_rows.ptr;
             L.cand = (const uint64_t*)ctx->cull_cand.ptr;
+            L.pixels = L.cand + (size_t)ngroups * kinds * kCandWords;
             L.slot_box = tlas_slot_boxes(tlas);
             L.cand_kinds = kinds;
         }

@@ -85,6 +85,7 @@ struct RayState {
     uint32_t inst_slot;
     uint32_t next;
     uint32_t steps;
+    int base;      // TLAS-free rays: the stack below the BLAS being walked
     bool in_blas;
 };
 
@@ -251,69 +252,41 @@ __device__ inline int wide_visit(RayState& r, STACK& st) {
     return kStepContinue;
 }
 
-// tlas_lds: tlas_nodes and recs point into LDS (a staged TLAS).
-// TLAS_FREE: the ray visits no TLAS node (its stack holds instance slots and
-// BLAS nodes only, as after ray-group culling), so the world slab ray is not
-// kept and every node visited is a BLAS node.
-template <bool CLOSEST, bool WIDE = false, typename STACK = Stack, bool TLAS_FREE = false>
-__device__ inline int ray_step(RayState& r, STACK& st, const Node* tlas_nodes, const InstRec* recs,
-                               const InstAux* aux, Best* best, bool tlas_lds = false,
-                               uint32_t max_steps = kMaxSteps) {
-    if (++r.steps > max_steps) return kStepOverflow;
-    if (r.next == kNone) {
-        if (st.sp == 0) return kStepDone;
-        r.next = st.pop();
-        if (r.next == kSentinel) {
-            r.in_blas = false;
-            r.next = kNone;
-            return kStepContinue;
-        }
-    }
-    // a TLAS-free ray holds only instance slots at the top level
-    if (TLAS_FREE && !r.in_blas && !(r.next & kLeaf)) return kStepOverflow;
-    if (!r.in_blas && (r.next & kLeaf)) {
-        uint32_t slot = r.next & ~kLeaf;
-        float4 w0, w1, w2;
-        uint4 pp;
-        load_rows(recs, slot, tlas_lds, w0, w1, w2, pp);
-        float w[12] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w};
-        V3 oo = xform_point(w, r.wbr.o);
-        V3 od = xform_vec(w, r.wd);
-        float thi = CLOSEST ? best->t : r.tmax;
-        r.br = box_setup(oo, od, r.tmin, thi);
-        r.tr = tri_setup(od);
-        // a NaN tmin on a NaN ray meets no box (every bound is NaN); wide_visit
-        // compares by the sign of a difference, which a NaN does not decide
-        if (WIDE && r.br.tlo != r.br.tlo && (oo.x != oo.x || od.x != od.x)) {
-            r.next = kNone;
-            return kStepContinue;
-        }
-        r.bnodes = reinterpret_cast<const Node*>(((uint64_t)pp.y << 32) | pp.x);
-        r.btris = reinterpret_cast<const float*>(((uint64_t)pp.w << 32) | pp.z);
-        r.inst_slot = slot;
-        if (!st.push(kSentinel)) return kStepOverflow;
-        r.in_blas = true;
-        r.next = 0;
-        return kStepContinue;
-    }
-    if (WIDE && (TLAS_FREE || r.in_blas)) return wide_visit(r, st);
-    float4 qx, qy, qz;
-    uint4 qc;
-    if (TLAS_FREE)
-        load_rows(r.bnodes, r.next, false, qx, qy, qz, qc);
-    else
-        load_rows(r.in_blas ? r.bnodes : tlas_nodes, r.next, tlas_lds && !r.in_blas, qx, qy, qz, qc);
+// Enters instance `slot`: its object-space ray and BLAS, the root next.  False
+// where the ray cannot meet any box of it.
+template <bool WIDE>
+__device__ inline bool enter_instance(RayState& r, const InstRec* recs, bool recs_lds, uint32_t slot, float thi) {
+    float4 w0, w1, w2;
+    uint4 pp;
+    load_rows(recs, slot, recs_lds, w0, w1, w2, pp);
+    float w[12] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w};
+    V3 oo = xform_point(w, r.wbr.o);
+    V3 od = xform_vec(w, r.wd);
+    r.br = box_setup(oo, od, r.tmin, thi);
+    r.tr = tri_setup(od);
+    // a NaN tmin on a NaN ray meets no box (every bound is NaN); wide_visit
+    // compares by the sign of a difference, which a NaN does not decide
+    if (WIDE && r.br.tlo != r.br.tlo && (oo.x != oo.x || od.x != od.x)) return false;
+    r.bnodes = reinterpret_cast<const Node*>(((uint64_t)pp.y << 32) | pp.x);
+    r.btris = reinterpret_cast<const float*>(((uint64_t)pp.w << 32) | pp.z);
+    r.inst_slot = slot;
+    r.in_blas = true;
+    r.next = 0;
+    return true;
+}
+
+// Visit of a binary node (rows qx, qy, qz, children qc) with slab ray cur: the
+// nearer hit child next, the other stacked; hit leaves of a BLAS are tested.
+template <bool CLOSEST, typename STACK>
+__device__ inline int binary_visit(RayState& r, STACK& st, bool blas, const BoxRay& cur, float4 qx, float4 qy,
+                                   float4 qz, uint4 qc, const InstAux* aux, Best* best) {
     float tn0, tn1;
-    // the ray of the tree being walked, selected per lane (restoring the world
-    // ray into a single slot on every return to the TLAS costs more)
-    const BoxRay cur = (TLAS_FREE || r.in_blas) ? r.br : r.wbr;
     const bool b0 = box_hit(cur, qx.x, qx.z, qy.x, qy.z, qz.x, qz.z, tn0);
     const bool b1 = box_hit(cur, qx.y, qx.w, qy.y, qy.w, qz.y, qz.w, tn1);
     const bool h0 = (qc.x != kEmpty) & b0;
     const bool h1 = (qc.y != kEmpty) & b1;
     // the hit leaves of a BLAS node (0, 1 or 2 triangles), and its other hit
     // children: the nearer one next, the other stacked
-    const bool blas = TLAS_FREE || r.in_blas;
     const bool l0 = h0 && blas && (qc.x & kLeaf), l1 = h1 && blas && (qc.y & kLeaf);
     const bool n0 = h0 && !l0, n1 = h1 && !l1;
     const bool second = n1 && (!n0 || tn1 < tn0);
@@ -344,6 +317,60 @@ __device__ inline int ray_step(RayState& r, STACK& st, const Node* tlas_nodes, c
         }
     }
     return kStepContinue;
+}
+
+// One node visit of a TLAS-free any-hit ray inside a BLAS (its stack holds
+// instance slots and, above r.base, nodes of that BLAS; no sentinel), and the
+// next node or instance slot taken from the stack.
+template <bool WIDE, typename STACK>
+__device__ inline int tlas_free_visit(RayState& r, STACK& st, uint32_t max_steps) {
+    if (++r.steps > max_steps) return kStepOverflow;
+    int res;
+    if (WIDE) {
+        res = wide_visit(r, st);
+    } else {
+        float4 qx, qy, qz;
+        uint4 qc;
+        load_rows(r.bnodes, r.next, false, qx, qy, qz, qc);
+        res = binary_visit<false>(r, st, true, r.br, qx, qy, qz, qc, nullptr, nullptr);
+    }
+    if (res != kStepContinue || r.next != kNone) return res;
+    if (st.sp == 0) return kStepDone;
+    r.in_blas = st.sp > r.base;
+    r.next = st.pop();
+    return kStepContinue;
+}
+
+// tlas_lds: tlas_nodes and recs point into LDS (a staged TLAS).
+template <bool CLOSEST, bool WIDE = false, typename STACK = Stack>
+__device__ inline int ray_step(RayState& r, STACK& st, const Node* tlas_nodes, const InstRec* recs,
+                               const InstAux* aux, Best* best, bool tlas_lds = false,
+                               uint32_t max_steps = kMaxSteps) {
+    if (++r.steps > max_steps) return kStepOverflow;
+    if (r.next == kNone) {
+        if (st.sp == 0) return kStepDone;
+        r.next = st.pop();
+        if (r.next == kSentinel) {
+            r.in_blas = false;
+            r.next = kNone;
+            return kStepContinue;
+        }
+    }
+    if (!r.in_blas && (r.next & kLeaf)) {
+        if (!st.push(kSentinel)) return kStepOverflow;
+        if (!enter_instance<WIDE>(r, recs, tlas_lds, r.next & ~kLeaf, CLOSEST ? best->t : r.tmax)) {
+            r.next = kNone;
+            r.in_blas = true;   // the sentinel comes next
+        }
+        return kStepContinue;
+    }
+    if (WIDE && r.in_blas) return wide_visit(r, st);
+    float4 qx, qy, qz;
+    uint4 qc;
+    load_rows(r.in_blas ? r.bnodes : tlas_nodes, r.next, tlas_lds && !r.in_blas, qx, qy, qz, qc);
+    // the ray of the tree being walked, selected per lane (restoring the world
+    // ray into a single slot on every return to the TLAS costs more)
+    return binary_visit<CLOSEST>(r, st, r.in_blas, r.in_blas ? r.br : r.wbr, qx, qy, qz, qc, aux, best);
 }
 
 }  // namespace luz

@@ -68,3 +68,59 @@ def test_special_rays_meet_the_same_triangles_in_both_trees(ctx):
     print(f"{int(got[0].sum())} of {len(rays)} rays hit", flush=True)
     assert 0 < got[0].sum() < len(rays)
     np.testing.assert_array_equal(got[1], got[0])
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("size", [(1, 1), (64, 1), (65, 3), (131, 77)])
+@pytest.mark.parametrize("lights", ["axis", "at_pixel", "near"])
+def test_culled_pixels_change_no_count(ctx, size, lights, wide):
+    """Culling by pixel keeps every count, on 102 instances (both words of a
+    candidate mask) with whole, partial and single-pixel groups: a directional
+    light along an axis (segments without extent in two axes), a point light at a
+    pixel's own position, and one just off the surface with a large radius; AO
+    rays far shorter and longer than the distance between instances."""
+    W, H = size
+    c = api.Context(0) if wide else ctx
+    if wide:
+        c.set_precision(api.PRECISION_WIDE)
+    s = api.HostScene(api.SCENE_SPHERES, 0)
+    g = api.GPUScene(c, s)
+    _, _, cam = s.camera()
+    o2w, mesh, mats = s.nodes()
+    moved = o2w.copy()
+    moved[:, 3::4] += np.float32([7.0, 5.0, 3.0])
+    o2w, mesh = np.concatenate([o2w, moved]), np.concatenate([mesh, mesh])
+    tlas = c.create_tlas(len(mesh))
+    tlas.build([api.make_instance(g.blas(int(m)), o2w[i], i) for i, m in enumerate(mesh)])
+    o = oracle_scene(s)
+    o.set_instances(o2w, mesh)
+    gd = api.GBufferDevice(c, W, H)
+    c.primary_gbuffer(tlas, cam, mats + mats, gd.desc())
+    gbuf = gd.download()
+    covered = np.flatnonzero(gbuf["normal"].reshape(H * W, -1)[:, :3].any(1))
+    sb = s.pack()
+    if len(covered):
+        p = gbuf["position"].reshape(H * W, -1)[covered[len(covered) // 2], :3]
+        for l in range(sb.num_lights):
+            light = sb.lights[l]
+            if lights == "axis":
+                light.type = api.LIGHT_DIRECTIONAL
+                light.direction[:] = [(0.0, -1.0, 0.0), (1.0, 0.0, 0.0), (0.0, 0.0, -1.0)][l % 3]
+            else:
+                light.type = api.LIGHT_POINT
+                off = 0.0 if lights == "at_pixel" else 0.02
+                light.position[:] = [float(v) + off for v in p]
+                light.radius = 0.5 if lights == "near" else 0.0
+    nl = sb.num_lights
+    for ao_max in (1 / 16, 4.0):
+        sb.ao_max = ao_max
+        want_sh, want_ao, _ = o.trace_visibility(gbuf, W, H, sb)
+        dsh, dao = c.buffer(nl * W * H), c.buffer(W * H)
+        print(f"{W}x{H} {lights} wide {wide} AO {ao_max}: {len(covered)} pixels", flush=True)
+        c.trace_visibility(tlas, gd.desc(), sb, dsh, dao)
+        np.testing.assert_array_equal(dsh.download(np.uint8, (nl, W * H)), want_sh)
+        np.testing.assert_array_equal(dao.download(np.uint8, W * H), want_ao)
+    tlas.destroy()
+    g.close()
+    if wide:
+        c.close()
