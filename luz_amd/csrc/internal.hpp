@@ -246,7 +246,7 @@ struct DevScene {
 
 // Device counters of one visibility call (ctx->counters).
 enum Counter { kCntFetch = 0, kCntActive = 1, kCntError = 2, kCntRays = 3, kCntBuildError = 4,
-               kCntPrimary = 5, kCntLive = 6, kCntCount = 8 };
+               kCntLive = 6, kCntCount = 8 };
 // A traversal launch claims its rays in chunks from kClaimSegments counters,
 // counter c owning chunks c, c + 8, c + 16, ..., each on a 128-byte line of
 // its own after the Counter array: one counter took every wave's
@@ -255,12 +255,19 @@ enum Counter { kCntFetch = 0, kCntActive = 1, kCntError = 2, kCntRays = 3, kCntB
 constexpr uint32_t kClaimSegments = 8;
 constexpr uint32_t kClaimBase = 256;      // word index of segment 0's counter
 constexpr uint32_t kClaimStride = 32;     // words between segment counters
-constexpr size_t kCounterBytes = ((kClaimBase + kClaimSegments * kClaimStride) * 4 + 255) & ~size_t(255);
+constexpr uint32_t kTileBase = kClaimBase + kClaimSegments * kClaimStride;   // likewise for pixel tiles (claim_tiles)
+constexpr size_t kCounterBytes = ((kTileBase + kClaimSegments * kClaimStride) * 4 + 255) & ~size_t(255);
 
 // Zeroes the claim counters (kClaimSegments threads of the calling block).
 __device__ inline void clear_claims(uint32_t* counters, uint32_t tid) {
     if (tid < kClaimSegments) counters[kClaimBase + tid * kClaimStride] = 0u;
 }
+__device__ inline void clear_tile_claims(uint32_t* counters, uint32_t tid) {
+    if (tid < kClaimSegments) counters[kTileBase + tid * kClaimStride] = 0u;
+}
+// Clears the tile counters with a kernel (a caller may capture the call in a
+// graph, where memset nodes are avoided).  primary.hip
+void launch_clear_tiles(hipStream_t st, uint32_t* counters);
 
 struct TraceLaunch {
     const Node* tlas_nodes;
@@ -322,15 +329,14 @@ struct BatchTlas {
 };
 constexpr uint32_t kMaxBatch = LUZRT_MAX_BATCH;
 constexpr uint32_t kRayGroup = 64;   // pixels per ray group of the grouped ray order (ray_row)
-// Persistent workgroups per CU of the primary-ray kernels (92 VGPRs and 16 KB
-// of LDS stacks per workgroup leave room for five waves per SIMD).  Their waves
-// claim 8x8 pixel tiles from the kCntPrimary counter, `primary_chunk` tiles
-// per claim: about 16 claims per wave, so that the claims of a large batch
-// do not queue on the one counter.
+// Persistent workgroups per CU of the closest-hit kernels (primary rays, shadow
+// maps; up to 96 VGPRs, 16 KB of LDS stacks and 15 KB of staged TLAS per
+// workgroup leave room for five waves per SIMD).
 constexpr uint32_t kPrimaryGroupsPerCu = 5;
-inline uint32_t primary_chunk(uint64_t ntiles, uint32_t groups) {
-    const uint64_t waves = (uint64_t)groups * 4;
-    const uint64_t c = ntiles / (waves * 16);
+// Tiles per claim: about 8 claims per wave, so that the claims of a large
+// launch do not queue on their counters.
+inline uint32_t tile_chunk(uint64_t ntiles, uint32_t groups) {
+    const uint64_t c = ntiles / ((uint64_t)groups * 4 * 8);
     return c < 1 ? 1u : (c > 64 ? 64u : (uint32_t)c);
 }
 luzrt_status launch_trace(luzrt_ctx* ctx, const TraceLaunch& L);

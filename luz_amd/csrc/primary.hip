@@ -15,44 +15,36 @@ namespace {
 
 constexpr int kBlock = 256;
 
-// Clears the tile counter of the call with a kernel (a caller may capture
-// the call in a graph, where memset nodes are avoided).  The error latch
-// kCntError is left set until the host reports it.
-__global__ void k_primary_init(uint32_t* counters) {
-    if (threadIdx.x == 0) counters[kCntPrimary] = 0u;
-}
+// The error latch kCntError is left set until the host reports it.
+__global__ void k_clear_tiles(uint32_t* counters) { clear_tile_claims(counters, threadIdx.x); }
 
-__global__ __launch_bounds__(kBlock) void k_primary(const Node* tlas_nodes, const InstRec* recs,
-                                                    const InstAux* aux, luzrt_camera cam,
-                                                    const luzrt_material* mats, uint32_t nmats,
-                                                    luzrt_gbuffer_out out, uint32_t* spill,
-                                                    uint32_t* counters, uint32_t chunk, bool empty) {
+// Waves claim 8x8 tiles (lane = pixel of a tile): those that drew cheap tiles
+// take more of them.  Bound by the latency of dependent node reads.
+__global__ __launch_bounds__(kBlock, 5) void k_primary(const Node* tlas_nodes, const InstRec* recs,
+                                                       const InstAux* aux, uint32_t tlas_count, uint32_t inst_count,
+                                                       luzrt_camera cam, const luzrt_material* mats, uint32_t nmats,
+                                                       luzrt_gbuffer_out out, uint32_t* spill, uint32_t* counters,
+                                                       uint32_t chunk) {
     __shared__ uint32_t lds[kShort * kBlock];
+    __shared__ float4 stlas[kTlasLdsEntries * 4];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t total = gridDim.x * kBlock;
     Stack st;
     st.init(lds + tid, kBlock, spill + (size_t)blockIdx.x * kBlock + tid, total);
     const uint32_t W = out.width, H = out.height;
     const uint32_t tiles_x = (W + 7) / 8;
-    const uint32_t ntiles = tiles_x * ((H + 7) / 8);
-    // each wave takes the next `chunk` 8x8 tiles (lane = pixel of a tile) until
-    // none is left: waves that drew cheap tiles take more of them
-    for (;;) {
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(&counters[kCntPrimary], chunk);
-        base = __shfl(base, 0);
-        if (base >= ntiles) break;
-        const uint32_t end = min(base + chunk, ntiles);
-        for (uint32_t tile = base; tile < end; ++tile) {
-            uint32_t x = (tile % tiles_x) * 8 + (lane & 7u), y = (tile / tiles_x) * 8 + (lane >> 3);
-            if (x < W && y < H)
-                primary_pixel(tlas_nodes, recs, aux, cam, mats, nmats, out, x, y, st,
-                              &counters[kCntError], empty);
-        }
-    }
+    const TlasView tl = stage_tlas(tlas_nodes, recs, tlas_count, inst_count, stlas);
+    claim_tiles(counters, tiles_x * ((H + 7) / 8), chunk, [&](uint32_t tile) {
+        const uint32_t x = (tile % tiles_x) * 8 + (lane & 7u), y = (tile / tiles_x) * 8 + (lane >> 3);
+        if (x < W && y < H)
+            primary_pixel(tl, aux, cam, mats, nmats, out, x, y, st, &counters[kCntError], inst_count == 0);
+    });
 }
 
 }  // namespace
+
+void launch_clear_tiles(hipStream_t st, uint32_t* counters) { k_clear_tiles<<<1, 64, 0, st>>>(counters); }
+
 }  // namespace luz
 
 using namespace luz;
@@ -84,11 +76,11 @@ extern "C" luzrt_status luzrt_primary_gbuffer(luzrt_ctx* ctx, const luzrt_tlas* 
     if ((s = ensure(ctx, ctx->spill, (size_t)groups * 256 * kSpill * 4)) != LUZRT_OK) return s;
     uint32_t* counters = (uint32_t*)ctx->counters.ptr;
     stage_begin(ctx, kStagePrimary);
-    k_primary_init<<<1, 64, 0, ctx->stream>>>(counters);
+    launch_clear_tiles(ctx->stream, counters);
     const uint32_t ntiles = ((out->width + 7) / 8) * ((out->height + 7) / 8);
-    k_primary<<<groups, 256, 0, ctx->stream>>>(tlas->nodes, tlas->recs, tlas->aux, *cam, dmats, nmats,
-                                              *out, (uint32_t*)ctx->spill.ptr, counters,
-                                              primary_chunk(ntiles, groups), tlas->count == 0);
+    k_primary<<<groups, 256, 0, ctx->stream>>>(tlas->nodes, tlas->recs, tlas->aux, tlas->node_count, tlas->count,
+                                              *cam, dmats, nmats, *out, (uint32_t*)ctx->spill.ptr, counters,
+                                              tile_chunk(ntiles, groups));
     stage_end(ctx, kStagePrimary);
     LUZ_HIP(ctx, hipGetLastError());
     LUZ_HIP(ctx, hipFreeAsync(dmats, ctx->stream));

@@ -48,20 +48,24 @@ __device__ inline V3 cube_dir(uint32_t f, uint32_t i, uint32_t j, uint32_t res) 
     }
 }
 
-// One ray per texel, persistent over the texels of every face.
-__global__ __launch_bounds__(kBlock) void k_shadow_map(const Node* tlas_nodes, const InstRec* recs,
-                                                       const InstAux* aux, luzrt_shadow_map m,
-                                                       uint32_t* spill, uint32_t* error_flag, bool empty) {
+// One ray per texel; waves claim 8x8 texel tiles of the faces (lane = texel of a
+// tile), whose rays stay closer together than those of a strip of a row.
+__global__ __launch_bounds__(kBlock, 5) void k_shadow_map(const Node* tlas_nodes, const InstRec* recs,
+                                                          const InstAux* aux, uint32_t tlas_count,
+                                                          uint32_t inst_count, luzrt_shadow_map m, uint32_t* spill,
+                                                          uint32_t* counters, uint32_t chunk) {
     __shared__ uint32_t lds[kShort * kBlock];
-    const uint32_t tid = threadIdx.x;
-    const uint32_t total = gridDim.x * kBlock;
+    __shared__ float4 stlas[kTlasLdsEntries * 4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
     Stack st;
-    st.init(lds + tid, kBlock, spill + (size_t)blockIdx.x * kBlock + tid, total);
-    const uint32_t res = m.resolution;
+    st.init(lds + tid, kBlock, spill + (size_t)blockIdx.x * kBlock + tid, gridDim.x * kBlock);
+    const uint32_t res = m.resolution, tiles_x = (res + 7) / 8, face_tiles = tiles_x * tiles_x;
     const bool point = m.light_type == LUZRT_LIGHT_POINT;
-    const uint32_t n = (point ? 6u : 1u) * res * res;
-    for (uint32_t k = blockIdx.x * kBlock + tid; k < n; k += total) {
-        const uint32_t f = k / (res * res), r = k % (res * res), i = r % res, j = r / res;
+    const TlasView tl = stage_tlas(tlas_nodes, recs, tlas_count, inst_count, stlas);
+    claim_tiles(counters, (point ? 6u : 1u) * face_tiles, chunk, [&](uint32_t tile) {
+        const uint32_t f = tile / face_tiles, r = tile % face_tiles;
+        const uint32_t i = (r % tiles_x) * 8 + (lane & 7u), j = (r / tiles_x) * 8 + (lane >> 3);
+        if (i >= res || j >= res) return;
         V3 o, d;
         float tmax;
         if (point) {
@@ -80,16 +84,7 @@ __global__ __launch_bounds__(kBlock) void k_shadow_map(const Node* tlas_nodes, c
         Best best;
         best.found = false;
         best.t = tmax;
-        if (!empty) {
-            RayState rs;
-            ray_begin(rs, st, o, d, 0.0f, tmax);
-            for (;;) {
-                int res_step = ray_step<true>(rs, st, tlas_nodes, recs, aux, &best);
-                if (res_step == kStepDone || (res_step == kStepContinue && rs.next == kNone && st.sp == 0))
-                    break;
-                if (res_step == kStepOverflow) { atomicOr(error_flag, 1u); break; }
-            }
-        }
+        if (inst_count) closest_hit(tl, aux, o, d, 0.0f, tmax, st, &counters[kCntError], best);
         float depth = 1.0f;
         if (best.found) {
             if (point) {
@@ -100,8 +95,8 @@ __global__ __launch_bounds__(kBlock) void k_shadow_map(const Node* tlas_nodes, c
                 depth = best.t;
             }
         }
-        m.depth[k] = depth;
-    }
+        m.depth[((size_t)f * res + j) * res + i] = depth;
+    });
 }
 
 __device__ inline int wrapi(int v, int n) { int r = v % n; return r < 0 ? r + n : r; }
@@ -182,14 +177,16 @@ extern "C" luzrt_status luzrt_shadow_map_build(luzrt_ctx* ctx, const luzrt_tlas*
     luzrt_status s = ensure(ctx, ctx->counters, kCounterBytes);
     if (s != LUZRT_OK) return s;
     if ((s = tlas_acquire(ctx, tlas)) != LUZRT_OK) return s;
-    uint32_t groups = (uint32_t)ctx->num_cus * 4;
+    uint32_t groups = (uint32_t)ctx->num_cus * kPrimaryGroupsPerCu;
     if (groups == 0) groups = 1;
     if ((s = ensure(ctx, ctx->spill, (size_t)groups * kBlock * kSpill * 4)) != LUZRT_OK) return s;
     uint32_t* counters = (uint32_t*)ctx->counters.ptr;
+    const uint64_t side = (m->resolution + 7) / 8;
     stage_begin(ctx, kStagePrimary);
-    k_shadow_map<<<groups, kBlock, 0, ctx->stream>>>(tlas->nodes, tlas->recs, tlas->aux, *m,
-                                                    (uint32_t*)ctx->spill.ptr, counters + kCntError,
-                                                    tlas->count == 0);
+    launch_clear_tiles(ctx->stream, counters);
+    k_shadow_map<<<groups, kBlock, 0, ctx->stream>>>(
+        tlas->nodes, tlas->recs, tlas->aux, tlas->node_count, tlas->count, *m, (uint32_t*)ctx->spill.ptr, counters,
+        tile_chunk((m->light_type == LUZRT_LIGHT_POINT ? 6 : 1) * side * side, groups));
     stage_end(ctx, kStagePrimary);
     LUZ_HIP(ctx, hipGetLastError());
     return LUZRT_OK;
