@@ -157,29 +157,34 @@ __global__ __launch_bounds__(kBlock) void k_cull_rows(const uint32_t* counters, 
 // Rays go to the waves in chunks.  A launch of at most kChunkMin rays per
 // resident wave is dealt out, each of them one chunk by its position in the
 // grid (the first waves of all workgroups before their second ones, so that few
-// rays spread over all CUs), as even as rows of 64 allow, and makes no claim: with every chunk claimed, 256-ray
-// chunks left most waves of a 256x256 frame without work, and each of them
-// tried all claim counters in vain (49k atomics on 8 addresses): the 256x256
-// cube frame 161 -> 68 us, 1M incoherent rays 241 -> 183 us.
+// rays spread over all CUs), as even as rows of 64 allow, and makes no claim:
+// with every chunk claimed, 256-ray chunks left most waves of a 256x256 frame
+// without work, and each of them tried all claim counters in vain (49k atomics
+// on 8 addresses): the 256x256 cube frame 161 -> 71 us, 1M incoherent rays
+// 236 -> 190 us.
 // Above that a wave claims its chunks, one device-scope atomic each (the
 // workgroups that wait for a place on the chip would sit on a dealt chunk until
-// the end: the soft-shadow frame lost 4%).  The
-// chunk then follows the launch's ray count, 1/kChunkShare of an even share per
-// wave, kept within kChunkMin .. kChunkMax rays: the rays in flight on the
+// the end: the soft-shadow frame lost 4%).  The chunk then follows the launch's
+// ray count, 1/kChunkShare of an even share per wave, kept within kChunkMin ..
+// 2 kChunkMin rays: the rays in flight on the
 // whole GPU (waves x chunk) then cover few image rows of one light at a time,
 // so the BVH nodes they read stay in L2, while the claims stay below the rate
-// the counters sustain.  Measured on 1080p sphere fields with a single counter
-// (trace ms, 2048 / 512 / 256-ray chunks): 1 shadow ray per light + 1 AO ray
-// 4.40 / 2.11 / 1.82; 1 shadow ray per light + 16 AO rays 3.13 / 2.10 / 2.55;
-// chunks of 64 or 128 lost again to the counter (3.6 and 2.3 ms at 1 + 1).
-constexpr uint32_t kChunkMin = 256, kChunkMax = 512, kChunkShare = 12;
+// the counters sustain (21 ns each on one address).  Half that for a culled
+// launch, whose rows are traced for some of their pixels only: the last chunks
+// of the waves end the launch (culled, kChunkMin 512 / 256 / 128 / 64: 1080p
+// sphere field 939 / 784 / 724 / 699 us, soft shadows 1162 / 980 / 865 / 867 us,
+// 4K terrain 18.9 / 18.2 / 18.2 / 18.9 ms).
+constexpr uint32_t kChunkMin = 256, kChunkShare = 12;
+constexpr uint32_t kSegTries = 2;   // claim counters a wave tries: its workgroup's and the next
 
 __device__ inline bool deal_rays(uint32_t nrays, uint32_t resident) { return nrays <= resident * kChunkMin; }
-// grain: 64 where a wave's rays should be whole rows of neighbouring pixels
-__device__ inline uint32_t claim_chunk(uint32_t nrays, uint32_t nwaves, uint32_t resident, uint32_t grain) {
+// grain: 64 where a wave's rays should be whole rows of neighbouring pixels;
+// cmin: the smallest chunk claimed
+__device__ inline uint32_t claim_chunk(uint32_t nrays, uint32_t nwaves, uint32_t resident, uint32_t grain,
+                                       uint32_t cmin) {
     if (deal_rays(nrays, resident)) return nrays ? ((nrays - 1) / resident / grain + 1u) * grain : grain;
     const uint32_t c = (nrays / (nwaves * kChunkShare)) & ~63u;
-    return c < kChunkMin ? kChunkMin : (c > kChunkMax ? kChunkMax : c);
+    return c < cmin ? cmin : (c > 2 * cmin ? 2 * cmin : c);
 }
 constexpr bool kStageTlas = true;
 
@@ -292,7 +297,8 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
     const uint32_t R = SRC == kGen ? L.ds->r_total : 1u;             // ray slots per pixel
     const uint32_t G = SRC == kGen ? L.ds->ray_group : 0u;           // pixels per ray group
     const uint32_t resident = min(gridDim.x, L.resident) * (kBlock / 64);   // waves on the chip at once
-    const uint32_t chunk = claim_chunk(nrays, total / 64u, resident, SRC == kRays ? 16u : 64u);
+    const uint32_t chunk = claim_chunk(nrays, total / 64u, resident, SRC == kRays ? 16u : 64u,
+                                       CULLED ? kChunkMin / 2 : kChunkMin);
     const uint64_t lt = lane ? (~0ull >> (64 - lane)) : 0ull;
     RayState r;
     uint32_t ray = kNone;
@@ -304,8 +310,9 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
     // rays, so the waves still advance one front through the rays (the BVH
     // nodes in use stay few) while their atomics spread over 8 addresses.  A
     // wave starts on the counter of its workgroup and moves to the next one
-    // when a counter's chunks run past the last ray.
-    const uint32_t seg0 = blockIdx.x % kClaimSegments;
+    // when a counter's chunks run past the last ray, and ends after kSegTries of
+    // them: the counters run out together, and more tries only queue on them.
+    const uint32_t nseg = min(kClaimSegments, gridDim.x), seg0 = blockIdx.x % nseg;
     uint32_t seg = 0;   // counters this wave has found exhausted (wave-uniform)
     if (deal_rays(nrays, resident)) {
         const uint32_t w = (tid >> 6) * (resident / (kBlock / 64)) + blockIdx.x;
@@ -314,21 +321,21 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
             chunk_next = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
             chunk_end = nrays - chunk_next > chunk ? chunk_next + chunk : nrays;
         }
-        seg = kClaimSegments;
+        seg = kSegTries;
     }
     // The next chunk, when the current one is used up (all lanes).
     auto claim = [&]() {
         while (chunk_next >= chunk_end && open) {
-            if (seg == kClaimSegments) {
+            if (seg == kSegTries) {
                 open = false;
                 break;
             }
-            const uint32_t c = (seg0 + seg) % kClaimSegments;
+            const uint32_t c = (seg0 + seg) % nseg;
             uint32_t got = 0;
             if (lane == 0) got = atomicAdd(&L.counters[kClaimBase + c * kClaimStride], 1u);
             // only lane 0 holds the atomic's result: every decision
             // below uses the broadcast copy, so the claim stays uniform
-            const uint64_t base = ((uint64_t)__shfl(got, 0) * kClaimSegments + c) * chunk;
+            const uint64_t base = ((uint64_t)__shfl(got, 0) * nseg + c) * chunk;
             if (base < nrays) {
                 chunk_next = (uint32_t)base;
                 chunk_end = nrays - chunk_next > chunk ? chunk_next + chunk : nrays;
