@@ -25,6 +25,7 @@
 #include <cstring>
 #include <vector>
 
+#include "closest.hpp"
 #include "cull.hpp"
 #include "internal.hpp"
 #include "lightpath.hpp"
@@ -43,15 +44,16 @@ struct BatchSceneDev {
     uint32_t* act_list;
     uint32_t* act_index;
     uint32_t* block_counts;
-    const Node* tlas_nodes;    // null: empty TLAS
+    const Node* tlas_nodes;
     const InstRec* recs;
     const InstAux* aux;
+    const float* slot_box;     // the TLAS slots' padded world boxes
+    uint32_t ninst;            // 0: empty TLAS
     uint32_t nmats;
     uint32_t npix;
     uint32_t ntiles_px;        // tile-ordered pixel slots (compaction)
     uint32_t nblocks;          // compaction blocks
     uint32_t has_camera;
-    uint32_t pad[3];
 };
 
 namespace {
@@ -97,21 +99,14 @@ __global__ void k_batch_init(uint32_t* counters) {
 __global__ __launch_bounds__(kBlock, 5) void k_bprimary(BatchTables T, uint32_t* spill,
                                                         uint32_t* counters, uint32_t chunk) {
     __shared__ uint32_t lds[kShort * kBlock];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t total = gridDim.x * kBlock;
+    const uint32_t tid = threadIdx.x;
     Stack st;
-    st.init(lds + tid, kBlock, spill + (size_t)blockIdx.x * kBlock + tid, total);
+    st.init(lds + tid, kBlock, spill + (size_t)blockIdx.x * kBlock + tid, gridDim.x * kBlock);
     claim_tiles(counters, T.ppx[T.n] >> 6, chunk, [&](uint32_t tile) {
-        const uint32_t gg = tile * 64u;
-        const uint32_t s = find_scene(T.ppx, T.n, gg);
+        const uint32_t s = find_scene(T.ppx, T.n, tile * 64u);
         const BatchSceneDev& S = T.sc[s];
-        const uint32_t W = S.gout.width, H = S.gout.height;
-        const uint32_t tiles_x = (W + 7) / 8;
-        const uint32_t t = (gg - T.ppx[s]) >> 6;
-        const uint32_t x = (t % tiles_x) * 8 + (lane & 7u), y = (t / tiles_x) * 8 + (lane >> 3);
-        if (x < W && y < H)
-            primary_pixel(TlasView{S.tlas_nodes, S.recs, false}, S.aux, S.cam, S.mats, S.nmats, S.gout, x, y, st,
-                          &counters[kCntError], S.tlas_nodes == nullptr);
+        primary_tile(TlasView{S.tlas_nodes, S.recs, S.slot_box, S.ninst, false}, S.aux, S.cam, S.mats, S.nmats, S.gout,
+                     tile - (T.ppx[s] >> 6), st, &counters[kCntError]);
     });
 }
 
@@ -403,6 +398,8 @@ luzrt_status upload_tables(luzrt_ctx* ctx, luzrt_batch* b) {
         b->sc[s].tlas_nodes = bt[s].nodes;
         b->sc[s].recs = bt[s].recs;
         b->sc[s].aux = b->desc[s].tlas->aux;
+        b->sc[s].slot_box = bt[s].slot_box;
+        b->sc[s].ninst = bt[s].ninst;
     }
     LUZ_HIP(ctx, hipMemcpyAsync((void*)b->tables.sc, b->sc.data(), n * sizeof(BatchSceneDev),
                                 hipMemcpyHostToDevice, ctx->stream));

@@ -606,79 +606,4 @@ __device__ inline void primary_texel(const luzrt_camera& cam, V3 d, const Best& 
     }
 }
 
-// Calls tile(i) for tiles 0 .. ntiles - 1 of a persistent launch, `chunk`
-// consecutive ones per claim: a wave's first chunk is the one of its number,
-// the rest are claimed from the counter of its workgroup's segment (one of
-// kClaimSegments, workgroups in turn, so a segment's waves share an XCD), which
-// deals chunks s, s + 8, s + 16, ... of those left.  A device-scope atomic on one
-// address takes about 21 ns whoever asks, and one counter bounded whole
-// launches: 14,400 tiles of 1280x720 and 5,120 waves that find none left took
-// 420 us (297 with eight), the 12 frames of a batch 1910 us (970).  A segment's
-// waves do not look at the other counters: neighbouring chunks belong to
-// different segments, so all eight end together, and the polls would queue again.
-template <typename F>
-__device__ inline void claim_tiles(uint32_t* counters, uint32_t ntiles, uint32_t chunk, F&& tile) {
-    const uint32_t lane = threadIdx.x & 63u, nseg = min(kClaimSegments, gridDim.x);
-    const uint32_t seg = blockIdx.x % nseg, waves = gridDim.x * (blockDim.x >> 6);
-    const uint32_t nchunks = (uint32_t)(((uint64_t)ntiles + chunk - 1) / chunk);
-    uint32_t c = (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
-    while (c < nchunks) {
-        const uint32_t begin = c * chunk, end = min(begin + chunk, ntiles);
-        for (uint32_t i = begin; i < end; ++i) tile(i);
-        if (waves >= nchunks) break;
-        uint32_t got = 0;
-        if (lane == 0) got = atomicAdd(&counters[kTileBase + seg * kClaimStride], 1u);
-        const uint64_t next = (uint64_t)__shfl(got, 0) * nseg + seg + waves;
-        if (next >= nchunks) break;
-        c = (uint32_t)next;
-    }
-}
-
-// The single-scene TLAS of a closest-hit launch, in LDS where it fits: every
-// ray starts there, and its reads no longer compete with BLAS data in L1.
-constexpr uint32_t kTlasLdsEntries = 240;   // TLAS nodes + instance records staged in LDS (15 KB)
-struct TlasView {
-    const Node* nodes;
-    const InstRec* recs;
-    bool lds;
-};
-__device__ inline TlasView stage_tlas(const Node* nodes, const InstRec* recs, uint32_t node_count,
-                                      uint32_t rec_count, float4* lds) {
-    if (node_count + rec_count > kTlasLdsEntries) return TlasView{nodes, recs, false};
-    const float4* gn = reinterpret_cast<const float4*>(nodes);
-    const float4* gr = reinterpret_cast<const float4*>(recs);
-    const uint32_t nn = node_count * 4, nr = rec_count * 4;
-    for (uint32_t i = threadIdx.x; i < nn; i += blockDim.x) lds[i] = gn[i];
-    for (uint32_t i = threadIdx.x; i < nr; i += blockDim.x) lds[nn + i] = gr[i];
-    __syncthreads();
-    return TlasView{reinterpret_cast<const Node*>(lds), reinterpret_cast<const InstRec*>(lds + nn), true};
-}
-
-// The closest hit of one ray, run to completion.
-template <typename STACK>
-__device__ inline void closest_hit(const TlasView& tl, const InstAux* aux, V3 o, V3 d, float tmin, float tmax,
-                                   STACK& st, uint32_t* error_flag, Best& best) {
-    RayState r;
-    ray_begin(r, st, o, d, tmin, tmax);
-    for (;;) {
-        int res = ray_step<true>(r, st, tl.nodes, tl.recs, aux, &best, tl.lds);
-        if (res == kStepDone || (res == kStepContinue && r.next == kNone && st.sp == 0)) break;
-        if (res == kStepOverflow) { atomicOr(error_flag, 1u); st.sp = st.lo = 0; break; }
-    }
-}
-
-// G-buffer texel (x, y) by a closest-hit primary ray.
-template <typename STACK>
-__device__ inline void primary_pixel(const TlasView& tl, const InstAux* aux, const luzrt_camera& cam,
-                                     const luzrt_material* mats, uint32_t nmats, const luzrt_gbuffer_out& out,
-                                     uint32_t x, uint32_t y, STACK& st, uint32_t* error_flag, bool empty) {
-    Best best;
-    best.found = false;
-    best.t = cam.tmax;
-    const V3 d = primary_dir(cam, x, y, out.width, out.height);
-    if (!empty)
-        closest_hit(tl, aux, v3(cam.eye[0], cam.eye[1], cam.eye[2]), d, cam.tmin, cam.tmax, st, error_flag, best);
-    primary_texel(cam, d, best, aux, mats, nmats, out, x, y);
-}
-
 }  // namespace luz

@@ -7,8 +7,8 @@
 // instance's inverse-transpose), and the material of the hit instance.
 // Ties in t are broken by (instance input index, primitive id), so the result
 // does not depend on traversal order.
+#include "closest.hpp"
 #include "internal.hpp"
-#include "lightpath.hpp"
 
 namespace luz {
 namespace {
@@ -20,24 +20,18 @@ __global__ void k_clear_tiles(uint32_t* counters) { clear_tile_claims(counters, 
 
 // Waves claim 8x8 tiles (lane = pixel of a tile): those that drew cheap tiles
 // take more of them.  Bound by the latency of dependent node reads.
-__global__ __launch_bounds__(kBlock, 5) void k_primary(const Node* tlas_nodes, const InstRec* recs,
-                                                       const InstAux* aux, uint32_t tlas_count, uint32_t inst_count,
-                                                       luzrt_camera cam, const luzrt_material* mats, uint32_t nmats,
+__global__ __launch_bounds__(kBlock, 5) void k_primary(TlasView tlas, const InstAux* aux, luzrt_camera cam,
+                                                       const luzrt_material* mats, uint32_t nmats,
                                                        luzrt_gbuffer_out out, uint32_t* spill, uint32_t* counters,
                                                        uint32_t chunk) {
     __shared__ uint32_t lds[kShort * kBlock];
-    __shared__ float4 stlas[kTlasLdsEntries * 4];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t total = gridDim.x * kBlock;
+    __shared__ float4 staged[kStageFloat4];
+    const uint32_t tid = threadIdx.x;
     Stack st;
-    st.init(lds + tid, kBlock, spill + (size_t)blockIdx.x * kBlock + tid, total);
-    const uint32_t W = out.width, H = out.height;
-    const uint32_t tiles_x = (W + 7) / 8;
-    const TlasView tl = stage_tlas(tlas_nodes, recs, tlas_count, inst_count, stlas);
-    claim_tiles(counters, tiles_x * ((H + 7) / 8), chunk, [&](uint32_t tile) {
-        const uint32_t x = (tile % tiles_x) * 8 + (lane & 7u), y = (tile / tiles_x) * 8 + (lane >> 3);
-        if (x < W && y < H)
-            primary_pixel(tl, aux, cam, mats, nmats, out, x, y, st, &counters[kCntError], inst_count == 0);
+    st.init(lds + tid, kBlock, spill + (size_t)blockIdx.x * kBlock + tid, gridDim.x * kBlock);
+    const TlasView tl = stage_tlas(tlas, staged);
+    claim_tiles(counters, ((out.width + 7) / 8) * ((out.height + 7) / 8), chunk, [&](uint32_t tile) {
+        primary_tile(tl, aux, cam, mats, nmats, out, tile, st, &counters[kCntError]);
     });
 }
 
@@ -78,9 +72,9 @@ extern "C" luzrt_status luzrt_primary_gbuffer(luzrt_ctx* ctx, const luzrt_tlas* 
     stage_begin(ctx, kStagePrimary);
     launch_clear_tiles(ctx->stream, counters);
     const uint32_t ntiles = ((out->width + 7) / 8) * ((out->height + 7) / 8);
-    k_primary<<<groups, 256, 0, ctx->stream>>>(tlas->nodes, tlas->recs, tlas->aux, tlas->node_count, tlas->count,
-                                              *cam, dmats, nmats, *out, (uint32_t*)ctx->spill.ptr, counters,
-                                              tile_chunk(ntiles, groups));
+    const TlasView view = {tlas->nodes, tlas->recs, tlas_slot_boxes(tlas), tlas->count, false};
+    k_primary<<<groups, 256, 0, ctx->stream>>>(view, tlas->aux, *cam, dmats, nmats, *out, (uint32_t*)ctx->spill.ptr,
+                                              counters, tile_chunk(ntiles, groups));
     stage_end(ctx, kStagePrimary);
     LUZ_HIP(ctx, hipGetLastError());
     LUZ_HIP(ctx, hipFreeAsync(dmats, ctx->stream));

@@ -17,8 +17,8 @@
 #include <cstring>
 #include <vector>
 
+#include "closest.hpp"
 #include "internal.hpp"
-#include "lightpath.hpp"
 
 namespace luz {
 namespace {
@@ -50,22 +50,21 @@ __device__ inline V3 cube_dir(uint32_t f, uint32_t i, uint32_t j, uint32_t res) 
 
 // One ray per texel; waves claim 8x8 texel tiles of the faces (lane = texel of a
 // tile), whose rays stay closer together than those of a strip of a row.
-__global__ __launch_bounds__(kBlock, 5) void k_shadow_map(const Node* tlas_nodes, const InstRec* recs,
-                                                          const InstAux* aux, uint32_t tlas_count,
-                                                          uint32_t inst_count, luzrt_shadow_map m, uint32_t* spill,
-                                                          uint32_t* counters, uint32_t chunk) {
+__global__ __launch_bounds__(kBlock, 5) void k_shadow_map(TlasView tlas, const InstAux* aux, luzrt_shadow_map m,
+                                                          uint32_t* spill, uint32_t* counters, uint32_t chunk) {
     __shared__ uint32_t lds[kShort * kBlock];
-    __shared__ float4 stlas[kTlasLdsEntries * 4];
+    __shared__ float4 staged[kStageFloat4];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     Stack st;
     st.init(lds + tid, kBlock, spill + (size_t)blockIdx.x * kBlock + tid, gridDim.x * kBlock);
     const uint32_t res = m.resolution, tiles_x = (res + 7) / 8, face_tiles = tiles_x * tiles_x;
     const bool point = m.light_type == LUZRT_LIGHT_POINT;
-    const TlasView tl = stage_tlas(tlas_nodes, recs, tlas_count, inst_count, stlas);
+    const TlasView tl = stage_tlas(tlas, staged);
     claim_tiles(counters, (point ? 6u : 1u) * face_tiles, chunk, [&](uint32_t tile) {
         const uint32_t f = tile / face_tiles, r = tile % face_tiles;
-        const uint32_t i = (r % tiles_x) * 8 + (lane & 7u), j = (r / tiles_x) * 8 + (lane >> 3);
-        if (i >= res || j >= res) return;
+        const uint32_t ti = (r % tiles_x) * 8 + (lane & 7u), tj = (r / tiles_x) * 8 + (lane >> 3);
+        // lanes outside the map repeat its last column or row and write nothing
+        const uint32_t i = min(ti, res - 1), j = min(tj, res - 1);
         V3 o, d;
         float tmax;
         if (point) {
@@ -84,7 +83,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_shadow_map(const Node* tlas_nodes
         Best best;
         best.found = false;
         best.t = tmax;
-        if (inst_count) closest_hit(tl, aux, o, d, 0.0f, tmax, st, &counters[kCntError], best);
+        if (tl.ninst) closest_hits(tl, aux, o, d, 0.0f, tmax, st, &counters[kCntError], best);
         float depth = 1.0f;
         if (best.found) {
             if (point) {
@@ -95,7 +94,7 @@ __global__ __launch_bounds__(kBlock, 5) void k_shadow_map(const Node* tlas_nodes
                 depth = best.t;
             }
         }
-        m.depth[((size_t)f * res + j) * res + i] = depth;
+        if (ti < res && tj < res) m.depth[((size_t)f * res + j) * res + i] = depth;
     });
 }
 
@@ -184,8 +183,9 @@ extern "C" luzrt_status luzrt_shadow_map_build(luzrt_ctx* ctx, const luzrt_tlas*
     const uint64_t side = (m->resolution + 7) / 8;
     stage_begin(ctx, kStagePrimary);
     launch_clear_tiles(ctx->stream, counters);
+    const TlasView view = {tlas->nodes, tlas->recs, tlas_slot_boxes(tlas), tlas->count, false};
     k_shadow_map<<<groups, kBlock, 0, ctx->stream>>>(
-        tlas->nodes, tlas->recs, tlas->aux, tlas->node_count, tlas->count, *m, (uint32_t*)ctx->spill.ptr, counters,
+        view, tlas->aux, *m, (uint32_t*)ctx->spill.ptr, counters,
         tile_chunk((m->light_type == LUZRT_LIGHT_POINT ? 6 : 1) * side * side, groups));
     stage_end(ctx, kStagePrimary);
     LUZ_HIP(ctx, hipGetLastError());

@@ -186,6 +186,7 @@ __device__ inline uint32_t claim_chunk(uint32_t nrays, uint32_t nwaves, uint32_t
     const uint32_t c = (nrays / (nwaves * kChunkShare)) & ~63u;
     return c < cmin ? cmin : (c > 2 * cmin ? 2 * cmin : c);
 }
+constexpr uint32_t kTlasLdsEntries = 240;   // TLAS nodes + instance records staged in LDS
 constexpr bool kStageTlas = true;
 
 // Scene of ray `rid` in a multi-scene launch: the last s < n with base[s] <= rid.

@@ -124,3 +124,43 @@ def test_culled_pixels_change_no_count(ctx, size, lights, wide):
     g.close()
     if wide:
         c.close()
+
+
+@pytest.mark.parametrize("copies", [1, 2, 3])
+@pytest.mark.parametrize("size", [(1, 1), (9, 7), (131, 77)])
+def test_closest_hits_of_tiles_match_oracle(ctx, size, copies):
+    """Primary rays of whole and partial 8x8 tiles on 51, 102 and 153 instances (one
+    and two words of candidates, and the walk from the TLAS root), from the scene's
+    camera and from inside an instance's box along an axis (directions of both signs
+    and zero components in one tile): the G-buffer bit for bit."""
+    W, H = size
+    s = api.HostScene(api.SCENE_SPHERES, 0)
+    g = api.GPUScene(ctx, s)
+    o2w, mesh, mats = s.nodes()
+    n = len(mesh)
+    all_o2w = np.concatenate([o2w] * copies)
+    for c in range(1, copies):
+        all_o2w[c * n:(c + 1) * n, 3::4] += np.float32([7.0, 5.0, 3.0]) * c
+    all_mesh = np.concatenate([mesh] * copies)
+    tlas = ctx.create_tlas(n * copies)
+    tlas.build([api.make_instance(g.blas(int(m)), all_o2w[i], i) for i, m in enumerate(all_mesh)])
+    o = oracle_scene(s)
+    o.set_instances(all_o2w, all_mesh)
+    _, _, cam = s.camera()
+    hit = 0
+    for inside in (False, True):
+        if inside:
+            cam.eye[:] = [float(v) for v in o2w[1, 3::4]]
+            cam.forward[:], cam.right[:], cam.up[:] = (0.0, 0.0, 1.0), (1.0, 0.0, 0.0), (0.0, 1.0, 0.0)
+        gd = api.GBufferDevice(ctx, W, H)
+        print(f"{W}x{H}, {n * copies} instances, inside {inside}", flush=True)
+        ctx.primary_gbuffer(tlas, cam, mats * copies, gd.desc())
+        got, want = gd.download(), o.primary_gbuffer(cam, mats * copies, W, H)
+        for k in ("position", "normal"):
+            np.testing.assert_array_equal(got[k].view(np.uint32), want[k].view(np.uint32), err_msg=k)
+        for k in ("albedo", "material", "emission"):
+            np.testing.assert_array_equal(got[k], want[k], err_msg=k)
+        hit += int((got["normal"] != 0).any())
+    assert hit
+    tlas.destroy()
+    g.close()
