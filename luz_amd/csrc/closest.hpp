@@ -4,8 +4,11 @@
 // The 64 rays of a tile are one beam.  With at most kMaxCullInst instances no
 // TLAS node is visited: the wave tests the slots' padded world boxes against
 // the beam (lane = slot), each lane then its own ray against the few boxes
-// left, and its nearest one is entered first.  Rays that stand before an
-// instance wait for each other as in the culled any-hit traversal.
+// left, and its nearest one is entered first.  A ray that leaves an instance
+// enters its next one at once: where such rays wait for each other, as in the
+// culled any-hit traversal, the longest rays of a tile get longer (shadow maps of
+// 1024 texels: 5.0 ms against 4.6).  Primary rays 1280x720 297 -> 280 us, shadow
+// maps 6.20 -> 4.55 ms against the walk from the TLAS root.
 #pragma once
 #include "cull.hpp"
 
@@ -118,8 +121,6 @@ __device__ inline bool beam_meets_box(const Beam& m, const float box[6], float t
     return !(tn > tf + 1e-5f * (fabsf(tn) + fabsf(tf)));
 }
 
-constexpr uint32_t kClosestEnterLanes = 8;   // lanes that wait for an instance entry at once
-
 // The closest hits of a wave's 64 rays (all lanes active; tmin and tmax the
 // wave's).  Ties in t go by (instance input index, primitive id), so the order
 // in which instances are entered does not show.
@@ -167,9 +168,8 @@ __device__ inline void closest_hits(const TlasView& tl, const InstAux* aux, V3 o
     r.next = first;
     if (waiting) mine[first >> 6] &= ~(1ull << (first & 63u));
     for (;;) {
-        const uint64_t before = __ballot(waiting), inside = __ballot(r.in_blas);
-        if (!(before | inside)) return;
-        if (waiting && ((uint32_t)__popcll(before) >= kClosestEnterLanes || !inside)) {
+        if (__ballot(waiting || r.in_blas) == 0ull) return;
+        if (waiting) {
             enter_instance<false>(r, tl.recs, tl.lds, r.next, best.t);
             waiting = false;
         }
