@@ -88,3 +88,32 @@ def test_compose_matches_oracle(ctx, frames):
     np.testing.assert_allclose(gf, wf, rtol=2e-6, atol=1e-7)
     diff = np.abs(g8.view(np.uint8).astype(int) - w8.view(np.uint8).astype(int))
     assert diff.max() <= 1 and (diff > 0).mean() < 1e-3
+
+
+@pytest.mark.parametrize("size", [(1, 1), (1, 9), (31, 7), (32, 8), (33, 9), (65, 17)])
+def test_taa_bit_exact_around_tiles(ctx, size):
+    """Images of one texel, of whole 32x8 tiles and of one more or less in each
+    direction (borders that wrap within a tile, and across tiles), on noise with
+    background texels and a camera that moves a texel or so."""
+    W, H = size
+    n = W * H
+    rng = np.random.default_rng(W * 100 + H)
+    light, history = (rng.uniform(0, 4, (n, 4)).astype(np.float32) for _ in range(2))
+    position = rng.uniform(-1, 1, (n, 3)).astype(np.float32)
+    position[:, 2] -= 4.0
+    normal = rng.normal(size=(n, 3)).astype(np.float32)
+    normal[rng.uniform(size=n) < 0.3] = 0.0
+    vp = np.float32([1, 0, 0, 0, 0, 1, 0, 0, 0, 0, -1.01, -1, 0, 0, -0.1, 0])   # column-major
+    pvp = vp.copy()
+    pvp[12:14] = (4.0 / W, -3.0 / H)
+    ivp = np.linalg.inv(vp.reshape(4, 4).astype(np.float64)).astype(np.float32).reshape(16)
+    d = api.TaaDesc()
+    bufs = [ctx.to_device(a) for a in (light, history, position, normal)]
+    out = ctx.buffer(n * 16)
+    d.width, d.height = W, H
+    d.light, d.history, d.position, d.normal, d.out = *(b.ptr for b in bufs), out.ptr
+    d.view_proj[:], d.prev_view_proj[:], d.inv_view_proj[:] = vp.tolist(), pvp.tolist(), ivp.tolist()
+    ctx.taa(d)
+    got = out.download(np.float32, (n, 4))
+    want = orc.taa(light, history, position, normal, W, H, vp, pvp, ivp, (0.0, 0.0), (0.0, 0.0), 0)
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
