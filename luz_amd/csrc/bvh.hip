@@ -1510,11 +1510,15 @@ luzrt_status blas_wide_device(luzrt_ctx* ctx, luzrt_blas* const* list, uint32_t 
     for (uint32_t k = 0; k < count; ++k) {
         luzrt_blas* b = list[k];
         const size_t n = b->tri_count ? b->tri_count : 1;
-        auto alloc = [](auto** p, size_t bytes) { return *p ? hipSuccess : hipMalloc((void**)p, bytes); };
-        LUZ_HIP(ctx, alloc(&b->wide, (size_t)b->node_count * sizeof(Node8)));   // wide nodes <= binary internal nodes
-        LUZ_HIP(ctx, alloc(&b->tris8, n * 36));
-        LUZ_HIP(ctx, alloc(&b->prims8, n * 4));
-        LUZ_HIP(ctx, alloc(&b->wide_count_dev, 4));
+        if (b->wide_mem) continue;
+        ArrayBlock block;
+        const size_t wide = block.add((size_t)b->node_count * sizeof(Node8));   // wide nodes <= binary internal nodes
+        const size_t tris8 = block.add(n * 36), prims8 = block.add(n * 4), counted = block.add(4);
+        LUZ_HIP(ctx, hipMalloc(&b->wide_mem, block.bytes));
+        place(&b->wide, b->wide_mem, wide);
+        place(&b->tris8, b->wide_mem, tris8);
+        place(&b->prims8, b->wide_mem, prims8);
+        place(&b->wide_count_dev, b->wide_mem, counted);
     }
     for (uint32_t k = 0; k < count; k += kWideJobs) {
         luzrt_status s = wide_build_some(ctx, list + k, count - k < kWideJobs ? count - k : kWideJobs);

@@ -81,6 +81,23 @@ struct luzrt_ctx {
     int staging_next = 0;
 };
 
+namespace luz {
+// Arrays that live and go together, in one allocation: an allocation and its
+// release cost the host tens of microseconds each, whatever their size (building,
+// querying and replacing a 200k-triangle BLAS with its 8-wide form, thirteen
+// arrays: 1500 -> 1273 us).
+struct ArrayBlock {
+    size_t bytes = 0;
+    size_t add(size_t size) {   // the array's offset
+        const size_t at = bytes;
+        bytes += (size + 255) & ~(size_t)255;
+        return at;
+    }
+};
+template <typename T>
+inline void place(T** array, void* mem, size_t offset) { *array = reinterpret_cast<T*>(static_cast<uint8_t*>(mem) + offset); }
+}  // namespace luz
+
 struct luzrt_blas {
     uint32_t tri_count = 0;
     uint32_t node_count = 0;
@@ -95,6 +112,7 @@ struct luzrt_blas {
     uint32_t* counters = nullptr;   // refit arrival counters (node_count)
     uint32_t* node_end = nullptr;   // per internal node: the far end of its leaf range
     uint32_t* span = nullptr;       // refit hand-over list: [0] = count, then node ids (tri_count)
+    void* mem = nullptr;            // the allocation that holds the arrays above
     int refs = 0;                   // live TLASes built over this BLAS
     // precision form: 8-wide quantised nodes, built on demand from the binary tree
     luz::Node8* wide = nullptr;
@@ -103,6 +121,7 @@ struct luzrt_blas {
     bool wide_counted = false;
     float* tris8 = nullptr;          // 9 floats per wide leaf
     uint32_t* prims8 = nullptr;
+    void* wide_mem = nullptr;        // the allocation that holds them
     bool wide_valid = false;
 };
 

@@ -615,17 +615,23 @@ luzrt_status luzrt_blas_build(luzrt_ctx* ctx, const void* vertices, uint32_t str
     b->vertex_count = vertex_count;
     b->stride = stride;
     const size_t n = b->tri_count ? b->tri_count : 1;
-    auto alloc = [&](void** p, size_t bytes) { return hipMalloc(p, bytes); };
-    hipError_t e = hipSuccess;
-    if (e == hipSuccess) e = alloc((void**)&b->nodes, (size_t)b->node_count * sizeof(Node));
-    if (e == hipSuccess) e = alloc((void**)&b->tris, n * 36);
-    if (e == hipSuccess) e = alloc((void**)&b->nrms, n * 36);
-    if (e == hipSuccess) e = alloc((void**)&b->prims, n * 4);
-    if (e == hipSuccess) e = alloc((void**)&b->slot_idx, n * 12);
-    if (e == hipSuccess) e = alloc((void**)&b->leaf_parent, n * 4);
-    if (e == hipSuccess) e = alloc((void**)&b->counters, (size_t)b->node_count * 4);
-    if (e == hipSuccess) e = alloc((void**)&b->node_end, (size_t)b->node_count * 4);
-    if (e == hipSuccess) e = alloc((void**)&b->span, (n + 1) * 4);
+    ArrayBlock block;
+    const size_t nodes = block.add((size_t)b->node_count * sizeof(Node)), tris = block.add(n * 36),
+                 nrms = block.add(n * 36), prims = block.add(n * 4), slot_idx = block.add(n * 12),
+                 leaf_parent = block.add(n * 4), counters = block.add((size_t)b->node_count * 4),
+                 node_end = block.add((size_t)b->node_count * 4), span = block.add((n + 1) * 4);
+    hipError_t e = hipMalloc(&b->mem, block.bytes);
+    if (e == hipSuccess) {
+        place(&b->nodes, b->mem, nodes);
+        place(&b->tris, b->mem, tris);
+        place(&b->nrms, b->mem, nrms);
+        place(&b->prims, b->mem, prims);
+        place(&b->slot_idx, b->mem, slot_idx);
+        place(&b->leaf_parent, b->mem, leaf_parent);
+        place(&b->counters, b->mem, counters);
+        place(&b->node_end, b->mem, node_end);
+        place(&b->span, b->mem, span);
+    }
     if (e == hipSuccess) e = hipMemset(b->span, 0, 4);   // refit hand-over list starts empty
     if (e != hipSuccess) {
         luzrt_blas_destroy(ctx, b);
@@ -664,10 +670,8 @@ luzrt_status luzrt_blas_destroy(luzrt_ctx* ctx, luzrt_blas* b) {
     if (b->refs > 0)
         return fail(ctx, LUZRT_E_IN_USE, "BLAS is referenced by %d TLAS(es)", b->refs);
     hipStreamSynchronize(ctx->stream);
-    void* ptrs[] = {b->nodes, b->tris, b->nrms, b->prims, b->slot_idx, b->leaf_parent, b->counters,
-                    b->node_end, b->span, b->wide, b->tris8, b->prims8, b->wide_count_dev};
-    for (void* p : ptrs)
-        if (p) hipFree(p);
+    if (b->mem) hipFree(b->mem);
+    if (b->wide_mem) hipFree(b->wide_mem);
     delete b;
     return LUZRT_OK;
 }
