@@ -165,8 +165,8 @@ typedef struct luzrt_timings {
           post_ms;
     uint64_t rays;          /* rays cast by the last visibility/light call */
     uint64_t active_pixels; /* non-background pixels of that call */
-    uint64_t traced_rays;   /* of those, ray ids the traversal ran (64 per live row when the
-                               call culled ray groups, luzrt_set_group_culling; else = rays) */
+    uint64_t traced_rays;   /* of those, rays the traversal ran (those of the pixels left when
+                               the call culled ray groups, luzrt_set_group_culling; else = rays) */
 } luzrt_timings;
 
 /* ------------------------------------------------------------ context */

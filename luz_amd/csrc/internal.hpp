@@ -49,7 +49,9 @@ struct luzrt_ctx {
     luz::DevBuf cull_cand, cull_bits, cull_rows;
     luz::DevBuf wide_work;         // work arrays of 8-wide collapses (bvh.hip)
     bool group_cull = true;        // luzrt_set_group_culling
-    bool last_culled = false;      // the last visibility call traced live rows only
+    bool last_culled = false;      // the last visibility call traced live rows only,
+    uint32_t last_groups = 0, last_kinds = 0;   // of so many ray groups and kinds,
+    uint8_t last_slots[LUZRT_MAX_LIGHTS + 1] = {};   // with so many slots per kind
     // timing
     hipEvent_t ev[luz::kStageCount][2] = {};
     bool ev_used[luz::kStageCount] = {};
@@ -265,7 +267,7 @@ struct DevScene {
 
 // Device counters of one visibility call (ctx->counters).
 enum Counter { kCntFetch = 0, kCntActive = 1, kCntError = 2, kCntRays = 3, kCntBuildError = 4,
-               kCntLive = 6, kCntCount = 8 };
+               kCntTraced = 5, kCntLive = 6, kCntCount = 8 };
 // A traversal launch claims its rays in chunks from kClaimSegments counters,
 // counter c owning chunks c, c + 8, c + 16, ..., each on a 128-byte line of
 // its own after the Counter array: one counter took every wave's
@@ -359,6 +361,8 @@ inline uint32_t tile_chunk(uint64_t ntiles, uint32_t groups) {
     return c < 1 ? 1u : (c > 64 ? 64u : (uint32_t)c);
 }
 luzrt_status launch_trace(luzrt_ctx* ctx, const TraceLaunch& L);
+// Rays the last visibility call traced, if it culled (waits for the count).
+luzrt_status count_traced(luzrt_ctx* ctx, uint32_t active_pixels, uint64_t* traced);
 // Exclusive scan in place of n live-row counts (16-byte aligned), the total to
 // counters[kCntLive] (one workgroup, trace.hip).
 void launch_cull_scan(hipStream_t st, uint32_t* counts, uint32_t n, uint32_t* counters);

@@ -467,7 +467,11 @@ luzrt_status luzrt_get_timings(luzrt_ctx* ctx, luzrt_timings* out) {
         LUZ_HIP(ctx, hipMemcpy(c, ctx->counters.ptr, sizeof(c), hipMemcpyDeviceToHost));
         out->rays = c[kCntRays];
         out->active_pixels = c[kCntActive];
-        out->traced_rays = ctx->last_culled ? (uint64_t)c[kCntLive] * 64u : out->rays;
+        out->traced_rays = out->rays;
+        if (ctx->last_culled) {
+            luzrt_status s = count_traced(ctx, c[kCntActive], &out->traced_rays);
+            if (s != LUZRT_OK) return s;
+        }
         if (c[kCntError]) return check_trace_latch(ctx);
         if (c[kCntBuildError])
             return fail(ctx, LUZRT_E_INVALID_ARG, "acceleration-structure build error flag %u",

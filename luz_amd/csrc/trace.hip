@@ -19,6 +19,7 @@
 //               per light and unoccluded AO samples, written as u8 planes;
 //               background pixels get zero counts.
 #include <algorithm>
+#include <cstring>
 
 #include "internal.hpp"
 #include "lightpath.hpp"
@@ -524,6 +525,20 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
     }
 }
 
+// The rays a culled call traced: the pixels of each kind times its slots, a
+// thread per group and kind.
+struct KindSlots {
+    uint8_t n[LUZRT_MAX_LIGHTS + 1];
+};
+__global__ __launch_bounds__(kBlock) void k_count_traced(const uint64_t* pix, uint32_t groups, uint32_t kinds,
+                                                         KindSlots slots, uint32_t* total) {
+    uint32_t sum = 0;
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < groups * kinds; i += gridDim.x * kBlock)
+        sum += (uint32_t)__popcll(pix[i]) * slots.n[i % kinds];
+    for (uint32_t off = 32; off; off >>= 1) sum += __shfl_xor(sum, off);
+    if ((threadIdx.x & 63u) == 0 && sum) atomicAdd(total, sum);
+}
+
 // Thread q zeroes the counts of pixel q if it is background and resolves
 // active pixel q (in active order, so a wave's hit reads are contiguous).
 __global__ __launch_bounds__(kBlock) void k_resolve(const DevScene* ds, const uint32_t* act_index,
@@ -543,6 +558,23 @@ inline uint32_t cdiv(uint64_t a, uint32_t b) { return (uint32_t)((a + b - 1) / b
 
 void launch_cull_scan(hipStream_t st, uint32_t* counts, uint32_t n, uint32_t* counters) {
     k_cull_scan<<<1, 1024, 0, st>>>(counts, n, counters);
+}
+
+luzrt_status count_traced(luzrt_ctx* ctx, uint32_t active_pixels, uint64_t* traced) {
+    uint32_t* total = (uint32_t*)ctx->counters.ptr + kCntTraced;
+    const uint32_t groups = std::min(ctx->last_groups, cdiv(active_pixels, kCullGroup));
+    KindSlots slots;
+    std::memcpy(slots.n, ctx->last_slots, sizeof(slots.n));
+    uint32_t n = 0;
+    LUZ_HIP(ctx, hipMemsetAsync(total, 0, 4, ctx->stream));
+    k_count_traced<<<256, kBlock, 0, ctx->stream>>>(
+        (const uint64_t*)ctx->cull_cand.ptr + (size_t)ctx->last_groups * ctx->last_kinds * kCandWords, groups,
+        ctx->last_kinds, slots, total);
+    LUZ_HIP(ctx, hipGetLastError());
+    LUZ_HIP(ctx, hipMemcpyAsync(&n, total, 4, hipMemcpyDeviceToHost, ctx->stream));
+    LUZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    *traced = n;
+    return LUZRT_OK;
 }
 
 luzrt_status launch_trace(luzrt_ctx* ctx, const TraceLaunch& L) {
@@ -656,6 +688,13 @@ luzrt_status visibility_core(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
                       (uint64_t)ngroups * kCullGroup * ds.r_total <= 0xFFFFFFFFull;
     ctx->last_culled = cull;
     const uint32_t kinds = (uint32_t)scene->num_lights + 1;
+    ctx->last_groups = ngroups;
+    ctx->last_kinds = kinds;
+    for (uint32_t k = 0; cull && k < kinds; ++k) {   // as the device's slot_light deals the slots
+        const uint32_t begin = k + 1 < kinds ? ds.slot_base[k] : ds.r_shadow;
+        const uint32_t end = k + 2 < kinds ? ds.slot_base[k + 1] : (k + 1 < kinds ? ds.r_shadow : ds.r_total);
+        ctx->last_slots[k] = (uint8_t)(end - begin);
+    }
     if (cull) {
         // candidate masks, then pixel masks
         if ((s = ensure(ctx, ctx->cull_cand, (size_t)ngroups * kinds * kKindWords * 8)) != LUZRT_OK) return s;
