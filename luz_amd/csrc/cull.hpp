@@ -25,7 +25,7 @@
 // its rays of that kind culled: on the 1080p sphere field seven of ten rays of
 // the rows that the group bounds leave meet no box, and generating them to find
 // that out was most of the traversal's work and left its waves two thirds idle
-// (1080p sphere field: k_cull 67 -> 170 us, traversal 745 -> 603 us; soft shadows
+// (1080p sphere field: k_cull 67 -> 170 us, traversal 600 -> 364 us; soft shadows
 // at 1277x713 1747 -> 1133 us for the call; batch of 12 frames 5.44 -> 4.55 ms;
 // the instance entries that wait for each other, trace.hip, are part of these).
 // k_cull writes, per group, the candidate mask of each kind (bit s: TLAS slot
