@@ -415,7 +415,7 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
                                 gen_ray_of(dsc, pixel_frame(bt.position, bt.normal, bt.width, dsc->s,
                                                             bt.act_list[a]),
                                            slot, l, o, d, tmin, tmax);
-                                ray_begin(r, st, o, d, tmin, tmax);
+                                ray_begin<WIDE>(r, st, o, d, tmin, tmax);
                                 if (!enter_candidates(r, st, cw, bt.slot_box)) {
                                     L.hits[ray] = 0;
                                     ray = kNone;
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
                                 gen_ray(bt.ds, pixel_frame(bt.position, bt.normal, bt.width, bt.ds->s,
                                                            bt.act_list[a]),
                                         slot, o, d, tmin, tmax);
-                                ray_begin(r, st, o, d, tmin, tmax);
+                                ray_begin<WIDE>(r, st, o, d, tmin, tmax);
                             }
                         } else {
                             if (SRC == kGen) {
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
                                     gen_ray_of(L.ds, pixel_from_record(r0, r1), slot,
                                                slot < rs ? (cull ? (int)s_kind[slot] : slot_light(L.ds, slot)) : 0, o,
                                                d, tmin, tmax);
-                                    ray_begin(r, st, o, d, tmin, tmax);
+                                    ray_begin<WIDE>(r, st, o, d, tmin, tmax);
                                     if (cull && !enter_candidates(r, st, cw, L.slot_box)) {
                                         L.hits[ray] = 0;
                                         ray = kNone;
@@ -473,7 +473,7 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
                             } else {
                                 float4 o = L.ray_o[(size_t)rid * L.ray_stride];
                                 float4 d = L.ray_d[(size_t)rid * L.ray_stride];
-                                ray_begin(r, st, v3(o.x, o.y, o.z), v3(d.x, d.y, d.z), o.w, d.w);
+                                ray_begin<WIDE>(r, st, v3(o.x, o.y, o.z), v3(d.x, d.y, d.z), o.w, d.w);
                             }
                         }
                     }

@@ -95,11 +95,16 @@ constexpr uint32_t kMaxSteps = 1u << 24;
 
 enum StepResult { kStepContinue = 0, kStepHit = 1, kStepDone = 2, kStepOverflow = 3 };
 
-template <typename STACK>
+// WIDE: the range of the object-space slab rays is 2^-24 of the ray's (wide_visit).
+template <bool WIDE = false, typename STACK>
 __device__ inline void ray_begin(RayState& r, STACK& st, V3 o, V3 d, float tmin, float tmax) {
     r.wd = d; r.tmin = tmin; r.tmax = tmax;
     r.wbr = box_setup(o, d, tmin, tmax);
     r.br = r.wbr;
+    if (WIDE) {
+        r.br.tlo *= 0x1p-24f;
+        r.br.thi *= 0x1p-24f;
+    }
     r.next = 0;
     r.steps = 0;
     r.in_blas = false;
@@ -190,7 +195,8 @@ __device__ inline int wide_visit(RayState& r, STACK& st) {
     const uint32_t nx[2] = {gx ? qb.z : qa.x, gx ? qb.w : qa.y}, fx[2] = {gx ? qa.x : qb.z, gx ? qa.y : qb.w};
     const uint32_t ny[2] = {gy ? qc.x : qa.z, gy ? qc.y : qa.w}, fy[2] = {gy ? qa.z : qc.x, gy ? qa.w : qc.y};
     const uint32_t nz[2] = {gz ? qc.z : qb.x, gz ? qc.w : qb.y}, fz[2] = {gz ? qb.x : qc.z, gz ? qb.y : qc.w};
-    // A child plane o + q x 2^e is met at t = (o + q x 2^e - ro) x inv =
+    // Distances here are 2^-24 of the ray's (the slab ray is scaled):
+    // a child plane o + q x 2^e is met at (o + q x 2^e - ro) x inv =
     // (q x 2^-24) x S + O, with S = 2^(e + 24) x inv (exact: a power-of-two
     // scaling, and the FP16 subnormal holds q x 2^-24 exactly) and
     // O = (o - ro) x inv per node and axis: one fused multiply-add per plane.
@@ -198,7 +204,9 @@ __device__ inline int wide_visit(RayState& r, STACK& st) {
     // ulps of the terms, covered as before by the far bound's widening and
     // the child boxes' outward rounding; an infinite reciprocal (a direction
     // component of zero) gives infinite or NaN distances that the max/min
-    // ignore or that keep the box, as before.
+    // ignore or that keep the box, as before.  (On an unscaled ray S overflows
+    // for reciprocals from 2^(104 - e), where a near plane at infinity loses
+    // boxes that hold the origin.)
     const float Sx = __builtin_ldexpf(r.br.inv.x, ex + 24), Sy = __builtin_ldexpf(r.br.inv.y, ey + 24),
                 Sz = __builtin_ldexpf(r.br.inv.z, ez + 24);
     const float Ox = (ox - r.br.o.x) * r.br.inv.x, Oy = (oy - r.br.o.y) * r.br.inv.y,
@@ -262,11 +270,17 @@ __device__ inline bool enter_instance(RayState& r, const InstRec* recs, bool rec
     float w[12] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w, w2.x, w2.y, w2.z, w2.w};
     V3 oo = xform_point(w, r.wbr.o);
     V3 od = xform_vec(w, r.wd);
-    r.br = box_setup(oo, od, r.tmin, thi);
+    const BoxRay obj = box_setup(oo, od, r.tmin, thi);
     r.tr = tri_setup(od);
     // a NaN tmin on a NaN ray meets no box (every bound is NaN); wide_visit
     // compares by the sign of a difference, which a NaN does not decide
     if (WIDE && r.br.tlo != r.br.tlo && (oo.x != oo.x || od.x != od.x)) return false;
+    if (WIDE) {   // any-hit: the range is the ray's; an infinite reciprocal stays infinite
+        r.br.o = obj.o;
+        r.br.inv = v3(obj.inv.x * 0x1p-24f, obj.inv.y * 0x1p-24f, obj.inv.z * 0x1p-24f);
+    } else {
+        r.br = obj;
+    }
     r.bnodes = reinterpret_cast<const Node*>(((uint64_t)pp.y << 32) | pp.x);
     r.btris = reinterpret_cast<const float*>(((uint64_t)pp.w << 32) | pp.z);
     r.inst_slot = slot;

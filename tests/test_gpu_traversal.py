@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 from luz_amd import api
-from tests.helpers import oracle_scene, random_rays
+from oracle import oracle as orc
+from tests.helpers import oracle_scene, random_rays, scaled_instances
 
 pytestmark = pytest.mark.gpu
 
@@ -164,3 +165,61 @@ def test_closest_hits_of_tiles_match_oracle(ctx, size, copies):
     assert hit
     tlas.destroy()
     g.close()
+
+
+def _unrotated(c, size=1.0):
+    """Five sphere meshes (vertices times `size`) in 40 instances of several scales
+    without rotation, so that a ray's zero and tiny components reach the object
+    space; returns GPU scene, TLAS and oracle scene."""
+    s = api.HostScene(api.SCENE_SPHERES, 0)
+    rng = np.random.default_rng(17)
+    xyz = rng.uniform(-6, 6, (40, 3)) * size
+    o2w = scaled_instances(xyz, rng.choice([0.5, 1.0, 2.0], 40))
+    mesh = np.arange(40, dtype=np.uint32) % 5
+    o = orc.OracleScene()
+    blas = []
+    for m in range(5):
+        v, idx = s.mesh(m)
+        v = v.copy()
+        v[:, :3] *= np.float32(size)
+        o.add_mesh(v, idx)
+        blas.append(c.create_blas(c.to_device(v), 48, len(v), c.to_device(idx), len(idx)))
+    o.set_instances(o2w, mesh)
+    tlas = c.create_tlas(40)
+    tlas.build([api.make_instance(blas[m], o2w[i], i) for i, m in enumerate(mesh)])
+    return blas, tlas, o
+
+
+def _both_trees(ctx, rays, size=1.0):
+    wide = api.Context(0)
+    wide.set_precision(api.PRECISION_WIDE)
+    got = []
+    for c in (ctx, wide):
+        blas, tlas, o = _unrotated(c, size)
+        got.append(_hits(c, tlas, c.to_device(rays), len(rays)))
+        tlas.destroy()
+        for b in blas:
+            b.destroy()
+    wide.close()
+    return got[0], got[1], o
+
+
+@pytest.mark.parametrize("size, smallest", [(1.0, -40), (1000.0, -36)])
+def test_tiny_direction_components_lose_no_hit(ctx, size, smallest):
+    """Direction components from 1e-40 to 1e-18 of both signs on one or two axes, origins
+    inside the boxes: the reciprocal of such a component is finite while a node's plane
+    distances come near the largest float."""
+    rng = np.random.default_rng(5)
+    n = 60000
+    rays = random_rays(rng, n, (0, 0, 0), 7.0 * size, 20.0 * size)
+    tiny = np.float32(10.0) ** rng.uniform(smallest, -18, (n, 2)) * rng.choice([-1.0, 1.0], (n, 2))
+    k = np.arange(n)
+    rays[k, 4 + k % 3] = tiny[:, 0].astype(np.float32)
+    two = k % 4 == 0
+    rays[two, 4 + (k[two] + 1) % 3] = tiny[two, 1].astype(np.float32)
+    plain, wide, o = _both_trees(ctx, rays, size)
+    want, _ = o.any_hit(rays)
+    print(f"size {size}: {int(want.sum())} of {n} rays hit, 8-wide {int(wide.sum())}", flush=True)
+    assert 0 < want.sum() < n
+    np.testing.assert_array_equal(plain, want)
+    np.testing.assert_array_equal(wide, want)
