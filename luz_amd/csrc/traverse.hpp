@@ -217,8 +217,8 @@ __device__ inline int wide_visit(RayState& r, STACK& st) {
                                   __builtin_fmaf(bnz, Sz, Oz));
         const float tf = box_far(r.br, __builtin_fmaf(bfx, Sx, Ox), __builtin_fmaf(bfy, Sy, Oy),
                                  __builtin_fmaf(bfz, Sz, Oz));
-        // the sign bit of tf - tn, shifted in (no NaN: tlo and thi are numbers, or
-        // some plane is where tmin is NaN: see the instance entry in ray_step)
+        // the sign bit of tf - tn, shifted in (no NaN: the range ends are numbers,
+        // or the planes of some axis are: see enter_instance)
         miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(tf - tn), 31);
     };
 #pragma unroll
@@ -272,9 +272,13 @@ __device__ inline bool enter_instance(RayState& r, const InstRec* recs, bool rec
     V3 od = xform_vec(w, r.wd);
     const BoxRay obj = box_setup(oo, od, r.tmin, thi);
     r.tr = tri_setup(od);
-    // a NaN tmin on a NaN ray meets no box (every bound is NaN); wide_visit
-    // compares by the sign of a difference, which a NaN does not decide
-    if (WIDE && r.br.tlo != r.br.tlo && (oo.x != oo.x || od.x != od.x)) return false;
+    // With a NaN range end, a ray that has no axis of plane distances that are
+    // numbers meets no box (its bounds are NaN); wide_visit compares by the sign
+    // of a difference, which a NaN does not decide.
+    auto numbers = [](float o, float inv) { return fabsf(inv) < INFINITY && o * inv == o * inv; };
+    if (WIDE && __builtin_isunordered(r.br.tlo, r.br.thi) && !numbers(oo.x, obj.inv.x) &&
+        !numbers(oo.y, obj.inv.y) && !numbers(oo.z, obj.inv.z))
+        return false;
     if (WIDE) {   // any-hit: the range is the ray's; an infinite reciprocal stays infinite
         r.br.o = obj.o;
         r.br.inv = v3(obj.inv.x * 0x1p-24f, obj.inv.y * 0x1p-24f, obj.inv.z * 0x1p-24f);

@@ -223,3 +223,23 @@ def test_tiny_direction_components_lose_no_hit(ctx, size, smallest):
     assert 0 < want.sum() < n
     np.testing.assert_array_equal(plain, want)
     np.testing.assert_array_equal(wide, want)
+
+
+def test_ranges_that_are_no_numbers_meet_the_same_triangles_in_both_trees(ctx):
+    """NaN and infinite range ends, on ordinary rays and on rays with a NaN component
+    (whose box tests compare NaN with NaN: a miss)."""
+    rng = np.random.default_rng(23)
+    n = 40000
+    rays = random_rays(rng, n, (0, 0, 0), 7.0, 20.0)
+    ends = np.array([np.nan, np.inf, -np.inf], np.float32)
+    k = np.arange(n)
+    rays[k, np.where(k % 2, 3, 7)] = ends[rng.integers(0, 3, n)]
+    both = k % 5 == 0
+    rays[both, 3], rays[both, 7] = ends[rng.integers(0, 3, both.sum())], ends[rng.integers(0, 3, both.sum())]
+    nan = k % 3 == 0
+    rays[nan, np.array([0, 1, 2, 4, 5, 6])[rng.integers(0, 6, nan.sum())]] = np.nan
+    rays[nan & (k % 2 == 0), 4] *= -1       # NaNs of both signs
+    plain, wide, _ = _both_trees(ctx, rays)
+    print(f"{int(plain.sum())} of {n} rays hit, 8-wide {int(wide.sum())}", flush=True)
+    assert 0 < plain.sum() < n
+    np.testing.assert_array_equal(wide, plain)
