@@ -669,6 +669,7 @@ luzrt_status visibility_core(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
     const DevScene* dsd = (const DevScene*)ctx->scene.ptr;
     hipStream_t st = ctx->stream;
 
+    ctx->last_culled = false;   // from here the counters are this call's
     stage_begin(ctx, kStageCompact);
     uint32_t ntiles_px = (uint32_t)ntiles_px_sz;
     uint32_t nblocks = cdiv(ntiles_px, kBlock);
@@ -691,15 +692,7 @@ luzrt_status visibility_core(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
     const bool cull = ctx->group_cull && ds.r_total > 0 && ds.r_total <= kMaxCullSlots &&
                       tlas->count > 0 && tlas->count <= kMaxCullInst && ds.ray_group == kCullGroup &&
                       (uint64_t)ngroups * kCullGroup * ds.r_total <= 0xFFFFFFFFull;
-    ctx->last_culled = cull;
     const uint32_t kinds = (uint32_t)scene->num_lights + 1;
-    ctx->last_groups = ngroups;
-    ctx->last_kinds = kinds;
-    for (uint32_t k = 0; cull && k < kinds; ++k) {   // as the device's slot_light deals the slots
-        const uint32_t begin = k + 1 < kinds ? ds.slot_base[k] : ds.r_shadow;
-        const uint32_t end = k + 2 < kinds ? ds.slot_base[k + 1] : (k + 1 < kinds ? ds.r_shadow : ds.r_total);
-        ctx->last_slots[k] = (uint8_t)(end - begin);
-    }
     if (cull) {
         // candidate masks, then pixel masks
         if ((s = ensure(ctx, ctx->cull_cand, (size_t)ngroups * kinds * kKindWords * 8)) != LUZRT_OK) return s;
@@ -720,6 +713,15 @@ luzrt_status visibility_core(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
                                                 (uint32_t*)ctx->cull_rows.ptr, (uint8_t*)ctx->hits.ptr);
         stage_end(ctx, kStageRaygen);
         LUZ_HIP(ctx, hipGetLastError());
+        // the pixel masks are there to be counted (count_traced)
+        ctx->last_groups = ngroups;
+        ctx->last_kinds = kinds;
+        for (uint32_t k = 0; k < kinds; ++k) {   // as the device's slot_light deals the slots
+            const uint32_t begin = k + 1 < kinds ? ds.slot_base[k] : ds.r_shadow;
+            const uint32_t end = k + 2 < kinds ? ds.slot_base[k + 1] : (k + 1 < kinds ? ds.r_shadow : ds.r_total);
+            ctx->last_slots[k] = (uint8_t)(end - begin);
+        }
+        ctx->last_culled = true;
     }
 
     stage_begin(ctx, kStageTrace);
@@ -849,6 +851,7 @@ extern "C" luzrt_status luzrt_trace_rays(luzrt_ctx* ctx, const luzrt_tlas* tlas,
     if (s != LUZRT_OK) return s;
     if ((s = tlas_acquire(ctx, tlas)) != LUZRT_OK) return s;
     uint32_t* counters = (uint32_t*)ctx->counters.ptr;
+    ctx->last_culled = false;
     stage_begin(ctx, kStageTrace);
     k_vis_init<<<1, 64, 0, ctx->stream>>>(counters, count);
     if (tlas->count == 0) {

@@ -243,3 +243,25 @@ def test_ranges_that_are_no_numbers_meet_the_same_triangles_in_both_trees(ctx):
     print(f"{int(plain.sum())} of {n} rays hit, 8-wide {int(wide.sum())}", flush=True)
     assert 0 < plain.sum() < n
     np.testing.assert_array_equal(wide, plain)
+
+
+def test_timings_after_ray_queries_count_their_rays(ctx):
+    """A ray query or an unculled call after a culled one reports its own traced rays."""
+    W, H = 160, 90
+    s = api.HostScene(api.SCENE_SPHERES, 0)
+    g = api.GPUScene(ctx, s)
+    _, _, cam = s.camera()
+    _, _, mats = s.nodes()
+    gd = api.GBufferDevice(ctx, W, H)
+    ctx.primary_gbuffer(g.tlas, cam, mats, gd.desc())
+    sb = s.pack()
+    sh, ao = ctx.buffer(sb.num_lights * W * H), ctx.buffer(W * H)
+    rays = random_rays(np.random.default_rng(1), 777, (0, 0.5, 0), 2.0)
+    for _ in range(2):
+        ctx.trace_visibility(g.tlas, gd.desc(), sb, sh, ao)
+        t = ctx.timings()
+        assert 0 < t.traced_rays < t.rays      # culled
+        _hits(ctx, g.tlas, ctx.to_device(rays), len(rays))
+        t = ctx.timings()
+        assert (t.rays, t.traced_rays) == (777, 777)
+    g.close()
