@@ -14,8 +14,8 @@
 //   length, so a TLAS slot whose padded world box, widened by that distance,
 //   misses the segment cannot hold a hit of any ray of the group and light;
 //   AO rays run from origins within 0.05 |N| of A for at most
-//   ao_max x max(|N|, |N|^2) (light.frag:86-97,229-231), so a slot box that
-//   misses A widened by that reach cannot hold one of their hits.
+//   max(|ao_min|, |ao_max|) x max(|N|, |N|^2) (light.frag:86-97,229-231), so a
+//   slot box that misses A widened by that reach cannot hold one of their hits.
 // Each candidate is then tested against the group's pixels one by one (lane =
 // pixel): the segment from the pixel's own shadow origin to its end point
 // against the box widened by the light's radius, or the distance of the box
@@ -315,7 +315,7 @@ __device__ inline GroupRows cull_group(const PixelFrame& f, uint64_t pixels, con
         }
     }
     {
-        const float amax = fmax_(ao_max, 0.0f);
+        const float amax = fmax_(fabsf(ao_min), fabsf(ao_max));   // (a range may lie behind the origin)
         const float reach = amax * fmax_(nmax, nmax * nmax) * 1.00001f + 0.05f * nmax;
         const float w = reach + 1e-3f + 2e-5f * (mag + reach);
         bool meet = own, meet1 = own1;
@@ -326,7 +326,7 @@ __device__ inline GroupRows cull_group(const PixelFrame& f, uint64_t pixels, con
         uint64_t m = __ballot(meet), m1 = __ballot(meet1), reached = 0;
         if (R == r_shadow) {
             m = m1 = 0;   // no AO rays
-        } else if (any_bad || !isfinite(ao_max) || !isfinite(w)) {
+        } else if (any_bad || !isfinite(ao_min) || !isfinite(ao_max) || !isfinite(w)) {
             m = all;
             m1 = all1;
             reached = pixels;

@@ -265,3 +265,27 @@ def test_timings_after_ray_queries_count_their_rays(ctx):
         t = ctx.timings()
         assert (t.rays, t.traced_rays) == (777, 777)
     g.close()
+
+
+@pytest.mark.parametrize("ao", [(-3.0, 0.5), (-0.5, 0.25), (-2.0, -0.5), (-4.0, 4.0)])
+def test_culling_keeps_ao_ranges_behind_the_surface(ctx, ao):
+    """AO ranges that start behind the origin, further than they reach ahead of it: the
+    culled counts equal the unculled ones and the oracle's."""
+    W, H = 96, 64
+    s = api.HostScene(api.SCENE_SPHERES, 0)
+    g = api.GPUScene(ctx, s)
+    _, _, cam = s.camera()
+    _, _, mats = s.nodes()
+    gd = api.GBufferDevice(ctx, W, H)
+    ctx.primary_gbuffer(g.tlas, cam, mats, gd.desc())
+    sb = s.pack()
+    sb.ao_min, sb.ao_max, sb.ao_num_samples = *ao, 8
+    want_sh, want_ao, _ = oracle_scene(s).trace_visibility(gd.download(), W, H, sb)
+    nl = sb.num_lights
+    for cull in (False, True):
+        ctx.set_group_culling(cull)
+        dsh, dao = ctx.buffer(nl * W * H), ctx.buffer(W * H)
+        ctx.trace_visibility(g.tlas, gd.desc(), sb, dsh, dao)
+        np.testing.assert_array_equal(dao.download(np.uint8, W * H), want_ao, err_msg=f"culled {cull}")
+        np.testing.assert_array_equal(dsh.download(np.uint8, (nl, W * H)), want_sh)
+    g.close()
