@@ -188,6 +188,18 @@ __device__ inline GroupRows cull_group(const PixelFrame& f, uint64_t pixels, con
             bhi1[k] = slot_box[(lane + 64) * 6 + 3 + k];
         }
     }
+    // a box that is not finite (a vertex near the largest float) bounds nothing:
+    // the per-pixel tests would take its NaN centre for out of reach
+    auto bound = [](float (&lo)[3], float (&hi)[3]) {
+        bool finite = true;
+        for (int k = 0; k < 3; ++k) finite = finite && isfinite(lo[k]) && isfinite(hi[k]);
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = finite ? lo[k] : -1e38f;
+            hi[k] = finite ? hi[k] : 1e38f;
+        }
+    };
+    bound(blo, bhi);
+    bound(blo1, bhi1);
     // slots whose box holds every shadow origin of the group: all pixels reach them
     bool holds = own, holds1 = own1;
     for (int k = 0; k < 3; ++k) {
@@ -199,7 +211,7 @@ __device__ inline GroupRows cull_group(const PixelFrame& f, uint64_t pixels, con
         auto put = [&](uint32_t sl, const float lo[3], const float hi[3]) {
             float c[3], h[3];
             for (int k = 0; k < 3; ++k) {
-                c[k] = 0.5f * (lo[k] + hi[k]);
+                c[k] = 0.5f * lo[k] + 0.5f * hi[k];
                 h[k] = fmax_(hi[k] - c[k], c[k] - lo[k]);
             }
             wave_boxes[sl].c = make_float4(c[0], c[1], c[2], 0.0f);

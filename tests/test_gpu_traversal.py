@@ -289,3 +289,37 @@ def test_culling_keeps_ao_ranges_behind_the_surface(ctx, ao):
         np.testing.assert_array_equal(dao.download(np.uint8, W * H), want_ao, err_msg=f"culled {cull}")
         np.testing.assert_array_equal(dsh.download(np.uint8, (nl, W * H)), want_sh)
     g.close()
+
+
+@pytest.mark.parametrize("far", [10.0, 1e18, 1e37, np.finfo(np.float32).max])
+def test_culling_keeps_an_instance_with_a_far_vertex(ctx, far):
+    """A box that reaches far, up to past the largest float (its padded bound is
+    infinite): rays still meet the triangle beside the pixels."""
+    W = H = 24
+    verts = np.zeros((6, 12), np.float32)
+    verts[:3, :3] = [(-1, 0.5, -1), (1, 0.5, -1), (0, 0.5, 1)]            # a roof over the pixels
+    verts[3:, :3] = [(5, 5, 5), (6, far, 5), (5, 5, 6)]
+    idx = np.arange(6, dtype=np.uint32)
+    blas = ctx.create_blas(ctx.to_device(verts), 48, 6, ctx.to_device(idx), 6)
+    tlas = ctx.create_tlas(1)
+    tlas.build([api.make_instance(blas, np.eye(3, 4, dtype=np.float32).reshape(12), 0)])
+    gd = api.GBufferDevice(ctx, W, H)
+    gbuf = gd.download()
+    y, x = np.mgrid[0:H, 0:W].astype(np.float32) / W - 0.5
+    gbuf["position"] = np.stack([x, 0 * x, y], -1).reshape(gbuf["position"].shape).astype(np.float32)
+    gbuf["normal"] = np.broadcast_to(np.float32([0, 1, 0]), gbuf["normal"].shape).copy()
+    gd.upload(gbuf)
+    sb = api.HostScene(api.SCENE_CUBE, 0).pack()
+    sb.ao_min, sb.ao_max, sb.ao_num_samples = 1e-4, 2.0, 16
+    got = []
+    for cull in (False, True):
+        ctx.set_group_culling(cull)
+        dsh, dao = ctx.buffer(sb.num_lights * W * H), ctx.buffer(W * H)
+        ctx.trace_visibility(tlas, gd.desc(), sb, dsh, dao)
+        got.append((dsh.download(np.uint8, (sb.num_lights, W * H)), dao.download(np.uint8, W * H)))
+    print(f"unoccluded AO samples: {int(got[0][1].sum())} unculled, {int(got[1][1].sum())} culled", flush=True)
+    assert got[0][1].sum() < 16 * W * H
+    np.testing.assert_array_equal(got[1][0], got[0][0])
+    np.testing.assert_array_equal(got[1][1], got[0][1])
+    tlas.destroy()
+    blas.destroy()
