@@ -582,6 +582,33 @@ luzrt_status count_traced(luzrt_ctx* ctx, uint32_t active_pixels, uint64_t* trac
     return LUZRT_OK;
 }
 
+namespace {
+
+// Launches one traversal kernel.  Its workgroups on the chip at once (deal_rays)
+// follow from the registers and LDS it was built with: five a CU with 16 stack
+// entries, three or four with 32.  Asked once per kernel.
+template <bool WIDE, int SHORT, int SRC, int DEPTH, bool CULLED>
+void launch_kernel(luzrt_ctx* ctx, uint32_t groups, TraceLaunch l, uint32_t refill) {
+    static const uint32_t per_cu = [] {
+        int n = 0;
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &n, k_trace_any<WIDE, SHORT, SRC, DEPTH, CULLED>, kBlock, 0);
+        return e == hipSuccess && n > 0 ? (uint32_t)n : 1u;
+    }();
+    l.resident = std::max(1u, (uint32_t)ctx->num_cus * per_cu);
+    k_trace_any<WIDE, SHORT, SRC, DEPTH, CULLED><<<groups, kBlock, 0, ctx->stream>>>(l, refill);
+}
+
+template <bool WIDE, int SRC, bool CULLED>
+void launch_any(luzrt_ctx* ctx, uint32_t groups, const TraceLaunch& l, uint32_t refill) {
+    const uint32_t sd = ctx->stack_entries;
+    if (sd <= 8) launch_kernel<WIDE, 8, SRC, kSpill, CULLED>(ctx, groups, l, refill);
+    else if (sd <= 16) launch_kernel<WIDE, 16, SRC, kSpill, CULLED>(ctx, groups, l, refill);
+    else launch_kernel<WIDE, 32, SRC, kSpill, CULLED>(ctx, groups, l, refill);
+}
+
+}  // namespace
+
 luzrt_status launch_trace(luzrt_ctx* ctx, const TraceLaunch& L) {
     uint32_t groups = (uint32_t)ctx->num_cus * ctx->groups_per_cu;
     if (L.max_rays > 0) groups = (uint32_t)std::min<uint64_t>(groups, (L.max_rays + kBlock - 1) / kBlock);
@@ -592,52 +619,22 @@ luzrt_status launch_trace(luzrt_ctx* ctx, const TraceLaunch& L) {
     TraceLaunch l = L;
     l.spill = (uint32_t*)ctx->spill.ptr;
     l.max_steps = ctx->max_steps;
-    // five waves per SIMD (launch bounds), four with 32 LDS stack entries per lane
-    l.resident = std::max(1u, (uint32_t)ctx->num_cus * (ctx->stack_entries > 16 ? 4u : 5u));
     uint32_t refill = ctx->refill_threshold ? ctx->refill_threshold : 64u;
-    auto launch = [&](auto kern) { kern<<<groups, kBlock, 0, ctx->stream>>>(l, refill); };
-    const uint32_t sd = ctx->stack_entries;
     if (L.nscenes > 0) {
         if (L.wide || L.nscenes > kMaxBatch)
             return fail(ctx, LUZRT_E_UNSUPPORTED, "multi-scene traversal: binary BVHs, <= %u scenes",
                         kMaxBatch);
-        if (L.live_rows) {
-            if (sd <= 8) launch(k_trace_any<false, 8, kBatch, kSpill, true>);
-            else if (sd <= 16) launch(k_trace_any<false, 16, kBatch, kSpill, true>);
-            else launch(k_trace_any<false, 32, kBatch, kSpill, true>);
-        } else {
-            if (sd <= 8) launch(k_trace_any<false, 8, kBatch>);
-            else if (sd <= 16) launch(k_trace_any<false, 16, kBatch>);
-            else launch(k_trace_any<false, 32, kBatch>);
-        }
+        if (L.live_rows) launch_any<false, kBatch, true>(ctx, groups, l, refill);
+        else launch_any<false, kBatch, false>(ctx, groups, l, refill);
     } else if (L.gen && L.live_rows) {
-        if (L.wide) {
-            if (sd <= 8) launch(k_trace_any<true, 8, kGen, kSpill, true>);
-            else if (sd <= 16) launch(k_trace_any<true, 16, kGen, kSpill, true>);
-            else launch(k_trace_any<true, 32, kGen, kSpill, true>);
-        } else {
-            if (sd <= 8) launch(k_trace_any<false, 8, kGen, kSpill, true>);
-            else if (sd <= 16) launch(k_trace_any<false, 16, kGen, kSpill, true>);
-            else launch(k_trace_any<false, 32, kGen, kSpill, true>);
-        }
+        if (L.wide) launch_any<true, kGen, true>(ctx, groups, l, refill);
+        else launch_any<false, kGen, true>(ctx, groups, l, refill);
     } else if (L.gen) {
-        if (L.wide) {
-            if (sd <= 8) launch(k_trace_any<true, 8, kGen>);
-            else if (sd <= 16) launch(k_trace_any<true, 16, kGen>);
-            else launch(k_trace_any<true, 32, kGen>);
-        } else {
-            if (sd <= 8) launch(k_trace_any<false, 8, kGen>);
-            else if (sd <= 16) launch(k_trace_any<false, 16, kGen>);
-            else launch(k_trace_any<false, 32, kGen>);
-        }
-    } else if (L.wide) {
-        if (sd <= 8) launch(k_trace_any<true, 8, kRays>);
-        else if (sd <= 16) launch(k_trace_any<true, 16, kRays>);
-        else launch(k_trace_any<true, 32, kRays>);
+        if (L.wide) launch_any<true, kGen, false>(ctx, groups, l, refill);
+        else launch_any<false, kGen, false>(ctx, groups, l, refill);
     } else {
-        if (sd <= 8) launch(k_trace_any<false, 8, kRays>);
-        else if (sd <= 16) launch(k_trace_any<false, 16, kRays>);
-        else launch(k_trace_any<false, 32, kRays>);
+        if (L.wide) launch_any<true, kRays, false>(ctx, groups, l, refill);
+        else launch_any<false, kRays, false>(ctx, groups, l, refill);
     }
     LUZ_HIP(ctx, hipGetLastError());
     return LUZRT_OK;
@@ -963,12 +960,9 @@ extern "C" luzrt_status luzrt_trace_visibility_static(luzrt_ctx* ctx, const luzr
         L.act_rec = act_rec;
         uint32_t groups = (uint32_t)ctx->num_cus * ctx->groups_per_cu;
         groups = groups == 0 ? 1u : (groups > kStaticGroups ? kStaticGroups : groups);
-        L.resident = std::max(1u, (uint32_t)ctx->num_cus * 5u);
         const uint32_t refill = ctx->refill_threshold ? ctx->refill_threshold : 64u;
-        if (L.wide)
-            k_trace_any<true, kStaticShort, kGen, kStaticDepth><<<groups, kBlock, 0, st>>>(L, refill);
-        else
-            k_trace_any<false, kStaticShort, kGen, kStaticDepth><<<groups, kBlock, 0, st>>>(L, refill);
+        if (L.wide) launch_kernel<true, kStaticShort, kGen, kStaticDepth, false>(ctx, groups, L, refill);
+        else launch_kernel<false, kStaticShort, kGen, kStaticDepth, false>(ctx, groups, L, refill);
         LUZ_HIP(ctx, hipGetLastError());
     } else if (ds.r_total > 0) {
         if ((s = zero_fill(ctx, hits, npix * ds.r_total)) != LUZRT_OK) return s;

@@ -41,6 +41,18 @@ def test_ray_counts_around_chunks(ctx, cube, n, groups):
     np.testing.assert_array_equal(got, want[:n])
 
 
+@pytest.mark.parametrize("stack", [8, 32])
+@pytest.mark.parametrize("n", [1, 786432, 786433, 1 << 20])
+def test_ray_counts_around_chunks_of_other_stacks(ctx, cube, n, stack):
+    # 32 entries leave three workgroups a CU (dealt up to 786,432 rays), 8 five
+    g, rays, want = cube
+    two = np.tile(rays.download(np.float32, (1 << 19, 8)), (2, 1))
+    ctx.set_trace_config(stack_entries=stack)
+    got = _hits(ctx, g.tlas, ctx.to_device(two), n)
+    ctx.set_trace_config(stack_entries=16)
+    np.testing.assert_array_equal(got, np.tile(want, 2)[:n])
+
+
 def test_special_rays_meet_the_same_triangles_in_both_trees(ctx):
     """Zero, negative-zero, infinite, denormal and NaN components: any-hit results of
     the 8-wide tree equal the binary tree's."""
