@@ -314,6 +314,8 @@ __device__ inline void store_child_box(Node* nd, int side, const float* b) {
 
 
 constexpr int kRefitChunk = 1024;   // leaf slots per workgroup of the chunk pass
+constexpr int kRefitFew = 256;      // the same for one BLAS of a few chunks (launch_refit_chunks)
+constexpr uint32_t kRefitFewMax = 16384;
 constexpr int kSpanThreads = 1024;  // threads per BLAS of the span pass
 
 // Union of a node's two child boxes, child 0 first (the operand order of
@@ -335,7 +337,7 @@ __device__ inline uint32_t chunk_job_of(const RefitJob* jobs, uint32_t njobs, ui
     return lo;
 }
 
-// Chunk pass of a refit (or of a build): one workgroup per kRefitChunk
+// Chunk pass of a refit (or of a build): one workgroup per CHUNK
 // consecutive leaf slots of a BLAS.  Every internal node covers a contiguous
 // range of slots that starts or ends at the slot of its own number (Karras), so
 // a node whose range lies inside the chunk has both children completed by this
@@ -352,15 +354,15 @@ __device__ inline uint32_t chunk_job_of(const RefitJob* jobs, uint32_t njobs, ui
 // 23 us against 256-slot chunks with the hierarchy read at every step; 200,978
 // triangles 96 -> 38 and 251 -> 66 us (512 slots: 16, 26, 56, 109).
 constexpr uint32_t kOutside = 0x80000000u;   // the node's range leaves the chunk
-template <bool FROM_VERTS>
-__global__ __launch_bounds__(kRefitChunk) void k_refit_chunks(const RefitJob* jobs, uint32_t njobs,
+template <bool FROM_VERTS, int CHUNK>
+__global__ __launch_bounds__(CHUNK) void k_refit_chunks(const RefitJob* jobs, uint32_t njobs,
                                                               RefitJob single, uint32_t* error) {
-    __shared__ uint32_t scnt[kRefitChunk];
-    __shared__ uint2 stopo[kRefitChunk];   // child 0; parent (31 bits, all set at the root) and kOutside
-    __shared__ float sbox[kRefitChunk * 12];
+    __shared__ uint32_t scnt[CHUNK];
+    __shared__ uint2 stopo[CHUNK];   // child 0; parent (31 bits, all set at the root) and kOutside
+    __shared__ float sbox[CHUNK * 12];
     const RefitJob& J = jobs ? jobs[chunk_job_of(jobs, njobs, blockIdx.x)] : single;
-    const uint32_t c0 = (blockIdx.x - J.chunk_offset) * kRefitChunk;
-    const uint32_t c1 = (c0 + kRefitChunk < J.n ? c0 + kRefitChunk : J.n) - 1;   // last slot
+    const uint32_t c0 = (blockIdx.x - J.chunk_offset) * CHUNK;
+    const uint32_t c1 = (c0 + CHUNK < J.n ? c0 + CHUNK : J.n) - 1;   // last slot
     const uint32_t s = c0 + threadIdx.x;
     scnt[threadIdx.x] = 0;
     if (s < J.n - 1) {
@@ -1317,6 +1319,23 @@ uint32_t* build_error_flag(luzrt_ctx* ctx) {
     return (uint32_t*)ctx->counters.ptr + kCntBuildError;
 }
 
+namespace {
+
+// The chunk pass of one BLAS.  Up to 1024 triangles are one chunk with nothing
+// left for the span pass.  A few chunks of 1024 slots put their sixteen waves
+// each on a few CUs, where they climb in turns, and the span pass has little to
+// save: refits (256 / 1024 slots) of 1,800 triangles 23.6 / 30.8 us, 5,000 29.3 /
+// 35.9, 9,800 35.4 / 40.9, 20,000 45.0 / 44.2, 80,000 118 / 57; of 800 21.0 / 18.3.
+template <bool FROM_VERTS>
+void launch_refit_chunks(hipStream_t st, const RefitJob& J, uint32_t* error) {
+    if (J.n > (uint32_t)kRefitChunk && J.n <= kRefitFewMax)
+        k_refit_chunks<FROM_VERTS, kRefitFew><<<cdiv(J.n, kRefitFew), kRefitFew, 0, st>>>(nullptr, 1, J, error);
+    else
+        k_refit_chunks<FROM_VERTS, kRefitChunk><<<refit_chunks(J.n), kRefitChunk, 0, st>>>(nullptr, 1, J, error);
+}
+
+}  // namespace
+
 luzrt_status blas_build_device(luzrt_ctx* ctx, luzrt_blas* b, const void* vertices,
                                const uint32_t* indices) {
     ctx->release_clean = false;   // BLAS data written on the context's stream
@@ -1369,7 +1388,7 @@ luzrt_status blas_build_device(luzrt_ctx* ctx, luzrt_blas* b, const void* vertic
     k_gather<<<nb, kBlock, 0, st>>>(verts, b->stride, b->vertex_count, indices, vin, n, boxes,
                                     b->tris, b->nrms, b->prims, b->slot_idx, slot_box, error);
     const RefitJob J = refit_job(b, nullptr, slot_box);
-    k_refit_chunks<false><<<refit_chunks(n), kRefitChunk, 0, st>>>(nullptr, 1, J, error);
+    launch_refit_chunks<false>(st, J, error);
     k_refit_spans<<<1, kSpanThreads, 0, st>>>(nullptr, J, error);
     LUZ_HIP(ctx, hipGetLastError());
     LUZ_HIP(ctx, hipFreeAsync(scratch, st));
@@ -1391,7 +1410,7 @@ luzrt_status blas_refit_device(luzrt_ctx* ctx, luzrt_blas* b, const void* vertic
         return LUZRT_OK;
     }
     const RefitJob J = refit_job(b, vertices, nullptr);
-    k_refit_chunks<true><<<refit_chunks(n), kRefitChunk, 0, st>>>(nullptr, 1, J, error);
+    launch_refit_chunks<true>(st, J, error);
     k_refit_spans<<<1, kSpanThreads, 0, st>>>(nullptr, J, error);
     LUZ_HIP(ctx, hipGetLastError());
     return LUZRT_OK;
@@ -1577,7 +1596,7 @@ luzrt_status launch_refit_batched(luzrt_ctx* ctx, const RefitJob* dev_jobs, uint
     if (!error) return fail(ctx, LUZRT_E_OUT_OF_MEMORY, "no device memory for the error flag");
     if (njobs == 0 || total_chunks == 0) return LUZRT_OK;
     RefitJob none{};
-    k_refit_chunks<true><<<total_chunks, kRefitChunk, 0, ctx->stream>>>(dev_jobs, njobs, none, error);
+    k_refit_chunks<true, kRefitChunk><<<total_chunks, kRefitChunk, 0, ctx->stream>>>(dev_jobs, njobs, none, error);
     k_refit_spans<<<njobs, kSpanThreads, 0, ctx->stream>>>(dev_jobs, none, error);
     LUZ_HIP(ctx, hipGetLastError());
     return LUZRT_OK;

@@ -36,6 +36,32 @@ def test_blas_bytes_match_oracle(ctx):
         g.close()
 
 
+@pytest.mark.parametrize("tris", [2, 255, 257, 1024, 1025, 1281, 16384, 16385])
+def test_blas_bytes_of_any_chunk_count_match_oracle(ctx, tris):
+    """Built and refitted nodes of meshes on both sides of the chunk sizes of the box pass
+    (256 slots for 1,025 .. 16,384 triangles, else 1024)."""
+    rng = np.random.default_rng(tris)
+    verts = [np.zeros((3 * tris, 12), np.float32) for _ in range(2)]
+    c = rng.normal(size=(tris, 1, 3)) * (40, 3, 40)
+    verts[0][:, :3] = (c + rng.normal(size=(tris, 3, 3)) * 0.3).astype(np.float32).reshape(-1, 3)
+    verts[1][:, :3] = verts[0][:, :3] * np.float32([1.5, -2.0, 1.0])     # the refit's
+    idx = np.arange(3 * tris, dtype=np.uint32)
+    blas = ctx.create_blas(ctx.to_device(verts[0]), 48, 3 * tris, ctx.to_device(idx), len(idx))
+    o = orc.OracleScene()
+    m = o.add_mesh(verts[0], idx)
+    o.set_instances(np.eye(3, 4, dtype=np.float32).reshape(1, 12), [m])
+    for refit in (False, True):
+        if refit:
+            blas.refit(ctx.to_device(verts[1]))
+            o.refit_mesh(m, verts[1])
+        on, ot, op = o.blas_arrays(m)
+        gn, gt, gp = blas.arrays()
+        np.testing.assert_array_equal(gp, op)
+        np.testing.assert_array_equal(gt.view(np.uint32), ot.view(np.uint32))
+        np.testing.assert_array_equal(gn, on)
+    blas.destroy()
+
+
 def test_tlas_bytes_match_oracle(ctx):
     s, g = _gpu_scene(ctx, api.SCENE_SPHERES)
     o = oracle_scene(s)
