@@ -191,11 +191,10 @@ __device__ inline GroupRows cull_group(const PixelFrame& f, uint64_t pixels, con
     // a box that is not finite (a vertex near the largest float) bounds nothing:
     // the per-pixel tests would take its NaN centre for out of reach
     auto bound = [](float (&lo)[3], float (&hi)[3]) {
-        bool finite = true;
-        for (int k = 0; k < 3; ++k) finite = finite && isfinite(lo[k]) && isfinite(hi[k]);
+        if (isfinite((hi[0] - lo[0]) + (hi[1] - lo[1]) + (hi[2] - lo[2]))) return;
         for (int k = 0; k < 3; ++k) {
-            lo[k] = finite ? lo[k] : -1e38f;
-            hi[k] = finite ? hi[k] : 1e38f;
+            lo[k] = -1e38f;
+            hi[k] = 1e38f;
         }
     };
     bound(blo, bhi);
