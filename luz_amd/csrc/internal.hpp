@@ -52,6 +52,7 @@ struct luzrt_ctx {
     bool last_culled = false;      // the last visibility call traced live rows only,
     uint32_t last_groups = 0, last_kinds = 0;   // of so many ray groups and kinds,
     uint8_t last_slots[LUZRT_MAX_LIGHTS + 1] = {};   // with so many slots per kind
+    bool last_counted = false;     // its traced rays are in counters[kCntTraced]
     // timing
     hipEvent_t ev[luz::kStageCount][2] = {};
     bool ev_used[luz::kStageCount] = {};
@@ -361,8 +362,9 @@ inline uint32_t tile_chunk(uint64_t ntiles, uint32_t groups) {
     return c < 1 ? 1u : (c > 64 ? 64u : (uint32_t)c);
 }
 luzrt_status launch_trace(luzrt_ctx* ctx, const TraceLaunch& L);
-// Rays the last visibility call traced, if it culled (waits for the count).
-luzrt_status count_traced(luzrt_ctx* ctx, uint32_t active_pixels, uint64_t* traced);
+// Counts the rays that the last visibility call, a culled one, traced, if that
+// is still to be done (counters[kCntTraced], on the context's stream).
+luzrt_status count_traced(luzrt_ctx* ctx);
 // Exclusive scan in place of n live-row counts (16-byte aligned), the total to
 // counters[kCntLive] (one workgroup, trace.hip).
 void launch_cull_scan(hipStream_t st, uint32_t* counts, uint32_t n, uint32_t* counters);

@@ -446,6 +446,10 @@ luzrt_status luzrt_sync(luzrt_ctx* ctx) {
 
 luzrt_status luzrt_get_timings(luzrt_ctx* ctx, luzrt_timings* out) {
     if (!ctx || !out) return LUZRT_E_INVALID_ARG;
+    if (ctx->last_culled) {
+        luzrt_status s = count_traced(ctx);
+        if (s != LUZRT_OK) return s;
+    }
     LUZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (build_stream_sync(ctx) != LUZRT_OK) return LUZRT_E_DEVICE;
     float* f[kStageCount] = {&out->build_ms, &out->compact_ms, &out->raygen_ms, &out->trace_ms,
@@ -467,11 +471,7 @@ luzrt_status luzrt_get_timings(luzrt_ctx* ctx, luzrt_timings* out) {
         LUZ_HIP(ctx, hipMemcpy(c, ctx->counters.ptr, sizeof(c), hipMemcpyDeviceToHost));
         out->rays = c[kCntRays];
         out->active_pixels = c[kCntActive];
-        out->traced_rays = out->rays;
-        if (ctx->last_culled) {
-            luzrt_status s = count_traced(ctx, c[kCntActive], &out->traced_rays);
-            if (s != LUZRT_OK) return s;
-        }
+        out->traced_rays = ctx->last_culled ? c[kCntTraced] : c[kCntRays];
         if (c[kCntError]) return check_trace_latch(ctx);
         if (c[kCntBuildError])
             return fail(ctx, LUZRT_E_INVALID_ARG, "acceleration-structure build error flag %u",

@@ -59,6 +59,7 @@ __global__ __launch_bounds__(1024) void k_compact_scan(uint32_t* block_counts, u
         counters[kCntActive] = total;
         counters[kCntRays] = total * ds->r_total;
         counters[kCntFetch] = 0;
+        counters[kCntTraced] = 0;
     }
     clear_claims(counters, threadIdx.x);
 }
@@ -531,17 +532,18 @@ __global__ __launch_bounds__(kBlock, SHORT > 16 ? 1 : 5) void k_trace_any(TraceL
 }
 
 // The rays a culled call traced: the pixels of each kind times its slots, a
-// thread per group and kind.
+// thread per group and kind of the groups with active pixels.
 struct KindSlots {
     uint8_t n[LUZRT_MAX_LIGHTS + 1];
 };
 __global__ __launch_bounds__(kBlock) void k_count_traced(const uint64_t* pix, uint32_t groups, uint32_t kinds,
-                                                         KindSlots slots, uint32_t* total) {
+                                                         KindSlots slots, uint32_t* counters) {
+    const uint32_t n = min(groups, (counters[kCntActive] + kCullGroup - 1) / kCullGroup) * kinds;
     uint32_t sum = 0;
-    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < groups * kinds; i += gridDim.x * kBlock)
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
         sum += (uint32_t)__popcll(pix[i]) * slots.n[i % kinds];
     for (uint32_t off = 32; off; off >>= 1) sum += __shfl_xor(sum, off);
-    if ((threadIdx.x & 63u) == 0 && sum) atomicAdd(total, sum);
+    if ((threadIdx.x & 63u) == 0 && sum) atomicAdd(&counters[kCntTraced], sum);
 }
 
 // Thread q zeroes the counts of pixel q if it is background and resolves
@@ -565,20 +567,16 @@ void launch_cull_scan(hipStream_t st, uint32_t* counts, uint32_t n, uint32_t* co
     k_cull_scan<<<1, 1024, 0, st>>>(counts, n, counters);
 }
 
-luzrt_status count_traced(luzrt_ctx* ctx, uint32_t active_pixels, uint64_t* traced) {
-    uint32_t* total = (uint32_t*)ctx->counters.ptr + kCntTraced;
-    const uint32_t groups = std::min(ctx->last_groups, cdiv(active_pixels, kCullGroup));
+luzrt_status count_traced(luzrt_ctx* ctx) {
+    if (ctx->last_counted) return LUZRT_OK;
+    uint32_t* counters = (uint32_t*)ctx->counters.ptr;
     KindSlots slots;
     std::memcpy(slots.n, ctx->last_slots, sizeof(slots.n));
-    uint32_t n = 0;
-    LUZ_HIP(ctx, hipMemsetAsync(total, 0, 4, ctx->stream));
     k_count_traced<<<256, kBlock, 0, ctx->stream>>>(
-        (const uint64_t*)ctx->cull_cand.ptr + (size_t)ctx->last_groups * ctx->last_kinds * kCandWords, groups,
-        ctx->last_kinds, slots, total);
+        (const uint64_t*)ctx->cull_cand.ptr + (size_t)ctx->last_groups * ctx->last_kinds * kCandWords, ctx->last_groups,
+        ctx->last_kinds, slots, counters);
     LUZ_HIP(ctx, hipGetLastError());
-    LUZ_HIP(ctx, hipMemcpyAsync(&n, total, 4, hipMemcpyDeviceToHost, ctx->stream));
-    LUZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    *traced = n;
+    ctx->last_counted = true;
     return LUZRT_OK;
 }
 
@@ -719,6 +717,7 @@ luzrt_status visibility_core(luzrt_ctx* ctx, const luzrt_tlas* tlas, const luzrt
             ctx->last_slots[k] = (uint8_t)(end - begin);
         }
         ctx->last_culled = true;
+        ctx->last_counted = false;
     }
 
     stage_begin(ctx, kStageTrace);

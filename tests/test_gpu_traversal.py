@@ -273,6 +273,7 @@ def test_timings_after_ray_queries_count_their_rays(ctx):
         ctx.trace_visibility(g.tlas, gd.desc(), sb, sh, ao)
         t = ctx.timings()
         assert 0 < t.traced_rays < t.rays      # culled
+        assert ctx.timings().traced_rays == t.traced_rays
         _hits(ctx, g.tlas, ctx.to_device(rays), len(rays))
         t = ctx.timings()
         assert (t.rays, t.traced_rays) == (777, 777)
