@@ -352,8 +352,8 @@ struct BatchTlas {
 constexpr uint32_t kMaxBatch = LUZRT_MAX_BATCH;
 constexpr uint32_t kRayGroup = 64;   // pixels per ray group of the grouped ray order (ray_row)
 // Persistent workgroups per CU of the closest-hit kernels (primary rays, shadow
-// maps; up to 96 VGPRs, 16 KB of LDS stacks and 15 KB of staged TLAS per
-// workgroup leave room for five waves per SIMD).
+// maps): up to 96 VGPRs, 16 KB of LDS stacks and, in single-scene launches, 11 KB
+// of staged TLAS per workgroup leave room for five waves per SIMD.
 constexpr uint32_t kPrimaryGroupsPerCu = 5;
 // Tiles per claim: about 8 claims per wave, so that the claims of a large
 // launch do not queue on their counters.

@@ -6,7 +6,7 @@
 //   shadow_setup / gen_ray                    light.frag:86-146, 111-135, 229-231
 //   resolve_pixel                             occluded / unoccluded sample counts
 //   shade_pixel                               light.frag:17-49, 171-235 (FP32, hardware rcp/rsq)
-//   primary_pixel / primary_texel             G-buffer texels by closest-hit primary rays
+//   primary_dir / primary_texel               G-buffer texels of closest-hit primary rays
 #pragma once
 #include "internal.hpp"
 #include "traverse.hpp"
