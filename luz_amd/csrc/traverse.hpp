@@ -180,7 +180,7 @@ __device__ inline Half2 byte_pair(uint32_t w) {
 // loop as often as its busiest lane needs, and in one loop a lane with a
 // triangle made the others wait for it at every position.  VALU instructions
 // per node 246 -> 173; frame of the 4K terrain 22.2 -> 20.9 ms (min, max, perm
-// and fma_mix issue at 4.4 cycles per wave64 here, add, mul and fma at 2.6).
+// and fma_mix issue at 4.4 cycles per wave64 here, add and mul at 2.6 to 2.9, fma at 3.1).
 template <typename STACK>
 __device__ inline int wide_visit(RayState& r, STACK& st) {
     const GlobalWords p = (GlobalWords)(reinterpret_cast<const Node8*>(r.bnodes) + r.next);
